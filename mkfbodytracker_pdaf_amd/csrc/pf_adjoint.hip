@@ -221,7 +221,7 @@ __global__ void __launch_bounds__(kAdjTile) __attribute__((amdgpu_waves_per_eu(3
     const uint32_t U1 = ba.uni[(size_t)(sd.tofs + a.t) * 2];
     unsigned flags = 0;   // the recorded forward run reported them
     (void)particle_update<D, kModeCand, SELJ>(ba.base, a.t, j, U1, reinterpret_cast<const float *>(sm4), x, P,
-                                              sd.pi_total, seq_comp_global(ba, sd), nullptr, flags);
+                                              seq_comp_global(ba, sd), nullptr, flags);
     store_state(a.out_x, a.out_P, ba.ld, sd.pofs + j, x, P);
 }
 
@@ -288,13 +288,13 @@ __global__ void __launch_bounds__(kAdjTile) k_adj_step(AdjArgs a)
         load_state(a.in_x, a.in_P, ba.ld, sd.pofs + src, x, P);
         // ---- forward recompute, recording each joint's inputs
         constexpr int CS = 2 + D + NP;
-        const unsigned long long *sthr = reinterpret_cast<const unsigned long long *>(sm);
-        const float *Hs = sm + 4 * K;
+        const unsigned long long *keys = reinterpret_cast<const unsigned long long *>(sm);
+        const float *Hs = sm + 2 * K;
         const float *BHs = Hs + ba.m * D;
         const float *Rs = BHs + ba.m;
         const float *stab = v.comp_global ? v.comp_global : sm + image_head_floats(K, ba.m, D, ba.J);
         const uint32_t U1 = ba.uni[(size_t)(sd.tofs + t) * 2];
-        k = draw_component(sthr, K, (uint32_t)j, U1, sd.pi_total);
+        k = draw_component(keys, K, (uint32_t)j, U1);
         const float *ck = stab + k * CS;
         const float g = ck[0], g2 = ck[1];
 #pragma unroll

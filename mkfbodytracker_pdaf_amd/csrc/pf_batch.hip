@@ -147,7 +147,7 @@ k_batch_step(BatchArgs a)
             if (j < sd.N) {
                 unsigned f = 0;
                 float lwj = particle_update<D, kModeCand, SELJ>(a.base, t, j, U1, reinterpret_cast<const float *>(sm4),
-                                                                x[r], P[r], sd.pi_total, comp_global, comp_out, f);
+                                                                x[r], P[r], comp_global, comp_out, f);
                 const unsigned doff = (unsigned)(sd.pofs + j) * 4u;
                 auto store = [&]() {
                     if constexpr (D > 16) {
@@ -427,7 +427,6 @@ int build_batch_tables(pf_batch *b)
         std::copy(imgs[i].T.begin(), imgs[i].T.end(), Ts.begin() + (size_t)i * d * d);
         std::copy(imgs[i].Ti.begin(), imgs[i].Ti.end(), Tis.begin() + (size_t)i * d * d);
         b->h_seqs[i].table_ofs = (int)(i * tf);
-        b->h_seqs[i].pi_total = imgs[i].pi_total;
     }
     (void)hipFree(b->tables); (void)hipFree(b->mus); (void)hipFree(b->sigs); (void)hipFree(b->Ts); (void)hipFree(b->Tis);
     HIP_TRYB(dallocb(&b->tables, tabs.size()));

@@ -26,7 +26,6 @@ constexpr int kSeqAlign = 512;    // particle offset alignment (largest tile)
 
 struct SeqDesc {
     int pofs, N, T, tofs, bofs, nb, table_ofs, pad;
-    unsigned long long pi_total;
 };
 
 struct BatchArgs {
@@ -77,9 +76,6 @@ __device__ __forceinline__ SeqDesc uniform_seq(const SeqDesc *seqs, int s)
     r.nb = uni_int(d.nb);
     r.table_ofs = uni_int(d.table_ofs);
     r.pad = 0;
-    const unsigned lo = (unsigned)uni_int((int)(unsigned)d.pi_total);
-    const unsigned hi = (unsigned)uni_int((int)(unsigned)(d.pi_total >> 32));
-    r.pi_total = ((unsigned long long)hi << 32) | lo;
     return r;
 }
 
@@ -118,7 +114,6 @@ __device__ __forceinline__ StepArgs seq_view(const BatchArgs &a, const SeqDesc &
     StepArgs v{};
     v.count = a.count + (size_t)sd.tofs * a.J;
     v.cand = a.cand + (size_t)sd.tofs * a.J * a.cap * 2;
-    v.pi_total = sd.pi_total;
     v.table_floats = a.table_floats;
     v.stage_floats = a.stage_floats;
     v.K = a.K;

@@ -75,7 +75,6 @@ struct pf_handle {
     float *table = nullptr;
     int table_floats = 0;          // floats of the image staged in LDS
     const float *comp_global = nullptr;   // component rows read from global memory (large images)
-    unsigned long long pi_total = 0;
     float *mu = nullptr, *sig = nullptr;
     HostModel hm;
     // state basis x' = T x (T = I when H has no usable row-selection basis)
@@ -416,7 +415,6 @@ StepArgs step_args(pf_handle *h, int mode, const uint32_t *uni, const float *Z, 
     a.zld = zld;
     a.count = count;
     a.cand = cand;
-    a.pi_total = h->pi_total;
     a.table_floats = h->table_floats;
     a.comp_global = h->comp_global;
     a.stage_floats = h->table_floats + (mode == kModeCand ? cand_lds_floats(h->J, h->cap) : 0);
@@ -497,7 +495,6 @@ int build_tables(pf_handle *h)
     int st = make_model_image(h->hm, h->order_packed, h->N, img);
     if (st) return st;
     h->sel_mode = img.sel_mode;
-    h->pi_total = img.pi_total;
     (void)hipFree(h->table); (void)hipFree(h->mu); (void)hipFree(h->sig);
     (void)hipFree(h->Tdev); (void)hipFree(h->Tinv);
     h->table = nullptr; h->mu = nullptr; h->sig = nullptr; h->Tdev = nullptr; h->Tinv = nullptr;

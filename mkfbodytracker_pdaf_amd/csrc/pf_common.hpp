@@ -1,6 +1,6 @@
 // pf_common.hpp -- helpers shared by host and device code of the particle
 // filter library: packed symmetric indexing, the deterministic exp used by the
-// resampler, fixed-point weights and 128-bit threshold arithmetic.
+// resampler, fixed-point weights and the exact systematic thresholds.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -113,24 +113,77 @@ __host__ __device__ inline int pow_shift(int E, int e)
 
 __host__ __device__ inline uint64_t shr64(uint64_t x, int s) { return s >= 64 ? 0 : x >> s; }
 
-// Systematic threshold of output i: (i * 2^32 + U) * total.
-__host__ __device__ inline u128 sys_target(uint32_t i, uint32_t U, uint64_t total)
+// Systematic resampling of N outputs: output i takes the first input whose
+// inclusive prefix C satisfies C N 2^32 > (i 2^32 + U) total, i.e. C > f_i
+// with the integer f_i = floor((i 2^32 + U) total / (N 2^32))
+//                     = floor((i total + floor(U total / 2^32)) / N).
+// With total = qt N + rt and floor(U total / 2^32) = qv N + rv this is
+// i qt + qv + floor((i rt + rv) / N): the two divisions by N are made once,
+// and the per-output one has a dividend below 2^53 (i, rt < N <= 2^26,
+// total <= 2^52), where the product with 1 / N in FP64 is off by at most one.
+// The searches then compare 64-bit prefixes with f_i.
+__host__ __device__ inline uint64_t div_near(uint64_t s, uint32_t n, double inv, uint64_t &rem)
 {
-    return (u128)((((uint64_t)i) << 32) | U) * total;
+    uint64_t q = (uint64_t)((double)s * inv);
+    int64_t r = (int64_t)(s - q * n);
+    if (r < 0) {
+        --q;
+        r += n;
+    } else if (r >= (int64_t)n) {
+        ++q;
+        r -= n;
+    }
+    rem = (uint64_t)r;
+    return q;
 }
 
-// Model image of the step kernels: [component thresholds, 4K floats][H
+struct SysThresholds {
+    uint64_t qt, qv, rv;
+    uint32_t rt, n;
+    double inv;
+    __host__ __device__ SysThresholds(uint64_t total, uint32_t U, uint32_t N) : n(N), inv(1.0 / (double)N)
+    {
+        uint64_t r;
+        qt = div_near(total, n, inv, r);
+        rt = (uint32_t)r;
+        qv = div_near((uint64_t)(((u128)total * U) >> 32), n, inv, rv);
+    }
+    // f_i for i < N
+    __host__ __device__ uint64_t operator()(uint32_t i) const
+    {
+        const uint64_t s = (uint64_t)i * rt + rv;
+        uint32_t q = (uint32_t)((double)s * inv);
+        const int64_t r = (int64_t)(s - (uint64_t)q * n);
+        q += r < 0 ? -1 : (r >= (int64_t)n ? 1 : 0);
+        return qt * i + qv + q;
+    }
+};
+
+// Component draw resample(gmm.weight, N) as 64-bit keys.  With the cumulative
+// fixed-point weights C_k, total T = C_{K-1}, output j draws the first k with
+// C_k N 2^32 > (j 2^32 + U) T.  Write C_k N = I T + r (0 <= r < T): since
+// j 2^32 + U is an integer, C_k N 2^32 <= (j 2^32 + U) T exactly when
+// I 2^32 + ceil(r 2^32 / T) <= j 2^32 + U.  The left side depends on the model
+// alone, so the draw compares 64-bit integers.
+__host__ inline uint64_t component_key(uint64_t cum, uint64_t total, uint64_t n)
+{
+    const u128 x = (u128)cum * n;
+    const u128 whole = x / total, rest = x % total;
+    return (uint64_t)((whole << 32) + ((rest << 32) + total - 1) / total);
+}
+
+// Model image of the step kernels: [component keys, K 64-bit words][H
 // (m x D), BH (m), R 2x2 blocks (3J), padded to even][per joint the FP64
-// innovation block (bh0, bh1, r00, r01, r11) as doubles (5J), padded to 4]
-// [component rows, K x (2 + D + D(D+1)/2)].  Offset of the FP64 blocks (8-byte
-// aligned) and floats of the part before the component rows:
+// innovation block (bh0, bh1, r00, r01, r11) as doubles (5J)], padded to 4
+// floats, then [component rows, K x (2 + D + D(D+1)/2)].  Offset of the FP64
+// blocks (8-byte aligned) and floats of the part before the component rows:
 __host__ __device__ constexpr int image_j64_floats(int K, int m, int D, int J)
 {
-    return 4 * K + ((m * D + m + 3 * J + 1) & ~1);
+    return 2 * K + ((m * D + m + 3 * J + 1) & ~1);
 }
 __host__ __device__ constexpr int image_head_floats(int K, int m, int D, int J)
 {
-    return 4 * K + ((((m * D + m + 3 * J + 1) & ~1) + 10 * J + 3) & ~3);
+    return (image_j64_floats(K, m, D, J) + 10 * J + 3) & ~3;
 }
 
 // A 2 x 2 innovation covariance S = [[s00, s01], [s01, s11]] whose FP32

@@ -9,8 +9,8 @@
 //           index and writes copy B at the particle index (the resampling
 //           gather of pf2DRao.cpp:153-156 is folded into the next frame's
 //           loads).
-//   table   LDS image of the model: 2K words of component thresholds
-//           C_pi[k] * N * 2^32 (128-bit), then per component k
+//   table   LDS image of the model: K 64-bit component keys
+//           (component_key), then per component k
 //           [g, g^2, (1-g) mu_k (D), (1-g^2) Sigma_k packed], then the shared
 //           H (m x D), BH (m) and the 2x2 joint blocks of R (r00, r01, r11).
 //
@@ -186,7 +186,6 @@ struct StepArgs {
     // candidate mode: count[t][J], cand[t][J][cap][2]
     const int *__restrict__ count;
     const float *__restrict__ cand;
-    unsigned long long pi_total;
     int table_floats;   // floats of the LDS model image (multiple of 4)
     int stage_floats;   // LDS floats before the resolver workspace: image + staged detections (candidate mode)
     const float *comp_global;  // component rows in global memory when the image head alone is staged, else null
@@ -429,7 +428,7 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
     unsigned long long *misc = stg + pd.stage;
     const int *shf = reinterpret_cast<const int *>(misc + 16);
     const int bs = 1 << pd.bshift;
-    // 2. the input block of each output: largest b with pre[b] * S <= t_j
+    // 2. the input block of each output: largest b with pre[b] <= f_j
     const int j = j0 + tid;
     const int jc = min(j, N - 1);
     if (total == 0ull) {
@@ -438,11 +437,12 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
         const u128 x = (u128)((((unsigned long long)(uint32_t)jc) << 32) | U) * (u128)(unsigned)pd.L;
         return (int)((unsigned long long)(x >> 32) / (unsigned long long)N);
     }
-    const u128 S = (u128)(unsigned long long)N << 32;
-    const u128 tj = sys_target((uint32_t)jc, U, total);
+    // a_j is the first input whose prefix exceeds f_j (SysThresholds)
+    const SysThresholds thr(total, U, (uint32_t)N);
+    const unsigned long long fj = thr((uint32_t)jc);
     int lo = 0, hi = nb - 1;
     if ((nt & 63) == 0) {
-        // t_j grows with j, so every output's block lies between the blocks
+        // f_j grows with j, so every output's block lies between the blocks
         // of the block's first and last outputs.  Each wave finds those two
         // by 64-way searches: lane l probes position lo + l * step of the
         // range (non-decreasing in l, lane 0 at a position known to pass),
@@ -451,13 +451,13 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
         // each).  The output's own search then covers that span only.
         const int lane = tid & 63;
         const int jl = min(j0 + nt, N) - 1;
-        const u128 tf = sys_target((uint32_t)j0, U, total), tl = sys_target((uint32_t)jl, U, total);
+        const unsigned long long ff = thr((uint32_t)j0), fl = thr((uint32_t)jl);
         int flo = 0, fhi = nb - 1, llo = 0, lhi = nb - 1;
         while (flo < fhi || llo < lhi) {
             const int fs = (fhi - flo + 64) >> 6, ls = (lhi - llo + 64) >> 6;
             const int fp = min(flo + lane * fs, fhi), lp = min(llo + lane * ls, lhi);
-            const int fc = __popcll(__ballot((u128)pre[fp] * S <= tf));
-            const int lc = __popcll(__ballot((u128)pre[lp] * S <= tl));
+            const int fc = __popcll(__ballot(pre[fp] <= ff));
+            const int lc = __popcll(__ballot(pre[lp] <= fl));
             const int fn = min(flo + (fc - 1) * fs, fhi), ln = min(llo + (lc - 1) * ls, lhi);
             fhi = fc < 64 ? min(flo + fc * fs, fhi) - 1 : fhi;
             lhi = lc < 64 ? min(llo + lc * ls, lhi) - 1 : lhi;
@@ -469,7 +469,7 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
     }
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if ((u128)pre[mid] * S <= tj) lo = mid;
+        if (pre[mid] <= fj) lo = mid;
         else hi = mid - 1;
     }
     const int bj = lo;
@@ -504,7 +504,7 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
         int l = (bj - blo) * bs, h = min(n, (bj - blo + 1) * bs) - 1;
         while (l < h) {
             const int mid = (l + h) >> 1;
-            if ((u128)stg[mid] * S > tj) h = mid;
+            if (stg[mid] > fj) h = mid;
             else l = mid + 1;
         }
         a = base + l;
@@ -514,7 +514,7 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
         int l = bj * bs, h = min(pd.L, (bj + 1) * bs) - 1;
         while (l < h) {
             const int mid = (l + h) >> 1;
-            if ((u128)(pb + shr64(pd.cloc[mid], sh)) * S > tj) h = mid;
+            if (pb + shr64(pd.cloc[mid], sh) > fj) h = mid;
             else l = mid + 1;
         }
         a = l;
@@ -957,23 +957,18 @@ __device__ __forceinline__ void rec_store(float *rec, int N, int j0w, float4 *gw
     }
 }
 
-__device__ __forceinline__ int draw_component(const unsigned long long *thr, int K, uint32_t j,
-                                              uint32_t U, unsigned long long total)
+__device__ __forceinline__ int draw_component(const unsigned long long *keys, int K, uint32_t j, uint32_t U)
 {
-    // The first k < K - 1 whose threshold exceeds the target, else K - 1.
-    // The thresholds are cumulative (non-decreasing), so k is the count of
-    // thresholds at or below the target: they are read in groups of eight
-    // (one LDS latency per group), and the wave stops after the first group
-    // whose last threshold exceeds every lane's target.
-    const u128 t = sys_target(j, U, total);
+    // The first k < K - 1 whose key exceeds j 2^32 + U, else K - 1.  The keys
+    // are non-decreasing, so k is the count of keys at or below it: they are
+    // read in groups of eight (one LDS latency per group), and the wave stops
+    // after the first group whose last key exceeds every lane's.
+    const unsigned long long t = ((unsigned long long)j << 32) | U;
     int k = 0;
     for (int k0 = 0; k0 < K - 1; k0 += 8) {
-        u128 th[8];
+        unsigned long long th[8];
 #pragma unroll
-        for (int u = 0; u < 8; ++u) {
-            const int i = min(k0 + u, K - 2);
-            th[u] = ((u128)thr[2 * i + 1] << 64) | (u128)thr[2 * i];
-        }
+        for (int u = 0; u < 8; ++u) th[u] = keys[min(k0 + u, K - 2)];
 #pragma unroll
         for (int u = 0; u < 8; ++u)
             if (k0 + u < K - 1 && th[u] <= t) ++k;
@@ -1254,7 +1249,7 @@ __host__ __device__ constexpr int step_lds_bytes_rec(bool rec, int stage_floats,
                            : kRecStageBytes);
 }
 
-// Model image layout: [component thresholds, 4K floats][H (m x D), BH (m),
+// Model image layout: [component keys, 2K floats][H (m x D), BH (m),
 // R 2x2 blocks (3J), padded to 4][component rows, K x (2 + D + D(D+1)/2)].
 // The head is always staged in LDS; the component rows are staged with it
 // when the whole image fits the LDS budget, and read from global memory
@@ -1264,7 +1259,7 @@ __host__ __device__ constexpr int step_lds_bytes_rec(bool rec, int stage_floats,
 // predict (KF_model.cpp:11-15) and the joint updates (pf2DRao.cpp:138-140);
 // returns the particle's log-weight.  sm is the staged LDS model image.
 // The shared constants come from a (a kernel argument, read on demand); the
-// per-sequence values pi_total (component thresholds' total), comp_global
+// per-sequence values comp_global
 // (component rows outside LDS, or null) and comp_out (optional component
 // record) are passed explicitly.
 // Likelihood and update parameters of a joint that is not positive definite
@@ -1284,18 +1279,18 @@ __device__ __forceinline__ float joint_reject(float (&w0)[D], float (&w1)[D], fl
 // (joint_factor64, a per-lane branch taken only for those joints).
 template <int D, int MODE, int SELJ>
 __device__ __forceinline__ float particle_update(const StepArgs &a, int t, int j, uint32_t U1, const float *sm,
-                                                 float (&x)[D], float (&P)[npacked(D)], unsigned long long pi_total,
+                                                 float (&x)[D], float (&P)[npacked(D)],
                                                  const float *comp_global, int *comp_out, unsigned &flags)
 {
     constexpr int NP = npacked(D);
     constexpr int CS = 2 + D + NP;
-    const unsigned long long *sthr = reinterpret_cast<const unsigned long long *>(sm);
-    const float *Hs = sm + 4 * a.K;
+    const unsigned long long *keys = reinterpret_cast<const unsigned long long *>(sm);
+    const float *Hs = sm + 2 * a.K;
     const float *BHs = Hs + a.m * D;
     const float *Rs = BHs + a.m;
     const double *J64 = reinterpret_cast<const double *>(sm + image_j64_floats(a.K, a.m, D, a.J));
     const float *stab = comp_global ? comp_global : sm + image_head_floats(a.K, a.m, D, a.J);
-    const int k = draw_component(sthr, a.K, (uint32_t)j, U1, pi_total);
+    const int k = draw_component(keys, a.K, (uint32_t)j, U1);
     if (comp_out) comp_out[j] = k;
     const float *ck = stab + k * CS;
     const float g = ck[0], g2 = ck[1];
@@ -1474,7 +1469,7 @@ __device__ __forceinline__ void step_body(const StepArgs &ain)
     float lwj = -INFINITY;
     unsigned pflags = 0;
     if (live) {
-        lwj = particle_update<D, MODE, SELJ>(a, t, j, U1, reinterpret_cast<const float *>(sm4), x, P, a.pi_total,
+        lwj = particle_update<D, MODE, SELJ>(a, t, j, U1, reinterpret_cast<const float *>(sm4), x, P,
                                              a.comp_global, a.comp_out, pflags);
         if constexpr (!REC) {
             const unsigned doff = (unsigned)j * 4u;

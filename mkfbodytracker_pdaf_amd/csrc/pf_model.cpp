@@ -230,7 +230,7 @@ int make_model_image(const HostModel &hm, unsigned order, int N, ModelImage &img
     };
     const int head = image_head_floats(K, m, d, J);
     std::vector<float> tab((size_t)K * CS);                     // component rows
-    std::vector<float> hbr((size_t)head - 4 * K, 0.f);         // H, BH, R blocks
+    std::vector<float> hbr((size_t)head - 2 * K, 0.f);         // H, BH, R blocks
     img.mu.assign((size_t)K * d, 0.f);
     img.sg.assign((size_t)K * NP, 0.f);
     std::vector<double> mut(d), sgt((size_t)d * d), sym((size_t)d * d);
@@ -273,19 +273,14 @@ int make_model_image(const HostModel &hm, unsigned order, int N, ModelImage &img
         j64[5 * b + 3] = Rm[(2 * b) * m + 2 * b + 1];
         j64[5 * b + 4] = Rm[(2 * b + 1) * m + 2 * b + 1];
     }
-    // Component thresholds for resample(gmm.weight, N) (pf2DRao.cpp:128).
-    std::vector<unsigned long long> thr(2 * (size_t)K);
-    unsigned long long acc = 0;
-    for (int k = 0; k < K; ++k) {
-        acc += fixed32(hm.pi[k] / hm.wmax);
-        const u128 th = (u128)acc * ((u128)(unsigned long long)N << 32);
-        thr[2 * k] = (unsigned long long)th;
-        thr[2 * k + 1] = (unsigned long long)(th >> 64);
-    }
-    img.pi_total = acc;
+    // Component keys of resample(gmm.weight, N) (pf2DRao.cpp:128).
+    std::vector<uint64_t> cum((size_t)K), keys((size_t)K);
+    uint64_t acc = 0;
+    for (int k = 0; k < K; ++k) cum[k] = acc += fixed32(hm.pi[k] / hm.wmax);
+    for (int k = 0; k < K; ++k) keys[k] = component_key(cum[k], acc, (uint64_t)N);
     img.blob.assign((size_t)head + tab.size(), 0.f);
-    std::memcpy(img.blob.data(), thr.data(), sizeof(unsigned long long) * thr.size());
-    std::memcpy(img.blob.data() + 4 * K, hbr.data(), sizeof(float) * hbr.size());
+    std::memcpy(img.blob.data(), keys.data(), sizeof(uint64_t) * keys.size());
+    std::memcpy(img.blob.data() + 2 * K, hbr.data(), sizeof(float) * hbr.size());
     std::memcpy(img.blob.data() + image_j64_floats(K, m, d, J), j64.data(), sizeof(double) * j64.size());
     std::memcpy(img.blob.data() + head, tab.data(), sizeof(float) * tab.size());
     img.blob.resize((img.blob.size() + 3) & ~(size_t)3, 0.f);

@@ -118,8 +118,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
     __syncthreads();
 
     const float *sm = reinterpret_cast<const float *>(sm4);
-    const unsigned long long *sthr = reinterpret_cast<const unsigned long long *>(sm);
-    const float *BHs = sm + 4 * a.K + a.m * D;
+    const unsigned long long *keys = reinterpret_cast<const unsigned long long *>(sm);
+    const float *BHs = sm + 2 * a.K + a.m * D;
     const float *Rs = BHs + a.m;
     const double *J64 = reinterpret_cast<const double *>(sm + image_j64_floats(a.K, a.m, D, a.J));
     const float *comp_global = seq_comp_global(a, sd);
@@ -157,7 +157,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
                                                  : soa_ld(rP, vb + (unsigned)drow[I][r] * rowb, 0);
 
         // component draw (pf2DRao.cpp:128) and predict (KF_model.cpp:11-15)
-        const int k = draw_component(sthr, a.K, (uint32_t)j, U1, sd.pi_total);
+        const int k = draw_component(keys, a.K, (uint32_t)j, U1);
         const float *ck = stab + k * CS;
         const float g = ck[0], g2 = ck[1];
 #pragma unroll

@@ -5,6 +5,7 @@ test_host_api      the reference's call sequences on the C++ mirror classes,
                    oracle (oracle/liboracle.so);
 test_adjoint_local the host-only check of the joint-local reverse (hipcc:
                    the header is host- and device-callable);
+test_systematic    the host-only check of the resampler's 64-bit thresholds;
 sanitize_host      the library's host-side sources (pf_io.cpp, pf_model.cpp,
                    pf_host.cpp) and the oracle built with g++/gcc under
                    AddressSanitizer and UndefinedBehaviorSanitizer.
@@ -26,6 +27,8 @@ SAN_BIN = os.path.join(HERE, "sanitize_host")
 SAN_FLAGS = ["-O1", "-g", "-fno-omit-frame-pointer", "-fsanitize=address,undefined", "-fno-sanitize-recover=all"]
 ADJ_SRC = os.path.join(HERE, "test_adjoint_local.cpp")
 ADJ_BIN = os.path.join(HERE, "test_adjoint_local")
+SYS_SRC = os.path.join(HERE, "test_systematic.cpp")
+SYS_BIN = os.path.join(HERE, "test_systematic")
 
 
 def _run(cmd, what):
@@ -48,6 +51,12 @@ def build_adjoint_local_test() -> str:
     return ADJ_BIN
 
 
+def build_systematic_test() -> str:
+    _run(["g++", "-std=c++17", "-O2", "-D__HIP_PLATFORM_AMD__", "-I", "/opt/rocm/include", SYS_SRC, "-o", SYS_BIN],
+         "g++ (test_systematic)")
+    return SYS_BIN
+
+
 def build_sanitize_test() -> str:
     import tempfile
     csrc = os.path.join(PKG, "csrc")
@@ -67,6 +76,7 @@ def build_sanitize_test() -> str:
 def build() -> None:
     build_host_api_test()
     build_adjoint_local_test()
+    build_systematic_test()
     build_sanitize_test()
 
 
