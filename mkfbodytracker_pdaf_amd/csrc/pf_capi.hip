@@ -90,6 +90,8 @@ struct pf_handle {
     unsigned long long *cloc = nullptr, *bsum = nullptr;
     double *bexp = nullptr;
     int *bpow = nullptr;
+    unsigned long long *gpre = nullptr;   // prefix of the block sums (k_prefix)
+    int *gshf = nullptr;
     int Lcap = 0;
     unsigned long long *cloc1 = nullptr, *bsum1 = nullptr;
     double *bexp1 = nullptr;
@@ -155,12 +157,17 @@ int ensure_resample_scratch(pf_handle *h, int L)
     (void)hipFree(h->bsum);
     (void)hipFree(h->bexp);
     (void)hipFree(h->bpow);
-    h->cloc = nullptr; h->bsum = nullptr; h->bexp = nullptr; h->bpow = nullptr;
+    (void)hipFree(h->gpre);
+    (void)hipFree(h->gshf);
+    h->cloc = nullptr; h->bsum = nullptr; h->bexp = nullptr; h->bpow = nullptr; h->gpre = nullptr; h->gshf = nullptr;
+    h->Lcap = 0;
     const int nb = (L + kWeightsBlock - 1) / kWeightsBlock;
     HIP_TRY(dalloc(&h->cloc, (size_t)L));
     HIP_TRY(dalloc(&h->bsum, (size_t)nb));
     HIP_TRY(dalloc(&h->bexp, (size_t)nb));
     HIP_TRY(dalloc(&h->bpow, (size_t)nb));
+    HIP_TRY(dalloc(&h->gpre, (size_t)nb + 1));
+    HIP_TRY(dalloc(&h->gshf, (size_t)nb));
     h->Lcap = L;
     return PF_OK;
 }
@@ -370,6 +377,11 @@ int launch_weights(pf_handle *h, const uint32_t *uni, int parity)
     return check_launch("k_weights");
 }
 
+// Above this many input blocks (262,144 weights) the ancestors take their
+// prefix from k_prefix: two launches, against one whose every block repeats it
+// (14 us per call at 391 input blocks, where k_ancestors takes 7).
+constexpr int kPrefixBlocks = 1024;
+
 // Materialise the pending resampling of L weights into N ancestors.  The log
 // mean weight goes to lml, or to lml[*lml_frame] when a frame counter is given.
 int launch_ancestors(pf_handle *h, int L, int N, int *out, int parity, int kind_linear, double *lml,
@@ -385,6 +397,12 @@ int launch_ancestors(pf_handle *h, int L, int N, int *out, int parity, int kind_
     an.N = N;
     an.parity = parity;
     an.kind_linear = kind_linear;
+    if (an.pend.nb > kPrefixBlocks) {
+        hipLaunchKernelGGL(k_prefix, dim3(1), dim3(kPrefixThreads), 0, h->stream, an, h->gpre, h->gshf);
+        hipLaunchKernelGGL(k_ancestors_prefixed, dim3((N + 255) / 256), dim3(256), 0, h->stream, an,
+                           (const unsigned long long *)h->gpre, (const int *)h->gshf);
+        return check_launch("k_ancestors_prefixed");
+    }
     const size_t lds = 8 * (size_t)resolve_lds_words(an.pend.nb);
     hipLaunchKernelGGL(k_ancestors, dim3((N + 255) / 256), dim3(256), lds, h->stream, an);
     return check_launch("k_ancestors");
@@ -431,6 +449,17 @@ StepArgs step_args(pf_handle *h, int mode, const uint32_t *uni, const float *Z, 
     a.b0 = (float)(1.0 - h->cfg.p_detect * pg);
     a.gate = (float)h->cfg.gate_chi2;
     return a;
+}
+
+// Has the step (256-thread blocks) write its frame's resampler weights to
+// scratch set 0 and the next frame's index to the other counter.
+void write_weights(pf_handle *h, StepArgs &a, int p)
+{
+    a.w_cloc = h->cloc;
+    a.w_bsum = h->bsum;
+    a.w_bexp = h->bexp;
+    a.w_bpow = h->bpow;
+    a.frame_next = h->frame + (1 - p);
 }
 
 void swap_state(pf_handle *h)
@@ -596,11 +625,7 @@ AncArgs frame_anc_args(pf_handle *h, int p, double *lml)
 bool fuse_step_weights(pf_handle *h, StepArgs &a, int p)
 {
     if ((h->cfg.block_size > 0 ? h->cfg.block_size : 256) != kWeightsBlock) return false;
-    a.w_cloc = h->cloc;
-    a.w_bsum = h->bsum;
-    a.w_bexp = h->bexp;
-    a.w_bpow = h->bpow;
-    a.frame_next = h->frame + (1 - p);
+    write_weights(h, a, p);
     return true;
 }
 
@@ -794,7 +819,7 @@ int pf_destroy(pf_handle *h)
     drop_graphs(h);
     void *ptrs[] = {h->run_desc, h->run_ctr, h->rec[0], h->rec[1], h->anc, h->comp, h->bins, h->lw, h->table,
                     h->mu, h->sig, h->fs, h->frame, h->uni, h->lml1, h->cloc, h->bsum, h->bexp, h->bpow,
-                    h->cloc1, h->bsum1, h->bexp1, h->bpow1, h->zbuf, h->cntbuf, h->candbuf, h->est_partial, h->est_out, h->gbuf, h->ibuf,
+                    h->gpre, h->gshf, h->cloc1, h->bsum1, h->bexp1, h->bpow1, h->zbuf, h->cntbuf, h->candbuf, h->est_partial, h->est_out, h->gbuf, h->ibuf,
                     h->Tdev, h->Tinv};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -1180,8 +1205,18 @@ int ensure_events(pf_handle *h, size_t need)
     return PF_OK;
 }
 
-// Frames whose model image and resolver workspace do not fit one workgroup's
-// LDS: step, weights and ancestor launches per frame, launched one by one.
+// Up to this many input blocks a frame is one launch that resolves its own
+// ancestors; above, every block's prefix and the search's latency at two
+// waves per SIMD cost more than two more launches.  Per frame (d = 12, 8
+// detections per hand), one launch against step, k_prefix and
+// k_ancestors_prefixed: N = 200k 44.4 / 47.5 us, 262k 52.1 / 54.5, 400k 95.2 /
+// 91.9, 524k 132 / 121, 650k 155 / 139; N = 1M (step, weights and k_ancestors
+// launches before) 337 / 200.
+constexpr int kFusedBlocks = 1024;
+
+// Frames of many input blocks, or whose model image and resolver workspace do
+// not fit one workgroup's LDS: step and ancestor launches per frame, launched
+// one by one.
 int run_frames_split(pf_handle *h, int T, int mode, const float *Z, const int *count, const float *cand,
                      const uint32_t *uniforms, double *lml, bool timing, bool run_timing)
 {
@@ -1194,13 +1229,12 @@ int run_frames_split(pf_handle *h, int T, int mode, const float *Z, const int *c
     for (int f = 0; f < T; ++f) {
         const int parity = f & 1;
         StepArgs a = step_args(h, mode, uniforms, Z, zstride, h->N, count, cand, nullptr, parity, kAncArray, lml);
+        write_weights(h, a, parity);
         if (timing) HIP_TRY(hipEventRecord(h->ev[2 * f], h->stream));
-        st = launch_step(h, a, mode);
+        st = launch_step_block(h, a, mode, kWeightsBlock);
         if (st) return st;
         if (timing) HIP_TRY(hipEventRecord(h->ev[2 * f + 1], h->stream));
-        st = launch_weights(h, uniforms, parity);
-        if (st) return st;
-        // counter f & 1 still holds this frame's index (k_weights wrote the
+        // counter f & 1 still holds this frame's index (the step wrote the
         // next one into the other counter)
         st = launch_ancestors(h, h->N, h->N, h->anc, parity, 0, lml, h->frame + parity);
         if (st) return st;
@@ -1228,13 +1262,14 @@ static int run_frames(pf_handle *h, int T, int mode, const float *Z, const int *
     h->graph_frames = 0;
     st = ensure_events(h, timing ? 2 * (size_t)T + 2 : 2);
     if (st) return st;
-    // A frame is one step launch when the step's LDS holds the model image,
+    // A frame is one step launch when it has few enough input blocks and the
+    // step's LDS holds the model image,
     // the frame's detections and the resolver's workspace: it resolves its
     // ancestors from the previous frame's resampler weights and writes its
     // own.  Otherwise the frame runs as separate launches, without graphs.
     const int nbp = (h->N + kWeightsBlock - 1) / kWeightsBlock;
     const int stage = h->table_floats + (mode == kModeCand ? cand_lds_floats(h->J, h->cap) : 0);
-    const bool fused = step_lds_bytes_rec(h->lay.row == 1, stage, nbp) <= kMaxLdsBytes;
+    const bool fused = nbp <= kFusedBlocks && step_lds_bytes_rec(h->lay.row == 1, stage, nbp) <= kMaxLdsBytes;
     if (!fused) {
         st = run_frames_split(h, T, mode, Z, count, cand, uniforms, lml, timing, run_timing);
     } else {

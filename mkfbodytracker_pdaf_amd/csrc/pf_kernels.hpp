@@ -418,15 +418,14 @@ __device__ __forceinline__ unsigned long long resolve_prefix(const Pending &pd, 
 }
 
 // Phase 2: a_j for outputs j in [j0, j0 + blockDim) (j = j0 + threadIdx.x),
-// given the prefix of phase 1.  Every thread of the block must call it.
-__device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned long long total, int j0,
-                              unsigned long long *w)
+// given the prefix of phase 1: pre(b) the aligned prefix before input block b
+// and shf(b) its shift, stg the LDS stage (pd.stage words) and misc 16 LDS
+// words.  Every thread of the block must call it.
+template <typename PRE, typename SHF>
+__device__ __forceinline__ int resolve_search_in(const Pending &pd, int N, uint32_t U, unsigned long long total, int j0,
+                                                 PRE pre, SHF shf, unsigned long long *stg, unsigned long long *misc)
 {
     const int tid = threadIdx.x, nt = blockDim.x, nb = pd.nb;
-    unsigned long long *pre = w;
-    unsigned long long *stg = w + nb + 1;
-    unsigned long long *misc = stg + pd.stage;
-    const int *shf = reinterpret_cast<const int *>(misc + 16);
     const int bs = 1 << pd.bshift;
     // 2. the input block of each output: largest b with pre[b] <= f_j
     const int j = j0 + tid;
@@ -456,8 +455,8 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
         while (flo < fhi || llo < lhi) {
             const int fs = (fhi - flo + 64) >> 6, ls = (lhi - llo + 64) >> 6;
             const int fp = min(flo + lane * fs, fhi), lp = min(llo + lane * ls, lhi);
-            const int fc = __popcll(__ballot(pre[fp] <= ff));
-            const int lc = __popcll(__ballot(pre[lp] <= fl));
+            const int fc = __popcll(__ballot(pre(fp) <= ff));
+            const int lc = __popcll(__ballot(pre(lp) <= fl));
             const int fn = min(flo + (fc - 1) * fs, fhi), ln = min(llo + (lc - 1) * ls, lhi);
             fhi = fc < 64 ? min(flo + fc * fs, fhi) - 1 : fhi;
             lhi = lc < 64 ? min(llo + lc * ls, lhi) - 1 : lhi;
@@ -469,7 +468,7 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
     }
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
-        if (pre[mid] <= fj) lo = mid;
+        if (pre(mid) <= fj) lo = mid;
         else hi = mid - 1;
     }
     const int bj = lo;
@@ -496,7 +495,7 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
                 const int k = k0 + u * nt;
                 if (k < n) {
                     const int b = blo + (k >> pd.bshift);
-                    stg[k] = pre[b] + (pd.bpow ? shr64(c4[u], shf[b]) : c4[u]);
+                    stg[k] = pre(b) + (pd.bpow ? shr64(c4[u], shf(b)) : c4[u]);
                 }
             }
         }
@@ -509,8 +508,8 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
         }
         a = base + l;
     } else {
-        const unsigned long long pb = pre[bj];
-        const int sh = pd.bpow ? shf[bj] : 0;
+        const unsigned long long pb = pre(bj);
+        const int sh = pd.bpow ? shf(bj) : 0;
         int l = bj * bs, h = min(pd.L, (bj + 1) * bs) - 1;
         while (l < h) {
             const int mid = (l + h) >> 1;
@@ -520,6 +519,18 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
         a = l;
     }
     return a;
+}
+
+// Phase 2 with the prefix of resolve_prefix in LDS.
+__device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned long long total, int j0,
+                              unsigned long long *w)
+{
+    const unsigned long long *pre = w;
+    unsigned long long *stg = w + pd.nb + 1;
+    unsigned long long *misc = stg + pd.stage;
+    const int *shf = reinterpret_cast<const int *>(misc + 16);
+    return resolve_search_in(pd, N, U, total, j0, [=](int b) { return pre[b]; }, [=](int b) { return shf[b]; }, stg,
+                             misc);
 }
 
 // The frame statistics of a resolved resampling: the largest block exponent
@@ -1640,6 +1651,110 @@ static __global__ void __launch_bounds__(256) k_ancestors(AncArgs a)
     if (blockIdx.x == 0 && threadIdx.x == 0)
         finish_resampling(a.fs, a.parity, es, rs, a.N, a.kind_linear,
                           (a.lml && a.lml_frame) ? a.lml + *a.lml_frame : a.lml);
+}
+
+// The ancestors of many input blocks.  k_ancestors has every block of 256
+// outputs repeat the prefix of all block sums, and its LDS (12 bytes per
+// input block) leaves two blocks per CU to hide the search's dependent
+// probes: bound by that latency, 146 us at 10^6 weights (3907 input blocks).
+// Here one block takes the prefix once (k_prefix, 8.6 us) and the outputs'
+// blocks read it from global memory with only the search's stage in LDS
+// (eight blocks per CU): 13.9 us.
+constexpr int kPrefixThreads = 1024;
+constexpr int kPrefixPer = kMaxScanBlocks / kPrefixThreads;   // input blocks per thread
+constexpr int kPrefixStage = 8 * kWeightsBlock;               // LDS elements of the staged search
+
+// The aligned prefix of all block sums: pre[0 .. nb] (pre[nb] the total) and
+// each block's shift, and the statistics of the resampled frame.
+static __global__ void __launch_bounds__(kPrefixThreads) k_prefix(AncArgs a, unsigned long long *pre, int *shf)
+{
+    __shared__ double s_v[kMaxScanBlocks];
+    __shared__ unsigned long long s_wave[kPrefixThreads / 64];
+    __shared__ int s_max[kPrefixThreads / 64];
+    const Pending pd = anc_pending(a);
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nb = pd.nb;
+    const int c0 = tid * kPrefixPer;
+    unsigned long long s[kPrefixPer];
+    double v[kPrefixPer];
+    int e[kPrefixPer];
+#pragma unroll
+    for (int u = 0; u < kPrefixPer; ++u) {
+        const bool in = c0 + u < nb;
+        s[u] = in ? pd.bsum[c0 + u] : 0ull;
+        e[u] = in && pd.bpow ? pd.bpow[c0 + u] : kPowEmpty;
+        v[u] = in && a.lml ? pd.bexp[c0 + u] : 0.0;
+    }
+    int E = 0;
+    if (pd.bpow) {
+        int m = kPowEmpty;
+#pragma unroll
+        for (int u = 0; u < kPrefixPer; ++u) m = max(m, e[u]);
+        m = max(m, xor_lane<32>(m));
+        m = max(m, xor_lane<16>(m));
+        m = max(m, xor_lane<8>(m));
+        m = max(m, xor_lane<4>(m));
+        m = max(m, xor_lane<2>(m));
+        m = max(m, xor_lane<1>(m));
+        if (lane == 0) s_max[wid] = m;
+        __syncthreads();
+        E = s_max[0];
+#pragma unroll
+        for (int w = 1; w < kPrefixThreads / 64; ++w) E = max(E, s_max[w]);
+    }
+    unsigned long long loc = 0;
+    int sh[kPrefixPer];
+#pragma unroll
+    for (int u = 0; u < kPrefixPer; ++u) {
+        sh[u] = pd.bpow ? pow_shift(E, e[u]) : 0;
+        s[u] = shr64(s[u], sh[u]);
+        loc += s[u];
+        if (pd.bpow) v[u] = e[u] != kPowEmpty ? ldexp(v[u], e[u] - E) : 0.0;
+        s_v[c0 + u] = v[u];
+    }
+    const unsigned long long sc = wave_incl_scan(loc);
+    if (lane == 63) s_wave[wid] = sc;
+    __syncthreads();
+    unsigned long long run = sc - loc, total = 0;
+#pragma unroll
+    for (int w = 0; w < kPrefixThreads / 64; ++w) {
+        if (w < wid) run += s_wave[w];
+        total += s_wave[w];
+    }
+#pragma unroll
+    for (int u = 0; u < kPrefixPer; ++u)
+        if (c0 + u < nb) {
+            pre[c0 + u] = run;
+            shf[c0 + u] = sh[u];
+            run += s[u];
+        }
+    if (wid == 0) {
+        // the FP64 weight sum in resolve_prefix's order
+        double es = 0.0;
+        for (int k = lane; k < nb; k += 64) es += s_v[k];
+        es = wave_sum(es);
+        if (tid == 0) {
+            pre[nb] = total;
+            ResolveStats st;
+            st.total = total;
+            st.pow = E;
+            finish_resampling(a.fs, a.parity, es, st, a.N, a.kind_linear,
+                              (a.lml && a.lml_frame) ? a.lml + *a.lml_frame : a.lml);
+        }
+    }
+}
+
+static __global__ void __launch_bounds__(256) k_ancestors_prefixed(AncArgs a, const unsigned long long *pre,
+                                                                   const int *shf)
+{
+    __shared__ unsigned long long s_stage[kPrefixStage];
+    __shared__ unsigned long long s_misc[16];
+    Pending pd = a.pend;
+    pd.stage = kPrefixStage;
+    const int j0 = blockIdx.x * blockDim.x, j = j0 + (int)threadIdx.x;
+    const unsigned long long total = gload(pre + pd.nb);
+    const int src = resolve_search_in(pd, a.N, a.fs->U_pending, total, j0, [=](int b) { return gload(pre + b); },
+                                      [=](int b) { return gload(shf + b); }, s_stage, s_misc);
+    if (j < a.N) a.anc[j] = src;
 }
 
 // block maximum of FP64 host weights (for the stand-alone resample entry points)
