@@ -867,11 +867,10 @@ int pf_batch_reset(pf_batch *b, int32_t s, const int32_t *bins)
     for (int j = 0; j < sd.N; ++j)
         if (bins[j] < 0 || bins[j] >= b->K) return set_error(PF_ERR_ARG, "bins[%d] out of range", j);
     HIP_TRYB(hipMemcpyAsync(b->rec_bins + sd.pofs, bins, sizeof(int) * sd.N, hipMemcpyHostToDevice, b->stream));
-    auto reset_kernel = b->D == 24 ? k_reset<24> : k_reset<kBD>;
-    hipLaunchKernelGGL(reset_kernel, dim3((sd.N + 255) / 256), dim3(256), 0, b->stream, b->rec_bins + sd.pofs,
-                       b->mus + (size_t)i * b->K * b->D, b->sigs + (size_t)i * b->K * npacked(b->D),
-                       b->bx[0] + sd.pofs, b->bP[0] + sd.pofs, sd.N, Lay{b->ld, 1});
-    hipLaunchKernelGGL(k_identity_seq, dim3((sd.N + 255) / 256), dim3(256), 0, b->stream, b->anc, sd.pofs, sd.N);
+    auto reset = b->D == 24 ? launch_reset<24> : launch_reset<kBD>;
+    reset(b->stream, b->rec_bins + sd.pofs, b->mus + (size_t)i * b->K * b->D,
+          b->sigs + (size_t)i * b->K * npacked(b->D), b->bx[0] + sd.pofs, b->bP[0] + sd.pofs, b->anc + sd.pofs, sd.N,
+          Lay{b->ld, 1});
     HIP_TRYB(hipGetLastError());
     HIP_TRYB(hipStreamSynchronize(b->stream));
     b->fresh[s] = 1;

@@ -294,8 +294,7 @@ template <int D>
 struct ResetL {
     static void run(pf_handle *h)
     {
-        hipLaunchKernelGGL((k_reset<D>), dim3((h->N + 255) / 256), dim3(256), 0, h->stream, h->bins,
-                           h->mu, h->sig, h->xA, h->PA, h->N, h->lay);
+        launch_reset<D>(h->stream, h->bins, h->mu, h->sig, h->xA, h->PA, h->anc, h->N, h->lay);
     }
 };
 
@@ -891,8 +890,8 @@ int pf_reset(pf_handle *h, const int32_t *bins)
         if (bins[j] < 0 || bins[j] >= h->K) return set_error(PF_ERR_ARG, "bins[%d]=%d out of range", j, bins[j]);
     HIP_TRY(hipMemcpyAsync(h->bins, bins, sizeof(int) * h->N, hipMemcpyHostToDevice, h->stream));
     st = dispatch_d<ResetL>(h->D, h);
+    if (!st) st = check_launch("k_reset");
     if (st) return st;
-    hipLaunchKernelGGL(k_iota, dim3((h->N + 255) / 256), dim3(256), 0, h->stream, h->anc, h->N);
     HIP_TRY(hipStreamSynchronize(h->stream));
     h->tracks = true;
     return PF_OK;
