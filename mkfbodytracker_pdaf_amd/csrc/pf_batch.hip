@@ -59,6 +59,7 @@ __device__ __forceinline__ void tile_ancestors(const BatchArgs &a, const SeqDesc
     for (int r = 0; r < PPL; ++r) {
         src[r] = 0;
         if (jt0 + r * bd >= sd.N) continue;        // block-uniform: no barrier is skipped by part of the block
+        if (r > 0) __syncthreads();                // the previous search's stage is free
         src[r] = resolve_search(pd, sd.N, U, total, jt0 + r * bd, wsp);
         const int j = jt0 + r * bd + (int)threadIdx.x;
         if (j < sd.N) {

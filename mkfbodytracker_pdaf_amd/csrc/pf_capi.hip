@@ -217,7 +217,8 @@ int launch_step_dj(pf_handle *h, const StepArgs &a, int mode, int block)
 {
     const bool rec = h->lay.row == 1;
     const size_t lds = (size_t)step_lds_bytes_rec(rec, a.stage_floats, a.anc_mode == kAncFused ? a.pend.nb : 0);
-    const int grid = (h->N + block - 1) / block;
+    // fused launches have one more block, for the frame's statistics
+    const int grid = (h->N + block - 1) / block + (a.anc_mode == kAncFused ? 1 : 0);
     if constexpr (rec_layout(D)) {
         if (rec) {
             if (mode == kModeRef)
@@ -1152,16 +1153,11 @@ StepArgs run_step_args(pf_handle *h, int mode, int p)
     a.Pin = h->Pbuf[0];
     a.xout = h->xbuf[1];
     a.Pout = h->Pbuf[1];
-    a.pend = pending_of(h, h->N, true, 1);     // even frames resolve set 1
-    a.pend1 = pending_of(h, h->N, true, 0);    // odd frames resolve set 0
-    a.w_cloc = h->cloc;
-    a.w_bsum = h->bsum;
-    a.w_bexp = h->bexp;
-    a.w_bpow = h->bpow;
-    a.w1_cloc = h->cloc1;
-    a.w1_bsum = h->bsum1;
-    a.w1_bexp = h->bexp1;
-    a.w1_bpow = h->bpow1;
+    a.pend = pending_of(h, h->N, true, 1 - p);   // the other parity's weights are resolved
+    a.w_cloc = p ? h->cloc1 : h->cloc;
+    a.w_bsum = p ? h->bsum1 : h->bsum;
+    a.w_bexp = p ? h->bexp1 : h->bexp;
+    a.w_bpow = p ? h->bpow1 : h->bpow;
     return a;
 }
 

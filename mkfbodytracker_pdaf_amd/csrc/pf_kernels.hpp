@@ -204,18 +204,14 @@ struct StepArgs {
     double *w_bexp;
     int *w_bpow;
     int *frame_next;
-    // Device-resident runs (run != null): the frame t = *frame (block 0 writes
-    // t + 1 to *frame_next) chooses everything else in the kernel: the state
+    // Device-resident runs (run != null; kAncFused): the frame t = *frame, of
+    // the launch's parity (block 0 writes t + 1 to *frame_next).  The state
     // buffer read is (t + run->flip) & 1 (xin/Pin = buffer 0, xout/Pout =
-    // buffer 1) and the other is written; frame t writes its resampler
-    // weights to set t & 1 (w_* = set 0, w1_* = set 1) and resolves frame
-    // t - 1's from the other set (pend views set 1, pend1 set 0); frame 0
-    // reads the ancestor array.  Inputs come from *run.
+    // buffer 1) and the other is written; frame t writes its resampler weights
+    // to set t & 1 and resolves frame t - 1's from the other set (both chosen
+    // by the launch's parity, so the resolver's first loads need not wait for
+    // t); frame 0 reads the ancestor array.  Inputs come from *run.
     const RunDesc *run;
-    Pending pend1;
-    unsigned long long *w1_cloc, *w1_bsum;
-    double *w1_bexp;
-    int *w1_bpow;
 };
 
 // The StepArgs of frame t of a device-resident run (see StepArgs::run), with
@@ -233,15 +229,7 @@ __device__ __forceinline__ StepArgs frame_args(const StepArgs &ain, int &t)
         a.xout = const_cast<float *>(x0);
         a.Pout = const_cast<float *>(P0);
     }
-    if (t & 1) {
-        a.w_cloc = a.w1_cloc;
-        a.w_bsum = a.w1_bsum;
-        a.w_bexp = a.w1_bexp;
-        a.w_bpow = a.w1_bpow;
-        a.pend = a.pend1;
-    }
     a.anc_mode = (t == 0) ? kAncArray : kAncFused;
-    a.parity = t & 1;
     a.Z = rd.Z;
     a.count = rd.count;
     a.cand = rd.cand;
@@ -308,43 +296,73 @@ struct NoHook {
     __device__ void operator()() const {}
 };
 
-// Phase 1 of the ancestor resolution: the largest block exponent E, the
-// exclusive prefix of the aligned block sums in LDS (pre[0..nb], pre[nb] =
-// total) with each block's shift, and, if want_es, the FP64 sum of the block
-// weight sums scaled to 2^E in es.  Every thread of the block must call it
-// (want_es block-uniform).  hook() runs once the block sums' loads are
-// issued: a caller's own loads placed there share their latency.
+// Up to kPrefixReg consecutive block sums and exponents of a thread, kept in
+// registers from one round of bounds-checked loads (blocks outside the
+// thread's share count as empty).
+constexpr int kPrefixReg = 4;
+struct PrefixRegs {
+    unsigned long long s[kPrefixReg];
+    int e[kPrefixReg];
+};
+
+// Input blocks per thread of the prefix.
+__device__ __forceinline__ int prefix_per(const Pending &pd) { return (pd.nb + blockDim.x - 1) / blockDim.x; }
+
+// Blocks c0 + first .. of the thread's share of `per` blocks (first a
+// multiple of kPrefixReg).
+__device__ __forceinline__ void prefix_load(const Pending &pd, int per, int first, PrefixRegs &r)
+{
+    const int c = (int)threadIdx.x * per + first, n = min(per - first, pd.nb - c);
+    const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<unsigned long long *>(pd.bsum), (short)0, pd.nb * 8, 0x00020000);
+    const __amdgpu_buffer_rsrc_t re =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<int *>(pd.bpow), (short)0, pd.bpow ? pd.nb * 4 : 0, 0x00020000);
+#pragma unroll
+    for (int u = 0; u < kPrefixReg; ++u) {
+        r.s[u] = 0ull;
+        r.e[u] = kPowEmpty;
+        if (first + u < per) {            // the same for every thread
+            r.s[u] = __builtin_bit_cast(unsigned long long, __builtin_amdgcn_raw_buffer_load_b64(rs, (c + u) * 8, 0, 0));
+            r.e[u] = __builtin_amdgcn_raw_buffer_load_b32(re, (c + u) * 4, 0, 0);
+        }
+    }
+#pragma unroll
+    for (int u = 0; u < kPrefixReg; ++u)
+        if (u >= n) {
+            r.s[u] = 0ull;
+            r.e[u] = kPowEmpty;
+        }
+}
+
+// Phase 1 of the ancestor resolution: the exclusive prefix of the aligned
+// block sums in LDS (pre[0..nb], pre[nb] = total) with each block's shift,
+// and, if want_es, the FP64 sum of the block weight sums scaled to 2^E in es.
+// r holds the first blocks of the thread's share (prefix_load); E is the
+// largest block exponent if have_pow, else it is reduced here (0 without
+// exponents).  Every thread of the block must call it (want_es
+// block-uniform).  hook() runs before the first use of r: a caller's own loads
+// placed there share their latency.
 template <typename Hook = NoHook>
-__device__ __forceinline__ unsigned long long resolve_prefix(const Pending &pd, unsigned long long *w, bool want_es,
-                                                             double &es_out, int &pow_out, Hook hook = Hook())
+__device__ __forceinline__ unsigned long long resolve_prefix_from(const Pending &pd, unsigned long long *w, int per,
+                                                                  PrefixRegs &r, bool have_pow, int E, bool want_es,
+                                                                  double &es_out, int &pow_out, Hook hook = Hook())
 {
     const int tid = threadIdx.x, nt = blockDim.x, nb = pd.nb;
-    const int lane = tid & 63, wid = tid >> 6, nwaves = (nt + 63) >> 6;
+    const int lane = tid & 63, wid = tid >> 6, nwaves = nt >> 6;
     unsigned long long *pre = w;
     unsigned long long *stg = w + nb + 1;
     unsigned long long *misc = stg + pd.stage;
     int *shf = reinterpret_cast<int *>(misc + 16);
-    const int per = (nb + nt - 1) / nt;
-    const int c0 = min(nb, tid * per), c1 = min(nb, c0 + per);
-    // A thread's blocks c0 .. c1 - 1; up to 8 of them stay in registers from
-    // one round of loads (more are loaded again in each pass).
-    constexpr int kReg = 8;
-    unsigned long long rs[kReg];
-    int re[kReg];
-#pragma unroll
-    for (int u = 0; u < kReg; ++u) {
-        rs[u] = (c0 + u < c1) ? pd.bsum[c0 + u] : 0ull;
-        re[u] = (pd.bpow && c0 + u < c1) ? pd.bpow[c0 + u] : kPowEmpty;
-    }
-    // 0. E, the largest block exponent (0 without exponents)
-    int E = 0;
-    if (pd.bpow && pd.pow_max) E = gload(pd.pow_max);
+    const int c0 = tid * per;
     hook();
-    if (pd.bpow && !pd.pow_max) {
+    if (pd.bpow && !have_pow) {
         int em = kPowEmpty;
+        PrefixRegs q = r;
+        for (int k = 0; k < per; k += kPrefixReg) {
+            if (k) prefix_load(pd, per, k, q);
 #pragma unroll
-        for (int u = 0; u < kReg; ++u) em = max(em, re[u]);
-        for (int k = c0 + kReg; k < c1; ++k) em = max(em, pd.bpow[k]);
+            for (int u = 0; u < kPrefixReg; ++u) em = max(em, q.e[u]);
+        }
         em = max(em, xor_lane<32>(em));
         em = max(em, xor_lane<16>(em));
         em = max(em, xor_lane<8>(em));
@@ -357,15 +375,21 @@ __device__ __forceinline__ unsigned long long resolve_prefix(const Pending &pd, 
         E = kPowEmpty;
         for (int k = 0; k < nwaves; ++k) E = max(E, (int)(long long)misc[8 + k]);
     }
-    auto shift_of = [&](int e) { return pd.bpow ? pow_shift(E, e) : 0; };
-    // 1. the aligned block sums of this thread's blocks
+    // E >= e, so the shift of a block that is not empty is their difference
+    const auto shift_of = [&](int e) {
+        return !pd.bpow ? 0 : (e == kPowEmpty ? 64 : (int)min((unsigned)E - (unsigned)e, 64u));
+    };
+    // the aligned block sums of this thread's blocks
     unsigned long long loc = 0;
+    {
+        PrefixRegs q = r;
+        for (int k = 0; k < per; k += kPrefixReg) {
+            if (k) prefix_load(pd, per, k, q);
 #pragma unroll
-    for (int u = 0; u < kReg; ++u)
-        if (c0 + u < c1) loc += shr64(rs[u], shift_of(re[u]));
-    for (int k = c0 + kReg; k < c1; ++k) loc += shr64(pd.bsum[k], shift_of(pd.bpow ? pd.bpow[k] : 0));
-    unsigned long long sc = loc;
-    sc = wave_incl_scan(sc);
+            for (int u = 0; u < kPrefixReg; ++u) loc += shr64(q.s[u], shift_of(q.e[u]));
+        }
+    }
+    const unsigned long long sc = wave_incl_scan(loc);
     // FP64 weight sum in an order fixed by nb alone (lane l of wave 0 takes
     // blocks l, l + 64, ...), so it does not depend on the block size; block
     // b's sum is relative to 2^e_b and scaled to 2^E (exactly).
@@ -397,19 +421,16 @@ __device__ __forceinline__ unsigned long long resolve_prefix(const Pending &pd, 
     unsigned long long total = 0;
     for (int k = 0; k < nwaves; ++k) total += misc[k];
     if (want_es) es_out = reinterpret_cast<double *>(stg)[0];
+    for (int k = 0; k < per; k += kPrefixReg) {
+        if (k) prefix_load(pd, per, k, r);
 #pragma unroll
-    for (int u = 0; u < kReg; ++u)
-        if (c0 + u < c1) {
-            const int sh = shift_of(re[u]);
-            pre[c0 + u] = run;
-            shf[c0 + u] = sh;
-            run += shr64(rs[u], sh);
-        }
-    for (int k = c0 + kReg; k < c1; ++k) {
-        const int sh = shift_of(pd.bpow ? pd.bpow[k] : 0);
-        pre[k] = run;
-        shf[k] = sh;
-        run += shr64(pd.bsum[k], sh);
+        for (int u = 0; u < kPrefixReg; ++u)
+            if (k + u < per && c0 + k + u < nb) {
+                const int sh = shift_of(r.e[u]);
+                pre[c0 + k + u] = run;
+                shf[c0 + k + u] = sh;
+                run += shr64(r.s[u], sh);
+            }
     }
     if (tid == 0) pre[nb] = total;
     __syncthreads();
@@ -417,13 +438,24 @@ __device__ __forceinline__ unsigned long long resolve_prefix(const Pending &pd, 
     return total;
 }
 
+template <typename Hook = NoHook>
+__device__ __forceinline__ unsigned long long resolve_prefix(const Pending &pd, unsigned long long *w, bool want_es,
+                                                             double &es_out, int &pow_out, Hook hook = Hook())
+{
+    const int per = prefix_per(pd);
+    PrefixRegs r;
+    prefix_load(pd, per, 0, r);
+    const bool have = pd.bpow && pd.pow_max;
+    return resolve_prefix_from(pd, w, per, r, have, have ? gload(pd.pow_max) : 0, want_es, es_out, pow_out, hook);
+}
+
 // Phase 2: a_j for outputs j in [j0, j0 + blockDim) (j = j0 + threadIdx.x),
 // given the prefix of phase 1: pre(b) the aligned prefix before input block b
-// and shf(b) its shift, stg the LDS stage (pd.stage words) and misc 16 LDS
-// words.  Every thread of the block must call it.
+// and shf(b) its shift, stg the LDS stage (pd.stage words; free when called).
+// Every thread of the block (a multiple of 64) must call it.
 template <typename PRE, typename SHF>
 __device__ __forceinline__ int resolve_search_in(const Pending &pd, int N, uint32_t U, unsigned long long total, int j0,
-                                                 PRE pre, SHF shf, unsigned long long *stg, unsigned long long *misc)
+                                                 PRE pre, SHF shf, unsigned long long *stg)
 {
     const int tid = threadIdx.x, nt = blockDim.x, nb = pd.nb;
     const int bs = 1 << pd.bshift;
@@ -439,45 +471,35 @@ __device__ __forceinline__ int resolve_search_in(const Pending &pd, int N, uint3
     // a_j is the first input whose prefix exceeds f_j (SysThresholds)
     const SysThresholds thr(total, U, (uint32_t)N);
     const unsigned long long fj = thr((uint32_t)jc);
-    int lo = 0, hi = nb - 1;
-    if ((nt & 63) == 0) {
-        // f_j grows with j, so every output's block lies between the blocks
-        // of the block's first and last outputs.  Each wave finds those two
-        // by 64-way searches: lane l probes position lo + l * step of the
-        // range (non-decreasing in l, lane 0 at a position known to pass),
-        // and the ballot's count of passing lanes narrows the range to one
-        // step (two levels up to 4096 input blocks, one LDS read per lane
-        // each).  The output's own search then covers that span only.
-        const int lane = tid & 63;
-        const int jl = min(j0 + nt, N) - 1;
-        const unsigned long long ff = thr((uint32_t)j0), fl = thr((uint32_t)jl);
-        int flo = 0, fhi = nb - 1, llo = 0, lhi = nb - 1;
-        while (flo < fhi || llo < lhi) {
-            const int fs = (fhi - flo + 64) >> 6, ls = (lhi - llo + 64) >> 6;
-            const int fp = min(flo + lane * fs, fhi), lp = min(llo + lane * ls, lhi);
-            const int fc = __popcll(__ballot(pre(fp) <= ff));
-            const int lc = __popcll(__ballot(pre(lp) <= fl));
-            const int fn = min(flo + (fc - 1) * fs, fhi), ln = min(llo + (lc - 1) * ls, lhi);
-            fhi = fc < 64 ? min(flo + fc * fs, fhi) - 1 : fhi;
-            lhi = lc < 64 ? min(llo + lc * ls, lhi) - 1 : lhi;
-            flo = fn;
-            llo = ln;
-        }
-        lo = flo;
-        hi = llo;
+    // f_j grows with j, so every output's block lies between the blocks of
+    // the block's first and last outputs.  Each wave finds those two by 64-way
+    // searches: lane l probes position lo + l * step of the range
+    // (non-decreasing in l, lane 0 at a position known to pass), and the
+    // ballot's count of passing lanes narrows the range to one step (two
+    // levels up to 4096 input blocks, one LDS read per lane each).  The
+    // output's own search then covers that span only.
+    const int lane = tid & 63;
+    const int jl = min(j0 + nt, N) - 1;
+    const unsigned long long ff = thr((uint32_t)j0), fl = thr((uint32_t)jl);
+    int blo = 0, fhi = nb - 1, bhi = 0, lhi = nb - 1;
+    while (blo < fhi || bhi < lhi) {
+        const int fs = (fhi - blo + 64) >> 6, ls = (lhi - bhi + 64) >> 6;
+        const int fp = min(blo + lane * fs, fhi), lp = min(bhi + lane * ls, lhi);
+        const int fc = __popcll(__ballot(pre(fp) <= ff));
+        const int lc = __popcll(__ballot(pre(lp) <= fl));
+        const int fn = min(blo + (fc - 1) * fs, fhi), ln = min(bhi + (lc - 1) * ls, lhi);
+        fhi = fc < 64 ? min(blo + fc * fs, fhi) - 1 : fhi;
+        lhi = lc < 64 ? min(bhi + lc * ls, lhi) - 1 : lhi;
+        blo = fn;
+        bhi = ln;
     }
+    int lo = blo, hi = bhi;
     while (lo < hi) {
         const int mid = (lo + hi + 1) >> 1;
         if (pre(mid) <= fj) lo = mid;
         else hi = mid - 1;
     }
     const int bj = lo;
-    const int jlast = min(j0 + nt, N) - 1;
-    __syncthreads();                     // stg / misc of a previous search are free
-    if (j == j0) misc[4] = (unsigned long long)bj;
-    if (j == jlast) misc[5] = (unsigned long long)bj;
-    __syncthreads();
-    const int blo = (int)misc[4], bhi = (int)misc[5];
     // 3. a span of input blocks that fits the stage (pd.stage elements) is
     //    staged in LDS (C = pre + aligned cloc, one memory latency) and
     //    searched there; wider spans (strongly concentrated weights) search
@@ -486,10 +508,14 @@ __device__ __forceinline__ int resolve_search_in(const Pending &pd, int N, uint3
     if (((bhi - blo + 1) << pd.bshift) <= pd.stage) {
         const int base = blo << pd.bshift;
         const int n = min(pd.L, (bhi + 1) << pd.bshift) - base;
-        for (int k0 = tid; k0 < n; k0 += 4 * nt) {      // 4 loads in flight per lane
+        const __amdgpu_buffer_rsrc_t rc = __builtin_amdgcn_make_buffer_rsrc(
+            const_cast<unsigned long long *>(pd.cloc + base), (short)0, n * 8, 0x00020000);
+        for (int k0 = tid; k0 < n; k0 += 4 * nt) {      // 4 bounds-checked loads in flight per lane
             unsigned long long c4[4];
 #pragma unroll
-            for (int u = 0; u < 4; ++u) c4[u] = (k0 + u * nt < n) ? pd.cloc[base + k0 + u * nt] : 0ull;
+            for (int u = 0; u < 4; ++u)
+                c4[u] = __builtin_bit_cast(unsigned long long,
+                                           __builtin_amdgcn_raw_buffer_load_b64(rc, (k0 + u * nt) * 8, 0, 0));
 #pragma unroll
             for (int u = 0; u < 4; ++u) {
                 const int k = k0 + u * nt;
@@ -527,10 +553,8 @@ __device__ int resolve_search(const Pending &pd, int N, uint32_t U, unsigned lon
 {
     const unsigned long long *pre = w;
     unsigned long long *stg = w + pd.nb + 1;
-    unsigned long long *misc = stg + pd.stage;
-    const int *shf = reinterpret_cast<const int *>(misc + 16);
-    return resolve_search_in(pd, N, U, total, j0, [=](int b) { return pre[b]; }, [=](int b) { return shf[b]; }, stg,
-                             misc);
+    const int *shf = reinterpret_cast<const int *>(stg + pd.stage + 16);
+    return resolve_search_in(pd, N, U, total, j0, [=](int b) { return pre[b]; }, [=](int b) { return shf[b]; }, stg);
 }
 
 // The frame statistics of a resolved resampling: the largest block exponent
@@ -540,12 +564,11 @@ struct ResolveStats {
     int pow;
 };
 
-// Both phases for one block of outputs (hook: as for resolve_prefix).
-template <typename Hook = NoHook>
+// Both phases for one block of outputs.
 __device__ __forceinline__ int resolve_ancestor(const Pending &pd, int N, uint32_t U, int j0, unsigned long long *w,
-                                                bool want_es, double &es_out, ResolveStats &st, Hook hook = Hook())
+                                                bool want_es, double &es_out, ResolveStats &st)
 {
-    st.total = resolve_prefix(pd, w, want_es, es_out, st.pow, hook);
+    st.total = resolve_prefix(pd, w, want_es, es_out, st.pow);
     return resolve_search(pd, N, U, st.total, j0, w);
 }
 
@@ -1407,8 +1430,35 @@ __device__ __forceinline__ void step_body(const StepArgs &ain)
 {
     constexpr int NP = npacked(D);
     extern __shared__ float4 sm4[];
+    // Fused launches: the previous frame's block sums and exponent maxima are
+    // loaded before anything the frame counter decides, without branches, and
+    // the frame's statistics are one extra block's work.  A frame is bound by
+    // this chain of dependent loads (its counter, the block sums, the scans,
+    // the gather) and by vector issue; with the sums loaded after the counter,
+    // eight guarded loads per thread, and block 0 also adding the FP64 weight
+    // sum, it took 17.9 us at N = 1000 and 24.5 at 100,000 against 15.6 and 22.9.
+    PrefixRegs pr;
+    const int per = prefix_per(ain.pend);
+    int pw[3] = {0, 0, 0};
+    if (ain.anc_mode == kAncFused) {
+#pragma unroll
+        for (int u = 0; u < 3; ++u) pw[u] = gload(&ain.fs->pow_max[u]);
+        prefix_load(ain.pend, per, 0, pr);
+    }
     int t;
     const StepArgs a = frame_args(ain, t);
+    if (ain.anc_mode == kAncFused && blockIdx.x == gridDim.x - 1) {
+        // the launch's extra block: the statistics of the consumed resampling
+        // (log mean weight, degenerate flag), off the particles' blocks
+        if (a.anc_mode != kAncFused) return;
+        const int m = (t + 2) % 3;
+        double es = 0.0;
+        ResolveStats rs;
+        rs.total = resolve_prefix_from(a.pend, reinterpret_cast<unsigned long long *>(sm4), per, pr, true,
+                                       m == 0 ? pw[0] : (m == 1 ? pw[1] : pw[2]), true, es, rs.pow);
+        if (threadIdx.x == 0) finish_resampling(a.fs, a.parity ^ 1, es, rs, a.N, 0, a.lml + (t - 1));
+        return;
+    }
     const uint32_t U1 = gload(a.uni + 2 * t);
     const int j0 = blockIdx.x * blockDim.x;
     const int j = j0 + threadIdx.x;
@@ -1429,20 +1479,17 @@ __device__ __forceinline__ void step_body(const StepArgs &ain)
     };
     int src;
     if (a.anc_mode == kAncFused) {
-        // Consume the previous frame's resampling: a_j, then the frame's
-        // statistics (block 0).
+        // the previous frame's resampling: its uniform and its largest block
+        // exponent (raised by its blocks)
         unsigned long long *wsp = reinterpret_cast<unsigned long long *>(
             reinterpret_cast<float *>(sm4) + a.stage_floats);
+        const int m = (t + 2) % 3;
         double es = 0.0;
-        ResolveStats rs;
-        // the previous frame's resampling uniform (its step recorded it as
-        // pending too) and its largest block exponent (raised by its blocks)
-        Pending pd = a.pend;
-        if (a.w_cloc) pd.pow_max = &a.fs->pow_max[(t - 1) % 3];
-        src = resolve_ancestor(pd, a.N, a.uni[2 * (t - 1) + 1], j0, wsp, blockIdx.x == 0, es, rs, prefetch);
+        int E;
+        const unsigned long long total = resolve_prefix_from(
+            a.pend, wsp, per, pr, true, m == 0 ? pw[0] : (m == 1 ? pw[1] : pw[2]), false, es, E, prefetch);
+        src = resolve_search(a.pend, a.N, gload(a.uni + 2 * (t - 1) + 1), total, j0, wsp);
         if (live) a.anc[j] = src;
-        if (blockIdx.x == 0 && threadIdx.x == 0)
-            finish_resampling(a.fs, a.parity ^ 1, es, rs, a.N, 0, a.lml ? a.lml + (t - 1) : nullptr);
     } else {
         prefetch();
         src = live ? a.anc[j] : 0;
@@ -1747,13 +1794,12 @@ static __global__ void __launch_bounds__(256) k_ancestors_prefixed(AncArgs a, co
                                                                    const int *shf)
 {
     __shared__ unsigned long long s_stage[kPrefixStage];
-    __shared__ unsigned long long s_misc[16];
     Pending pd = a.pend;
     pd.stage = kPrefixStage;
     const int j0 = blockIdx.x * blockDim.x, j = j0 + (int)threadIdx.x;
     const unsigned long long total = gload(pre + pd.nb);
     const int src = resolve_search_in(pd, a.N, a.fs->U_pending, total, j0, [=](int b) { return gload(pre + b); },
-                                      [=](int b) { return gload(shf + b); }, s_stage, s_misc);
+                                      [=](int b) { return gload(shf + b); }, s_stage);
     if (j < a.N) a.anc[j] = src;
 }
 
