@@ -6,7 +6,8 @@
  * sequentially (src/pfPose.cpp:325-326).  Every sequence here runs the same
  * algorithm as pf_step_candidates() of pf_rbpf.h (pf2DRao.cpp:125-158 with
  * the PDAF joint likelihood), with its own GMM, particle count and length.
- * One persistent step kernel and one weights kernel per frame serve all
+ * One step kernel (and one weights kernel, unless the step writes its own
+ * weights) per frame serves all
  * sequences still active at that frame; the frame loop is captured into a
  * hipGraph.  Tile size and persistence are picked by pf_batch_autotune().
  */
@@ -26,7 +27,7 @@ typedef struct pf_batch pf_batch;
 typedef struct pf_batch_schedule {
     int32_t block;          /* threads per tile: 64, 128 or 256 */
     int32_t ppl;            /* particles per lane per tile: 1 or 2 (tile = block * ppl) */
-    int32_t blocks_per_cu;  /* persistent grid = blocks_per_cu * CUs */
+    int32_t blocks_per_cu;  /* ppl = 2: persistent grid = blocks_per_cu * CUs (ppl = 1 has a block per tile) */
 } pf_batch_schedule;
 
 /* S sequences; sequence s has n_particles[s] particles and n_frames[s]

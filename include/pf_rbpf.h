@@ -159,7 +159,7 @@ int pf_get_sample_prob(pf_handle *h, const double *Hp, const double *M, int32_t 
  * the handle's first such run (the frames read the run's pointers from
  * device memory, so the graphs serve every later run of any length; they
  * are captured again after pf_load_model or pf_set_joint_clutter; runs of
- * more than 262,144 particles, whose frames are three longer launches each, are
+ * more than 435,200 particles, whose frames are three longer launches each, are
  * launched without graphs); bits 1
  * and 2 time the run (see
  * pf_last_run_kernel_time; bit 1 turns the graphs off).  Returns after

@@ -11,22 +11,16 @@ import subprocess
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.environ.get("MKFBT_LIB") or os.path.join(HERE, "libmkfbt.so")
-SOURCES = ["pf_capi.hip", "pf_model.cpp", "pf_io.cpp", "pf_host.cpp", "pf2d.hip", "pf_batch.hip", "pf_adjoint.hip", "pf_tracker.hip", "pf_noalloc.hip"]
+SOURCES = ["pf_capi.hip", "pf_step_rec.hip", "pf_step_rows.hip", "pf_model.cpp", "pf_io.cpp", "pf_host.cpp", "pf2d.hip", "pf_batch.hip", "pf_adjoint.hip", "pf_tracker.hip", "pf_noalloc.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 FLAGS = ["--offload-arch=gfx950", "-O3", "-std=c++17", "-fPIC", "-shared",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
+         # the joint loop of the widest kernels (8 joints of d = 16, two particles per
+         # lane) exceeds the default size for full unrolling, and the state of a loop
+         # that is not unrolled lives in scratch memory
+         "-mllvm", "-pragma-unroll-threshold=65536",
          "-Wall", "-Wno-unused-function", "-Wno-unused-command-line-argument"]
-# Per-source scheduler choice.  The memory-clause strategy groups each
-# kernel's independent loads into clauses.  On the source holding the
-# single-filter steps it shortens the tracker's paired filter step (frame
-# 99 -> 97.5 us) and leaves the single-sequence step unchanged; on the batched
-# engine's source it costs ~1% and on the proposal kernels' source ~0.5%, so
-# those keep the default.  Instruction order changes, the arithmetic does
-# not: results are bit-identical.
-SOURCE_FLAGS = {
-    "pf_capi.hip": ["-mllvm", "-amdgpu-sched-strategy=max-memory-clause"],
-}
 
 
 def sources():
@@ -48,8 +42,7 @@ def build(verbose: bool = False, jobs: int = 0) -> str:
 
         def compile_one(so):
             src, obj = so
-            extra = SOURCE_FLAGS.get(os.path.basename(src), [])
-            return subprocess.run([HIPCC, *cflags, *extra, *inc, "-c", src, "-o", obj], capture_output=True, text=True)
+            return subprocess.run([HIPCC, *cflags, *inc, "-c", src, "-o", obj], capture_output=True, text=True)
 
         n = jobs or min(len(srcs), os.cpu_count() or 1, 16)
         with ThreadPoolExecutor(max_workers=max(1, n)) as ex:

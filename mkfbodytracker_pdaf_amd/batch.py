@@ -3,7 +3,7 @@
 Each sequence runs the candidate-mode step of ``Rbpf.step_candidates``
 (src/pf2DRao.cpp:125-158 with the PDAF joint likelihood) with its own GMM,
 particle count and length; the reference runs one ParticleFilter per arm,
-one after the other (src/pfPose.cpp:325-326).  One persistent step kernel
+one after the other (src/pfPose.cpp:325-326).  One step kernel
 and one weights kernel per frame serve every sequence still active at that
 frame.
 """

@@ -18,6 +18,7 @@
 #include "pf_engine.hpp"
 #include "pf_kernels.hpp"
 #include "pf_model.hpp"
+#include "pf_step.hpp"
 
 using namespace mkfbt;
 
@@ -212,66 +213,10 @@ int check_launch(const char *what)
 }
 
 // ---------------------------------------------------------- kernel dispatch
-template <int D, int SELJ>
-int launch_step_dj(pf_handle *h, const StepArgs &a, int mode, int block)
-{
-    const bool rec = h->lay.row == 1;
-    const size_t lds = (size_t)step_lds_bytes_rec(rec, a.stage_floats, a.anc_mode == kAncFused ? a.pend.nb : 0);
-    // fused launches have one more block, for the frame's statistics
-    const int grid = (h->N + block - 1) / block + (a.anc_mode == kAncFused ? 1 : 0);
-    if constexpr (rec_layout(D)) {
-        if (rec) {
-            if (mode == kModeRef)
-                hipLaunchKernelGGL((k_step<D, kModeRef, SELJ, true>), dim3(grid), dim3(block), lds, h->stream, a);
-            else
-                hipLaunchKernelGGL((k_step<D, kModeCand, SELJ, true>), dim3(grid), dim3(block), lds, h->stream, a);
-            return check_launch("k_step");
-        }
-    }
-    if (mode == kModeRef)
-        hipLaunchKernelGGL((k_step<D, kModeRef, SELJ>), dim3(grid), dim3(block), lds, h->stream, a);
-    else
-        hipLaunchKernelGGL((k_step<D, kModeCand, SELJ>), dim3(grid), dim3(block), lds, h->stream, a);
-    return check_launch("k_step");
-}
-
-// Selection-basis kernels exist for every joint count J with 2J <= D.
-template <int D>
-int launch_step_d(pf_handle *h, const StepArgs &a, int mode, int block)
-{
-    if (!h->sel_mode) return launch_step_dj<D, 0>(h, a, mode, block);
-    switch (h->J) {
-    case 1: return launch_step_dj<D, 1>(h, a, mode, block);
-    case 2: return launch_step_dj<D, 2>(h, a, mode, block);
-    case 3: return launch_step_dj<D, 3>(h, a, mode, block);
-    case 4: return launch_step_dj<D, 4>(h, a, mode, block);
-    case 5: if constexpr (D >= 10) return launch_step_dj<D, 5>(h, a, mode, block); break;
-    case 6: if constexpr (D >= 12) return launch_step_dj<D, 6>(h, a, mode, block); break;
-    case 7: if constexpr (D >= 14) return launch_step_dj<D, 7>(h, a, mode, block); break;
-    case 8: if constexpr (D >= 16) return launch_step_dj<D, 8>(h, a, mode, block); break;
-    default: break;
-    }
-    return launch_step_dj<D, 0>(h, a, mode, block);
-}
-
-// The 24-dimensional state is compiled for 3 and 5 joints in the selection
-// basis (the scaled-state workloads); other joint counts report unsupported.
-int launch_step_d24(pf_handle *h, const StepArgs &a, int mode, int block)
-{
-    if (h->sel_mode && h->J == 3) return launch_step_dj<24, 3>(h, a, mode, block);
-    if (h->sel_mode && h->J == 5) return launch_step_dj<24, 5>(h, a, mode, block);
-    return set_error(PF_ERR_UNSUPPORTED, "d = 24 is compiled for 3 or 5 joints with a full-rank H");
-}
-
 int launch_step_block(pf_handle *h, const StepArgs &a, int mode, int block)
 {
-    switch (h->D) {
-    case 8: return launch_step_d<8>(h, a, mode, block);
-    case 12: return launch_step_d<12>(h, a, mode, block);
-    case 16: return launch_step_d<16>(h, a, mode, block);
-    case 24: return launch_step_d24(h, a, mode, block);
-    default: return set_error(PF_ERR_UNSUPPORTED, "state dimension %d not compiled", h->D);
-    }
+    const StepLaunch s{h->D, h->J, h->N, block, mode, h->sel_mode, h->stream};
+    return h->lay.row == 1 ? launch_step_rec(s, a) : launch_step_rows(s, a);
 }
 
 int launch_step(pf_handle *h, const StepArgs &a, int mode)
@@ -1201,13 +1146,12 @@ int ensure_events(pf_handle *h, size_t need)
 }
 
 // Up to this many input blocks a frame is one launch that resolves its own
-// ancestors; above, every block's prefix and the search's latency at two
-// waves per SIMD cost more than two more launches.  Per frame (d = 12, 8
-// detections per hand), one launch against step, k_prefix and
-// k_ancestors_prefixed: N = 200k 44.4 / 47.5 us, 262k 52.1 / 54.5, 400k 95.2 /
-// 91.9, 524k 132 / 121, 650k 155 / 139; N = 1M (step, weights and k_ancestors
-// launches before) 337 / 200.
-constexpr int kFusedBlocks = 1024;
+// ancestors; above, every block's prefix and the search's latency (and the
+// resolver's LDS, which leaves two blocks per CU) cost more than two more
+// launches.  Per frame (d = 12, 8 detections per hand), one launch against
+// step, k_prefix and k_ancestors_prefixed: N = 300k 52.4 / 58.1 us, 350k 62.2 /
+// 69.4, 400k 91.3 / 92.3, 450k 98.1 / 98.0, 524k 129 / 118, 650k 151 / 131.
+constexpr int kFusedBlocks = 1700;
 
 // Frames of many input blocks, or whose model image and resolver workspace do
 // not fit one workgroup's LDS: step and ancestor launches per frame, launched

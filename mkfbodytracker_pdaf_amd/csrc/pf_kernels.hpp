@@ -754,20 +754,22 @@ struct Joint {
             }
             return;
         }
-        float u0[D], u1[D];
+        // column k of M W is formed when column k of P is updated: two live
+        // temporaries instead of 2 D, which lets the row kernels fit three
+        // waves per SIMD (165 registers instead of 190 to 230) with no spills.
+        // These kernels are bound by memory latency: 150,000 particles 38.6 ->
+        // 32.9 us per frame, 262,144 52.1 -> 47.0, 10^6 200 -> 195.
 #pragma unroll
-        for (int c = 0; c < D; ++c) {
-            x[c] = fmaf(w0[c], v0, fmaf(w1[c], v1, x[c]));
-            u0[c] = fmaf(m00, w0[c], m01 * w1[c]);
-            u1[c] = fmaf(m01, w0[c], m11 * w1[c]);
-        }
+        for (int k = 0; k < D; ++k) {
+            x[k] = fmaf(w0[k], v0, fmaf(w1[k], v1, x[k]));
+            const float u0 = fmaf(m00, w0[k], m01 * w1[k]);
+            const float u1 = fmaf(m01, w0[k], m11 * w1[k]);
 #pragma unroll
-        for (int i = 0; i < D; ++i)
-#pragma unroll
-            for (int k = i; k < D; ++k) {
-                float p = fmaf(-w0[i], u0[k], P[pk(D, i, k)]);
-                P[pk(D, i, k)] = fmaf(-w1[i], u1[k], p);
+            for (int i = 0; i <= k; ++i) {
+                const float p = fmaf(-w0[i], u0, P[pk(D, i, k)]);
+                P[pk(D, i, k)] = fmaf(-w1[i], u1, p);
             }
+        }
     }
 };
 
@@ -1311,7 +1313,7 @@ __device__ __forceinline__ float joint_reject(float (&w0)[D], float (&w1)[D], fl
 // A joint whose innovation covariance FP32 cannot factor reliably
 // (innovation_ill) is factored in FP64 from the particle's current state
 // (joint_factor64, a per-lane branch taken only for those joints).
-template <int D, int MODE, int SELJ>
+template <int D, int MODE, int SELJ, bool PIECES = false>
 __device__ __forceinline__ float particle_update(const StepArgs &a, int t, int j, uint32_t U1, const float *sm,
                                                  float (&x)[D], float (&P)[npacked(D)],
                                                  const float *comp_global, int *comp_out, unsigned &flags)
@@ -1326,12 +1328,18 @@ __device__ __forceinline__ float particle_update(const StepArgs &a, int t, int j
     const float *stab = comp_global ? comp_global : sm + image_head_floats(a.K, a.m, D, a.J);
     const int k = draw_component(keys, a.K, (uint32_t)j, U1);
     if (comp_out) comp_out[j] = k;
+    // The mean-reverting predict.  PIECES: the component row's loads are kept
+    // in pieces of 26 values, for a kernel whose register count all 92 (d = 12)
+    // in flight beside the state would set (the batched step: 192 instead of 160).
     const float *ck = stab + k * CS;
     const float g = ck[0], g2 = ck[1];
 #pragma unroll
     for (int i = 0; i < D; ++i) x[i] = fmaf(g, x[i], ck[2 + i]);
 #pragma unroll
-    for (int p = 0; p < NP; ++p) P[p] = fmaf(g2, P[p], ck[2 + D + p]);
+    for (int p = 0; p < NP; ++p) {
+        P[p] = fmaf(g2, P[p], ck[2 + D + p]);
+        if (PIECES && p % 26 == 25) __builtin_amdgcn_sched_barrier(0);
+    }
 
     float acc = 0.f;
     if constexpr (SELJ > 0) {
@@ -1556,11 +1564,16 @@ __device__ __forceinline__ void step_body(const StepArgs &ain)
     }
 }
 
-// At least two waves per SIMD for states up to d = 16 in the selection
-// basis: the reference-mode kernels would otherwise take more than 256
-// registers (their FP64 joint branch) and run one.
+// Waves per SIMD the step kernels are compiled for: three for states up to
+// d = 12 in rows and the selection basis (168 registers), two for records (the
+// gather's registers) and up to d = 16, one otherwise.
+constexpr int step_waves(int D, int SELJ, bool rec)
+{
+    return D > 16 || SELJ == 0 ? 1 : (D <= 12 && !rec ? 3 : 2);
+}
+
 template <int D, int MODE, int SELJ, bool REC = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D > 16 || SELJ == 0) ? 1 : 2, 8))) k_step(StepArgs a)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(step_waves(D, SELJ, REC), 8))) k_step(StepArgs a)
 {
     step_body<D, MODE, SELJ, REC>(a);
 }
@@ -1569,7 +1582,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D > 1
 // tracker advances its two arms together (state in rows: the paired launch
 // has twice the blocks, where rows are the faster layout).
 template <int D, int MODE, int SELJ>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu((D > 16 || SELJ == 0) ? 1 : 2, 8))) k_step_pair(StepArgs a0, StepArgs a1)
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(step_waves(D, SELJ, false), 8))) k_step_pair(StepArgs a0, StepArgs a1)
 {
     step_body<D, MODE, SELJ, false>(blockIdx.y ? a1 : a0);
 }

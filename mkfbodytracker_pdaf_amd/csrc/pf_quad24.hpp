@@ -90,8 +90,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
     constexpr int D = 24, NP = npacked(24), CS = 2 + D + NP;
     extern __shared__ float4 sm4[];
     const int t = *a.frame;
-    const int tile = xcd_tile();
-    if (tile >= a.n_tiles[t]) return;                   // block-uniform: inactive sequences' tiles
+    const int ntiles = a.n_tiles[t];
+    if ((int)blockIdx.x >= ntiles) return;              // block-uniform: inactive sequences' tiles
+    const int tile = xcd_tile(ntiles);
     const bool odd = (t & 1) != 0;
     const float *xin = odd ? a.buf_x[1] : a.buf_x[0], *Pin = odd ? a.buf_P[1] : a.buf_P[0];
     float *xout = odd ? a.buf_x[0] : a.buf_x[1], *Pout = odd ? a.buf_P[0] : a.buf_P[1];

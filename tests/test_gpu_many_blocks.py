@@ -1,8 +1,9 @@
 """Resampling with more than 1024 input blocks of 256 weights, where the
-prefix of the block sums is taken once in its own kernel and the frames of a
+prefix of the block sums is taken once in its own kernel, and, with more than
+1700, the frames of a
 device-resident run are step, prefix and ancestor launches: indices bit-exact
 against the oracle, and a run equal to host-driven steps bit for bit, on both
-sides of the boundary (262,144 weights) and at the largest size."""
+sides of both boundaries and at the largest size."""
 import numpy as np
 import pytest
 
@@ -13,7 +14,8 @@ from mkfbodytracker_pdaf_amd.rbpf import Rbpf
 
 pytestmark = pytest.mark.gpu
 
-EDGE = 262144
+EDGE = 262144      # k_prefix above
+SPLIT = 435200     # separate launches above
 
 
 @pytest.mark.parametrize("L", [EDGE, EDGE + 1, 300007, 1 << 20])
@@ -42,7 +44,7 @@ def test_indices_bit_exact(L, kind):
     rb.close()
 
 
-@pytest.mark.parametrize("N", [EDGE, EDGE + 1, 270011])
+@pytest.mark.parametrize("N", [EDGE, EDGE + 1, SPLIT, SPLIT + 1])
 def test_run_equals_host_steps(N):
     T, cap = 3, 8
     mdl = synthetic.make_model(seed=5)
