@@ -808,28 +808,23 @@ int pf_batch_lml_grad(pf_batch *b, const int32_t *count, const float *cand, cons
                         const double v = gk[D + pk(D, std::min(r, c), std::max(r, c))];
                         Gp[r * D + c] = (r == c) ? v : 0.5 * v;
                     }
-                for (int r = 0; r < D; ++r)                 // G = T^T G' T
-                    for (int c = 0; c < D; ++c) {
-                        double acc = 0.0;
-                        for (int q = 0; q < D; ++q) acc += T[q * D + r] * Gp[q * D + c];
-                        TG[r * D + c] = acc;
-                    }
-                for (int r = 0; r < D; ++r)
-                    for (int c = 0; c < D; ++c) {
-                        double acc = 0.0;
-                        for (int q = 0; q < D; ++q) acc += TG[r * D + q] * T[q * D + c];
-                        G[r * D + c] = acc;
-                    }
+                // G = T^T G' T, a row at a time (each entry's sum in the order of q)
+                for (int r = 0; r < D; ++r) {
+                    for (int c = 0; c < D; ++c) TG[r * D + c] = G[r * D + c] = 0.0;
+                    for (int q = 0; q < D; ++q)
+                        for (int c = 0; c < D; ++c) TG[r * D + c] += T[q * D + r] * Gp[q * D + c];
+                    for (int q = 0; q < D; ++q)
+                        for (int c = 0; c < D; ++c) G[r * D + c] += TG[r * D + q] * T[q * D + c];
+                }
                 if (!chol_lower(D, hm.sig.data() + (size_t)k * D * D, L))
                     return set_error(PF_ERR_NOT_SPD, "sequence %d component %d: covariance not SPD", s, k);
                 double *out = grad_chol + ((size_t)s * K + k) * D * D;
-                for (int r = 0; r < D; ++r)                 // Lbar = 2 G L, lower triangle
-                    for (int c = 0; c < D; ++c) {
-                        double acc = 0.0;
-                        if (c <= r)
-                            for (int q = 0; q < D; ++q) acc += G[r * D + q] * L[q * D + c];
-                        out[r * D + c] = 2.0 * acc;
-                    }
+                for (int r = 0; r < D; ++r) {               // Lbar = 2 G L, lower triangle
+                    double acc[D] = {};
+                    for (int q = 0; q < D; ++q)
+                        for (int c = 0; c < D; ++c) acc[c] += G[r * D + q] * L[q * D + c];
+                    for (int c = 0; c < D; ++c) out[r * D + c] = c <= r ? 2.0 * acc[c] : 0.0;
+                }
             }
         }
     }

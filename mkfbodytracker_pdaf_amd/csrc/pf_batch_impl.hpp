@@ -191,7 +191,13 @@ struct pf_batch {
     bool recorded = false;
     double last_fwd_ms = 0.0, last_bwd_ms = 0.0;
     std::vector<size_t> adj_have = std::vector<size_t>(24, 0);   // element capacities of the buffers above
-    std::vector<double> h_T;      // state bases per sequence (internal order), D x D each
+    // model images on the host, by internal order: the images, reset tables and
+    // state bases with their inverses (D x D each); img_order[i] is the
+    // processing order image i was built for (-1: not since its model was loaded)
+    std::vector<float> h_tabs, h_mus, h_sgs;
+    std::vector<double> h_T, h_Ti;
+    std::vector<long long> img_order;
+    bool tables_stale = false;    // the device copies are older
 };
 
 
