@@ -1208,7 +1208,10 @@ static int run_frames(pf_handle *h, int T, int mode, const float *Z, const int *
     // own.  Otherwise the frame runs as separate launches, without graphs.
     const int nbp = (h->N + kWeightsBlock - 1) / kWeightsBlock;
     const int stage = h->table_floats + (mode == kModeCand ? cand_lds_floats(h->J, h->cap) : 0);
-    const bool fused = nbp <= kFusedBlocks && step_lds_bytes_rec(h->lay.row == 1, stage, nbp) <= kMaxLdsBytes;
+    // (records: as much LDS as leaves the blocks that share a CU their place)
+    const bool rec = h->lay.row == 1;
+    const int lds_limit = !rec ? kMaxLdsBytes : (nbp <= h->cus ? kCuLdsBytes : kCuLdsBytes / 2);
+    const bool fused = nbp <= kFusedBlocks && step_lds_bytes_rec(rec, stage, nbp) <= lds_limit;
     if (!fused) {
         st = run_frames_split(h, T, mode, Z, count, cand, uniforms, lml, timing, run_timing);
     } else {

@@ -125,6 +125,7 @@ constexpr int kWeightsBlock = 256;     // input block of the resampler scans
 constexpr int kStageBlocks = 12;       // input blocks the ancestor search stages in LDS
 constexpr int kMaxScanBlocks = 4096;   // => at most 2^20 resampled weights
 constexpr int kMaxLdsBytes = 64 * 1024;  // per-workgroup LDS budget
+constexpr int kCuLdsBytes = 160 * 1024;  // LDS of a CU
 
 enum StepMode { kModeRef = 0, kModeCand = 1 };
 enum AncMode { kAncArray = 0, kAncFused = 1 };
@@ -875,41 +876,47 @@ __host__ __device__ constexpr int rec_floats(int D) { return (D + npacked(D) + 3
 __host__ __device__ constexpr bool rec_layout(int D) { return D <= 12; }     // records compiled for this d
 __host__ __device__ inline size_t lidx(const Lay &L, int r, int j) { return (size_t)r * L.row + (size_t)j * L.part; }
 
-// LDS of the record gather and store of the step: per wave the records of
-// 16 particles (d <= 12: at most 16 x 23 chunks of 16 bytes), 4 waves.
-constexpr int kRecStageChunks = 16 * 23;
+// LDS of the record gather and store of the step: per wave the records of a
+// round's particles (d <= 12: at most 23 chunks of 16 bytes each), 4 waves.
+// Rounds of 32 particles: each chunk's LDS read and write serves half the
+// wave, and two blocks' slices (47 KB each) fit a CU; rounds of 16 need twice the
+// LDS instructions and waits, and all 64 at once leave one block per CU.
+// Per frame, rounds of 16 against 32: N = 1000 16.2 / 14.9 us, 20,000 17.0 / 16.2,
+// 100,000 22.5 / 21.0, 131,072 24.1 / 22.9; all 64 at once 14.8, 16.2, 33.5, 34.5.
+constexpr int kRecRound = 32;
+constexpr int kRecStageChunks = kRecRound * 23;
 constexpr int kRecStageBytes = 4 * kRecStageChunks * 16;
 
-// Wave-cooperative gather of the records of the wave's 64 particles, in four
-// rounds of 16: lane k of a round loads 16-byte chunk k % NCH of particle
+// Wave-cooperative gather of the records of the wave's 64 particles, in rounds
+// of kRecRound: lane k of a round loads 16-byte chunk k % NCH of particle
 // k / NCH's ancestor src (consecutive lanes read consecutive bytes of one
-// record, then of the next); the four rounds' loads are issued together,
-// then each round's chunks go to the wave's LDS slice gw in turn and the
-// round's 16 lanes take their particle's chunks into x and P.  Particles
-// j0w + p >= N read nothing (the buffer resource's bound returns zeros for
-// them).  Every lane of the wave calls it.
+// record, then of the next); all rounds' loads are issued together, then each
+// round's chunks go to the wave's LDS slice gw in turn and the round's lanes
+// take their particle's chunks into x and P.  Particles j0w + p >= N read
+// nothing (the buffer resource's bound returns zeros for them).  Every lane of
+// the wave calls it.
 template <int D>
 __device__ __forceinline__ void rec_gather(const float *rec, int N, int j0w, int src, float4 *gw, float (&x)[D],
                                            float (&P)[npacked(D)])
 {
-    constexpr int NP = npacked(D), RS = rec_floats(D), NCH = RS / 4;
-    static_assert(16 * NCH <= kRecStageChunks, "a round of 16 records exceeds the LDS slice");
+    constexpr int NP = npacked(D), RS = rec_floats(D), NCH = RS / 4, RD = kRecRound;
+    static_assert(RD * NCH <= kRecStageChunks, "a round of records exceeds the LDS slice");
     const int lane = threadIdx.x & 63;
     const unsigned lim = (unsigned)N * RS * 4u;
     const __amdgpu_buffer_rsrc_t ra =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<float *>(rec), (short)0, (int)lim, 0x00020000);
     // every round's loads first: the wave's 64 records share one memory
     // latency; the rounds then pass through the LDS slice in turn
-    constexpr int NI = (16 * NCH + 63) / 64;
-    u32x4 c[4][NI];
+    constexpr int NI = (RD * NCH + 63) / 64;
+    u32x4 c[64 / RD][NI];
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    for (int g = 0; g < 64 / RD; ++g) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int k = i * 64 + lane;
             const int p = k / NCH, ch = k - p * NCH;
-            const int sp = __shfl(src, 16 * g + (p < 16 ? p : 15), 64);
-            const bool ok = k < 16 * NCH && j0w + 16 * g + p < N;
+            const int sp = __shfl(src, RD * g + (p < RD ? p : RD - 1), 64);
+            const bool ok = k < RD * NCH && j0w + RD * g + p < N;
             c[g][i] = __builtin_amdgcn_raw_buffer_load_b128(ra, ok ? (int)((unsigned)(sp * RS + ch * 4) * 4u) : (int)lim,
                                                             0, 0);
         }
@@ -918,19 +925,19 @@ __device__ __forceinline__ void rec_gather(const float *rec, int N, int j0w, int
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
+    for (int g = 0; g < 64 / RD; ++g) {
 #pragma unroll
         for (int i = 0; i < NI; ++i) {
             const int k = i * 64 + lane;
-            if (k < 16 * NCH) reinterpret_cast<u32x4 *>(gw)[k] = c[g][i];
+            if (k < RD * NCH) reinterpret_cast<u32x4 *>(gw)[k] = c[g][i];
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        if ((lane >> 4) == g) {
+        if (lane / RD == g) {
 #pragma unroll
             for (int cc = 0; cc < NCH; ++cc) {
-                const float4 v = gw[(lane & 15) * NCH + cc];
+                const float4 v = gw[(lane & (RD - 1)) * NCH + cc];
                 const float ve[4] = {v.x, v.y, v.z, v.w};
 #pragma unroll
                 for (int e = 0; e < 4; ++e) {
@@ -947,22 +954,21 @@ __device__ __forceinline__ void rec_gather(const float *rec, int N, int j0w, int
 }
 
 // The inverse: the wave's 64 records (particles j0w .. j0w + 63, contiguous
-// in the buffer) written from x and P through gw in four rounds of 16; each
-// round stores 16 whole records as consecutive 16-byte chunks, so the stores
+// in the buffer) written from x and P through gw in rounds of kRecRound; each
+// round stores whole records as consecutive 16-byte chunks, so the stores
 // write whole lines and carry device scope like the row stores.  Every lane
 // of the wave calls it.
 template <int D>
 __device__ __forceinline__ void rec_store(float *rec, int N, int j0w, float4 *gw, const float (&x)[D],
                                           const float (&P)[npacked(D)])
 {
-    constexpr int NP = npacked(D), RS = rec_floats(D), NCH = RS / 4;
-    static_assert(16 * NCH <= kRecStageChunks, "a round of 16 records exceeds the LDS slice");
+    constexpr int NP = npacked(D), RS = rec_floats(D), NCH = RS / 4, RD = kRecRound;
     const int lane = threadIdx.x & 63;
     const unsigned lim = (unsigned)N * RS * 4u;
     const __amdgpu_buffer_rsrc_t wa = __builtin_amdgcn_make_buffer_rsrc(rec, (short)0, (int)lim, 0x00020000);
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-        if ((lane >> 4) == g) {
+    for (int g = 0; g < 64 / RD; ++g) {
+        if (lane / RD == g) {
 #pragma unroll
             for (int cc = 0; cc < NCH; ++cc) {
                 float ve[4];
@@ -971,19 +977,19 @@ __device__ __forceinline__ void rec_store(float *rec, int N, int j0w, float4 *gw
                     const int f = cc * 4 + e;
                     ve[e] = f < D ? x[f] : (f < D + NP ? P[f - D] : 0.f);
                 }
-                gw[(lane & 15) * NCH + cc] = make_float4(ve[0], ve[1], ve[2], ve[3]);
+                gw[(lane & (RD - 1)) * NCH + cc] = make_float4(ve[0], ve[1], ve[2], ve[3]);
             }
         }
         __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
         __builtin_amdgcn_wave_barrier();
         __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-        const unsigned base = (unsigned)(j0w + 16 * g) * RS * 4u;
-        const int nvalid = min(16, N - (j0w + 16 * g)) * NCH;
+        const unsigned base = (unsigned)(j0w + RD * g) * RS * 4u;
+        const int nvalid = min(RD, N - (j0w + RD * g)) * NCH;
 #pragma unroll
-        for (int i = 0; i < (16 * NCH + 63) / 64; ++i) {
+        for (int i = 0; i < (RD * NCH + 63) / 64; ++i) {
             const int k = i * 64 + lane;
-            const bool ok = k < 16 * NCH && k < nvalid;
-            const u32x4 v = reinterpret_cast<const u32x4 *>(gw)[k < 16 * NCH ? k : 0];
+            const bool ok = k < RD * NCH && k < nvalid;
+            const u32x4 v = reinterpret_cast<const u32x4 *>(gw)[k < RD * NCH ? k : 0];
             __builtin_amdgcn_raw_buffer_store_b128(v, wa, ok ? (int)(base + (unsigned)k * 16u) : (int)lim, 0,
                                                    kStoreDeviceScope);
         }
