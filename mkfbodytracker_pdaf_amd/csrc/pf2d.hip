@@ -450,7 +450,7 @@ int pf2d_update(pf2d_handle *h, const double *meas, uint32_t u, const double *no
     an.N = N;
     an.parity = 0;
     an.kind_linear = 0;
-    hipLaunchKernelGGL(k_ancestors, dim3((N + 255) / 256), dim3(256), 8 * (size_t)resolve_lds_words(nb), h->stream, an);
+    hipLaunchKernelGGL(k_ancestors, dim3(anc_blocks(N)), dim3(256), 8 * (size_t)resolve_lds_words(nb), h->stream, an);
     HIP_TRY2(hipGetLastError());
     hipLaunchKernelGGL(k_pf2d_lsum, dim3(1), dim3(64), 0, h->stream, h->lsum, h->lml, N);
     FrameScratch fs;

@@ -349,7 +349,7 @@ int launch_ancestors(pf_handle *h, int L, int N, int *out, int parity, int kind_
         return check_launch("k_ancestors_prefixed");
     }
     const size_t lds = 8 * (size_t)resolve_lds_words(an.pend.nb);
-    hipLaunchKernelGGL(k_ancestors, dim3((N + 255) / 256), dim3(256), lds, h->stream, an);
+    hipLaunchKernelGGL(k_ancestors, dim3(anc_blocks(N)), dim3(256), lds, h->stream, an);
     return check_launch("k_ancestors");
 }
 
@@ -541,7 +541,7 @@ struct AncEstimateL {
     {
         const int nb = (h->N + 255) / 256;
         const size_t lds = (size_t)anc_estimate_lds_bytes(an.pend.nb, D);
-        hipLaunchKernelGGL((k_ancestors_estimate<D>), dim3(nb), dim3(256), lds, h->stream, an, (const float *)h->xB,
+        hipLaunchKernelGGL((k_ancestors_estimate<D>), dim3(anc_blocks(h->N)), dim3(256), lds, h->stream, an, (const float *)h->xB,
                            h->lay, h->est_partial);
         hipLaunchKernelGGL((k_estimate_final<D>), dim3(1), dim3(256), 0, h->stream, (const double *)h->est_partial, nb,
                            h->N, (const double *)h->Tinv, h->est_out);
@@ -618,8 +618,7 @@ struct PairL {
                            (size_t)step_lds_bytes(a0.stage_floats, 0), s, a0, a1);
         const dim3 wg((h0->N + kWeightsBlock - 1) / kWeightsBlock, 2);
         if (!fused) hipLaunchKernelGGL((k_weights_pair<kLogF32>), wg, dim3(kWeightsBlock), 0, s, w0, w1);
-        const int nb = (h0->N + 255) / 256;
-        hipLaunchKernelGGL((k_ancestors_estimate_pair<D>), dim3(nb, 2), dim3(256),
+        hipLaunchKernelGGL((k_ancestors_estimate_pair<D>), dim3(anc_blocks(h0->N), 2), dim3(256),
                            (size_t)anc_estimate_lds_bytes(e0.an.pend.nb, D), s, e0, e1);
         if (final_sums) hipLaunchKernelGGL((k_estimate_final_pair<D>), dim3(2), dim3(256), 0, s, f0, f1);
     }

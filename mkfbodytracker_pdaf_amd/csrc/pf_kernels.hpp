@@ -565,15 +565,7 @@ struct ResolveStats {
     int pow;
 };
 
-// Both phases for one block of outputs.
-__device__ __forceinline__ int resolve_ancestor(const Pending &pd, int N, uint32_t U, int j0, unsigned long long *w,
-                                                bool want_es, double &es_out, ResolveStats &st)
-{
-    st.total = resolve_prefix(pd, w, want_es, es_out, st.pow);
-    return resolve_search(pd, N, U, st.total, j0, w);
-}
-
-// Frame statistics of a consumed resampling (block 0, thread 0): the log
+// Frame statistics of a consumed resampling (one thread): the log
 // mean weight, the degenerate flag (no positive weight), and the reset of the
 // maximum slot (linear weights).  bexp_sum is the block weight sums' total,
 // relative to 2^E for log-weights.
@@ -1705,19 +1697,50 @@ __device__ __forceinline__ Pending anc_pending(const AncArgs &a)
     return pd;
 }
 
+// Both phases for one block of outputs of a (a_j is returned), or, in the
+// launch's last block, which has no outputs, the statistics of the resampled
+// frame (returns -1).  The block sums, the exponent maxima and the frame
+// counter that picks one of them are loaded together.  The statistics' FP64
+// sum and logarithms in the first outputs' block made it end last: at N = 500
+// the ancestors with the estimates of two filters took 8.6 us against 7.6.
+__device__ __forceinline__ int resolve_ancestor(const AncArgs &a, unsigned long long *w)
+{
+    const Pending &pd = a.pend;
+    const int per = prefix_per(pd);
+    PrefixRegs r;
+    prefix_load(pd, per, 0, r);
+    const bool have = a.pow_frame && pd.bpow;
+    int E = 0;
+    if (have) {
+        const int p0 = gload(&a.fs->pow_max[0]), p1 = gload(&a.fs->pow_max[1]), p2 = gload(&a.fs->pow_max[2]);
+        const int m = gload(a.pow_frame) % 3;
+        E = m == 0 ? p0 : (m == 1 ? p1 : p2);
+    }
+    const bool stats = blockIdx.x == gridDim.x - 1;
+    double es = 0.0;
+    ResolveStats st;
+    st.total = resolve_prefix_from(pd, w, per, r, have, E, stats && a.lml, es, st.pow);
+    if (stats) {
+        if (threadIdx.x == 0)
+            finish_resampling(a.fs, a.parity, es, st, a.N, a.kind_linear,
+                              (a.lml && a.lml_frame) ? a.lml + *a.lml_frame : a.lml);
+        return -1;
+    }
+    const int j0 = blockIdx.x * blockDim.x;
+    const int src = resolve_search(pd, a.N, a.fs->U_pending, st.total, j0, w);
+    if (j0 + (int)threadIdx.x < a.N) a.anc[j0 + threadIdx.x] = src;
+    return src;
+}
+
 static __global__ void __launch_bounds__(256) k_ancestors(AncArgs a)
 {
     extern __shared__ unsigned long long wsp[];
-    const int j0 = blockIdx.x * blockDim.x;
-    const int j = j0 + threadIdx.x;
-    double es = 0.0;
-    ResolveStats rs;
-    const int src = resolve_ancestor(anc_pending(a), a.N, a.fs->U_pending, j0, wsp, blockIdx.x == 0 && a.lml, es, rs);
-    if (j < a.N) a.anc[j] = src;
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        finish_resampling(a.fs, a.parity, es, rs, a.N, a.kind_linear,
-                          (a.lml && a.lml_frame) ? a.lml + *a.lml_frame : a.lml);
+    resolve_ancestor(a, wsp);
 }
+
+// Blocks of k_ancestors and the kernels that share its form: one per 256
+// outputs and one for the statistics.
+inline int anc_blocks(int N) { return (N + 255) / 256 + 1; }
 
 // The ancestors of many input blocks.  k_ancestors has every block of 256
 // outputs repeat the prefix of all block sums, and its LDS (12 bytes per
@@ -2144,15 +2167,9 @@ template <int D>
 __device__ __forceinline__ void ancestors_estimate_body(const AncArgs &a, const float *x, Lay L, double *partial)
 {
     extern __shared__ unsigned long long wsp[];
-    const int j0 = blockIdx.x * blockDim.x;
-    const int j = j0 + threadIdx.x;
-    double es = 0.0;
-    ResolveStats rs;
-    const int src = resolve_ancestor(anc_pending(a), a.N, a.fs->U_pending, j0, wsp, blockIdx.x == 0 && a.lml, es, rs);
-    if (j < a.N) a.anc[j] = src;
-    if (blockIdx.x == 0 && threadIdx.x == 0)
-        finish_resampling(a.fs, a.parity, es, rs, a.N, a.kind_linear,
-                          (a.lml && a.lml_frame) ? a.lml + *a.lml_frame : a.lml);
+    const int src = resolve_ancestor(a, wsp);
+    if (src < 0) return;                 // the statistics' block
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
     double v[D];
     load_x64<D>(x, L, src, j < a.N, v);
     __syncthreads();                     // every lane is done with the resolver's LDS

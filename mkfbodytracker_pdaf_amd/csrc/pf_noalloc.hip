@@ -143,7 +143,7 @@ extern "C" int pf_resample_log_noalloc(const double *lw, int32_t L, int32_t N, u
     an.parity = 0;
     an.kind_linear = 0;
     const size_t lds = 8 * (size_t)resolve_lds_words(nb);
-    hipLaunchKernelGGL(k_ancestors, dim3((N + 255) / 256), dim3(256), lds, s, an);
+    hipLaunchKernelGGL(k_ancestors, dim3(anc_blocks(N)), dim3(256), lds, s, an);
     if (status) hipLaunchKernelGGL(k_noalloc_status, dim3(1), dim3(64), 0, s, (const FrameScratch *)fs, status);
     const hipError_t e = hipGetLastError();
     if (e != hipSuccess) return set_error(PF_ERR_HIP, "resample launch failed: %s", hipGetErrorString(e));
