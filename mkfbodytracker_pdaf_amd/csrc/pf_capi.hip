@@ -121,6 +121,7 @@ struct pf_handle {
     int *run_ctr = nullptr;
     static constexpr int kGroups = 7;  // 1, 2, 4, ..., 64 frames
     hipGraphExec_t groups[2][2][kGroups] = {};
+    unsigned long long generation = 1;   // raised whenever device addresses or tables of the handle change
 };
 
 namespace {
@@ -138,9 +139,11 @@ hipError_t dalloc(T **p, size_t n)
     return hipMalloc((void **)p, sizeof(T) * std::max<size_t>(n, 1));
 }
 
-// Destroys the captured frame groups (they bake in device addresses).
+// Destroys the captured frame groups (they bake in device addresses), and
+// marks those that others captured with this handle's as out of date.
 void drop_graphs(pf_handle *h)
 {
+    ++h->generation;
     for (auto &per_mode : h->groups)
         for (auto &per_parity : per_mode)
             for (hipGraphExec_t &g : per_parity)
@@ -514,15 +517,13 @@ int reserve_resample(pf_handle *h, int L) { return ensure_resample_scratch(h, L)
 const double *estimate_ptr(pf_handle *h) { return h->est_out; }
 
 
-int set_frame(pf_handle *h, int f)
-{
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, h->stream, h->frame, f);
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, h->stream, h->frame + 1, f);
-    // the exponent slot of frame f (a step that writes its own weights
-    // raises it; later slots are cleared by the step before them)
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, h->stream, &h->fs->pow_max[f % 3], kPowEmpty);
-    return check_launch("k_set_int");
-}
+int *frame_counters(pf_handle *h) { return h->frame; }
+
+unsigned long long generation(const pf_handle *h) { return h->generation; }
+
+int state_buffer(const pf_handle *h) { return h->xA == h->xbuf[1] ? 1 : 0; }
+
+void swap_state_buffer(pf_handle *h) { swap_state(h); }
 
 int estimate(pf_handle *h)
 {
@@ -788,6 +789,7 @@ int pf_load_model(pf_handle *h, int32_t K, int32_t d, int32_t npose, int32_t m, 
     h->D = d; h->K = K; h->m = m; h->J = J; h->npose = npose;
 
     // (re)allocate device buffers sized by the model
+    drop_graphs(h);
     (void)hipFree(h->rec[0]); (void)hipFree(h->rec[1]);
     h->rec[0] = h->rec[1] = nullptr;
     h->xA = h->PA = h->xB = h->PB = nullptr;

@@ -26,8 +26,16 @@ int info(pf_handle *h, Info *out);
 int reserve_resample(pf_handle *h, int L);
 // Device address of the estimate written by estimate(): D doubles, model basis.
 const double *estimate_ptr(pf_handle *h);
-// Sets both frame counters of the handle to f.
-int set_frame(pf_handle *h, int f);
+// The handle's two frame counters (frame t reads counter t & 1, t + 1 goes to
+// the other); a caller sets both to 0, and scratch()->pow_max[0] to kPowEmpty,
+// before frame 0.
+int *frame_counters(pf_handle *h);
+// Raised whenever device addresses or tables that a captured frame bakes in
+// change; and which of its two state buffers (0 or 1) the next step reads.
+unsigned long long generation(const pf_handle *h);
+int state_buffer(const pf_handle *h);
+// Counts a replayed step: the state buffers change roles.
+void swap_state_buffer(pf_handle *h);
 // getEstimator (pf2DRao.cpp:23-31) of the current tracks into estimate_ptr().
 int estimate(pf_handle *h);
 // ParticleFilter::update (pf2DRao.cpp:125-158) with one measurement column per

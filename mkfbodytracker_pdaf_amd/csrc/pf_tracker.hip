@@ -49,7 +49,8 @@ constexpr int kMaxRadius = 15;
 constexpr int kBlurW = 32, kBlurH = 16, kBlurThreads = 128;
 constexpr int kProposeBlock = 256;
 constexpr int kMaxArmD = 24;              // k_propose stages 3 D + 2 projection operands per arm
-constexpr int kTrGraphFrames = 16;        // frames per captured graph of a device-resident run (even)
+constexpr int kTrGroups = 5;              // captured groups of 1, 2, 4, 8, 16 frames
+constexpr int kBlurSlots = 1 << (kTrGroups - 1);   // blurred images held: one per frame of the largest group
 constexpr int kPropShift = 10;            // the proposal resampler's input blocks: 1024 proposals
 constexpr int kMaxProposals = 1 << 20;    // resampler scan limit
 
@@ -61,6 +62,18 @@ struct FrameRec {
     long long g;     // global frame index
     int uniform;     // first-frame (uniform) proposals
     int pad;
+};
+
+// Inputs and outputs of a device-resident run, in device memory (k_tr_begin),
+// so that the captured frames do not depend on the run's buffers and serve
+// every later run.
+struct TrackerRun {
+    const uint8_t *lik;       // T x rows x cols
+    const int *roi;           // T x 4
+    double *lml, *pose, *pos3d, *tf, *pose2d;   // the run's outputs (nullable)
+    long long g0;             // global index of frame t = 0
+    long long uniform_frame;  // global index of the uniform-proposal frame (-1: none)
+    int T;
 };
 
 struct ArmDev {
@@ -76,11 +89,11 @@ struct ArmDev {
 
 // ------------------------------------------------------------------ blur
 struct BlurArgs {
-    const uint8_t *src;
-    uint8_t *dst;
+    const uint8_t *src;       // one image (run == nullptr)
+    uint8_t *dst;             // its blur, or the kBlurSlots slots of a run's frames
     const float *taps;        // 2 radius + 1
-    const int *frame;         // source frame = *frame (nullptr: 0)
-    long long frame_stride;
+    const TrackerRun *run;    // the images of frames *frame + blockIdx.z
+    const int *frame;
     int rows, cols;
 };
 
@@ -94,7 +107,10 @@ __device__ __forceinline__ int reflect101(int i, int n)
 // GaussianBlur(ksize, sigma, BORDER_REFLECT_101) (pfPose.cpp:213): row pass
 // then column pass, each an FP32 fma chain over the taps in index order,
 // round to nearest even and saturate to uint8.  One 32 x 16 output tile per
-// block (1200 blocks for 640 x 480), source tile and row-pass results in LDS.
+// block (600 blocks for 640 x 480), source tile and row-pass results in LDS.
+// A group of frames' images are blurred in one launch ahead of the frames
+// (grid.z): one image leaves the launch's latency exposed, 6.7 us a frame
+// against 2.5 in groups of 16.
 template <int R>
 __global__ void __launch_bounds__(kBlurThreads) k_blur(BlurArgs a)
 {
@@ -103,8 +119,15 @@ __global__ void __launch_bounds__(kBlurThreads) k_blur(BlurArgs a)
     __shared__ float s_row[IH * kBlurW];
     __shared__ float s_tap[NT];
     const int x0 = blockIdx.x * kBlurW, y0 = blockIdx.y * kBlurH;
-    const long long f = a.frame ? (long long)*a.frame : 0;
-    const uint8_t *src = a.src + f * a.frame_stride;
+    const size_t px = (size_t)a.rows * a.cols;
+    const uint8_t *src = a.src;
+    uint8_t *dst = a.dst;
+    if (a.run) {
+        const int f = *a.frame + (int)blockIdx.z;
+        if (f >= a.run->T) return;
+        src = a.run->lik + (size_t)f * px;
+        dst += (size_t)(f % kBlurSlots) * px;
+    }
     if ((int)threadIdx.x < NT) s_tap[threadIdx.x] = a.taps[threadIdx.x];
     // all of a thread's source loads are issued before its first LDS store,
     // so the tile costs one memory latency rather than one per element
@@ -150,7 +173,7 @@ __global__ void __launch_bounds__(kBlurThreads) k_blur(BlurArgs a)
             float acc = 0.f;
 #pragma unroll
             for (int k = 0; k < NT; ++k) acc = fmaf(s_tap[k], p[k * kBlurW], acc);
-            a.dst[(size_t)gy * a.cols + gx] = (uint8_t)fminf(fmaxf(rintf(acc), 0.f), 255.f);
+            dst[(size_t)gy * a.cols + gx] = (uint8_t)fminf(fmaxf(rintf(acc), 0.f), 255.f);
         }
     }
 }
@@ -158,9 +181,7 @@ __global__ void __launch_bounds__(kBlurThreads) k_blur(BlurArgs a)
 // --------------------------------------------------------------- proposals
 struct PropParams {
     uint64_t seed;
-    long long g0;             // global index of frame t = 0 of this run
-    long long uniform_frame;  // global index of the uniform-proposal frame (-1: none)
-    const int *roi;           // frames x 4
+    const TrackerRun *run;
     const int *frame;         // t
     const uint32_t *u_prop;   // frames x 2: the proposal resampling uniform of each arm
     int n_c, rows, cols;
@@ -267,9 +288,10 @@ __global__ void __launch_bounds__(kProposeBlock) k_propose(PropParams p, ArmDev 
     __shared__ double s_y[4];
     __shared__ unsigned long long s_wave[2][kProposeBlock / 64];
     const int t = *p.frame;
-    const long long g = p.g0 + t;
-    const bool uniform = (g == p.uniform_frame);
-    const int *roi = p.roi + 4 * (size_t)t;
+    const long long g = p.run->g0 + t;
+    const bool uniform = (g == p.run->uniform_frame);
+    const int *roi = p.run->roi + 4 * (size_t)t;
+    img += (size_t)(t % kBlurSlots) * p.rows * p.cols;
     const int arm = blockIdx.y;
     const ArmDev &A = arm ? a1 : a0;
     hand_projections(a0, a1, s_stage, s_y);
@@ -415,10 +437,11 @@ __global__ void __launch_bounds__(256) k_dump_proposals(PropParams p, const Fram
 struct PoseArgs {
     ArmDev arm[2];
     int *frame;               // t (incremented at the end)
-    double *pose;             // frames x 2 x npose (nullable)
-    double *pos3d;            // frames x 2 x 15 (nullable)
-    double *tf;               // frames x 24 (nullable)
-    double *pose2d;           // frames x 16 (nullable)
+    const TrackerRun *run;    // the outputs of a run's frames, else:
+    double *pose;             // 2 x npose (nullable)
+    double *pos3d;            // 2 x 15 (nullable)
+    double *tf;               // 24 (nullable)
+    double *pose2d;           // 16 (nullable)
     int npose;
     double fx, fy, cx, cy;
 };
@@ -492,8 +515,15 @@ __device__ double pose2d_entry(const double (*e)[64], int i)
 // then the TF-tree and 2-D point lists.
 // x0, x1: the arms' estimates (model basis).  Every thread of the block
 // calls it.
-__device__ inline void pose_body(const PoseArgs &a, const double *x0, const double *x1)
+__device__ inline void pose_body(const PoseArgs &ain, const double *x0, const double *x1)
 {
+    PoseArgs a = ain;
+    if (a.run) {
+        a.pose = a.run->pose;
+        a.pos3d = a.run->pos3d;
+        a.tf = a.run->tf;
+        a.pose2d = a.run->pose2d;
+    }
     __shared__ double s_e[2][64];
     __shared__ double s_tg[2][6];
     __shared__ double s_p[2][15];
@@ -588,6 +618,50 @@ __global__ void k_tr_set(int *p, int v)
     if (threadIdx.x == 0 && blockIdx.x == 0) *p = v;
 }
 
+// Start of a run: its descriptor, the frame counters at 0 with frame 0's
+// exponent slot cleared, and the frame uniforms of its T frames from the
+// Philox stream (words 8 g .. of stream kStreamFrame: arm 1's component draw
+// and resampling, arm 2's, both proposal resamplings).
+struct BeginArgs {
+    TrackerRun v;
+    TrackerRun *run;
+    int *fctr;
+    int *arm_frame[2];
+    FrameScratch *fs[2];
+    uint32_t *uni[3];         // arm 1, arm 2, proposals: T x 2
+    uint64_t seed;
+};
+
+__global__ void __launch_bounds__(64) k_tr_begin(BeginArgs a)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x;
+    if (t == 0) {
+        *a.run = a.v;
+        *a.fctr = 0;
+        for (int k = 0; k < 2; ++k) {
+            a.arm_frame[k][0] = 0;
+            a.arm_frame[k][1] = 0;
+            a.fs[k]->pow_max[0] = kPowEmpty;
+        }
+    }
+    if (t >= a.v.T) return;
+    const uint64_t b = 2 * (uint64_t)(a.v.g0 + t);
+    uint32_t f[8];
+    philox_stream_block(a.seed, kStreamFrame, b, f);
+    philox_stream_block(a.seed, kStreamFrame, b + 1, f + 4);
+#pragma unroll
+    for (int k = 0; k < 6; ++k) a.uni[k >> 1][2 * (size_t)t + (k & 1)] = f[k];
+}
+
+// End of a run: the arms' log mean weights (lml0, lml1: T each) to its output.
+__global__ void k_tr_end(const TrackerRun *run, const double *lml0, const double *lml1)
+{
+    const int t = blockIdx.x * blockDim.x + threadIdx.x, T = run->T;
+    if (!run->lml || t >= T) return;
+    run->lml[t] = lml0[t];
+    run->lml[T + t] = lml1[t];
+}
+
 template <typename T>
 hipError_t talloc(T **p, size_t n)
 {
@@ -612,8 +686,15 @@ struct pf_tracker {
     FrameRec *rec = nullptr;
     int *fctr = nullptr, *fctr_aux = nullptr;
     uint32_t *uni = nullptr;          // [arm 0: cap x 2][arm 1: cap x 2][proposals: cap x 2]
-    int uni_cap = 0;
-    std::vector<uint32_t> h_uni;
+    double *lml = nullptr;            // [arm 0: cap][arm 1: cap]
+    int run_cap = 0;                  // frames of a run they hold
+    TrackerRun *run = nullptr;
+    int last_slot = 0;                // blurred image of the last frame
+    // captured frames: group g holds 2^g, by which buffer each arm's state is
+    // in; dropped when a buffer of the tracker or an arm that they bake in is
+    // allocated again (eng::generation)
+    hipGraphExec_t groups[4][kTrGroups] = {};
+    unsigned long long gen[2] = {0, 0};
     pf_tracker_outputs stage_out{};     // device outputs of one host-driven frame
     hipEvent_t ev_fork[2] = {nullptr, nullptr}, ev_join[2] = {nullptr, nullptr}, ev_pre = nullptr;
     hipEvent_t ev_t0 = nullptr, ev_t1 = nullptr;
@@ -655,15 +736,13 @@ ArmDev arm_dev(pf_tracker *tr, int a)
     return d;
 }
 
-PropParams prop_params(pf_tracker *tr, const int *roi, const int *frame)
+PropParams prop_params(pf_tracker *tr)
 {
     PropParams p{};
     p.seed = tr->cfg.seed;
-    p.g0 = tr->frames_done;
-    p.uniform_frame = tr->uniform_frame;
-    p.roi = roi;
-    p.frame = frame;
-    p.u_prop = tr->uni + 4 * (size_t)tr->uni_cap;
+    p.run = tr->run;
+    p.frame = tr->fctr;
+    p.u_prop = tr->uni + 4 * (size_t)tr->run_cap;
     p.n_c = tr->n_c;
     p.rows = tr->cfg.rows;
     p.cols = tr->cfg.cols;
@@ -680,17 +759,19 @@ int launch_check(const char *what)
     return PF_OK;
 }
 
-int launch_blur(pf_tracker *tr, const uint8_t *src, const int *frame, uint8_t *dst)
+// The blur of one image src to dst, or (src null) of the run's next n frames
+// to their slots.
+int launch_blur(pf_tracker *tr, const uint8_t *src, uint8_t *dst, int n)
 {
     BlurArgs b{};
     b.src = src;
     b.dst = dst;
     b.taps = tr->taps;
-    b.frame = frame;
-    b.frame_stride = (long long)tr->cfg.rows * tr->cfg.cols;
+    b.run = src ? nullptr : tr->run;
+    b.frame = tr->fctr;
     b.rows = tr->cfg.rows;
     b.cols = tr->cfg.cols;
-    const dim3 grid((tr->cfg.cols + kBlurW - 1) / kBlurW, (tr->cfg.rows + kBlurH - 1) / kBlurH);
+    const dim3 grid((tr->cfg.cols + kBlurW - 1) / kBlurW, (tr->cfg.rows + kBlurH - 1) / kBlurH, n);
     using K = void (*)(BlurArgs);
     static const K kernels[kMaxRadius + 1] = {k_blur<0>, k_blur<1>, k_blur<2>, k_blur<3>, k_blur<4>, k_blur<5>,
                                               k_blur<6>, k_blur<7>, k_blur<8>, k_blur<9>, k_blur<10>, k_blur<11>,
@@ -699,16 +780,21 @@ int launch_blur(pf_tracker *tr, const uint8_t *src, const int *frame, uint8_t *d
     return launch_check("k_blur");
 }
 
-PoseArgs pose_args(pf_tracker *tr, int *frame, const pf_tracker_outputs &out)
+// The pose output of the run's frame (out null) or to out.
+PoseArgs pose_args(pf_tracker *tr, int *frame, const pf_tracker_outputs *out)
 {
     PoseArgs pa{};
     pa.arm[0] = arm_dev(tr, 0);
     pa.arm[1] = arm_dev(tr, 1);
     pa.frame = frame;
-    pa.pose = out.pose;
-    pa.pos3d = out.pos3d;
-    pa.tf = out.tf;
-    pa.pose2d = out.pose2d;
+    if (out) {
+        pa.pose = out->pose;
+        pa.pos3d = out->pos3d;
+        pa.tf = out->tf;
+        pa.pose2d = out->pose2d;
+    } else {
+        pa.run = tr->run;
+    }
     pa.npose = tr->npose;
     pa.fx = tr->cfg.fx;
     pa.fy = tr->cfg.fy;
@@ -717,7 +803,7 @@ PoseArgs pose_args(pf_tracker *tr, int *frame, const pf_tracker_outputs &out)
     return pa;
 }
 
-int launch_pose(pf_tracker *tr, int *frame, const pf_tracker_outputs &out)
+int launch_pose(pf_tracker *tr, int *frame, const pf_tracker_outputs *out)
 {
     hipLaunchKernelGGL(k_pose, dim3(1), dim3(64), 0, tr->s[0], pose_args(tr, frame, out));
     return launch_check("k_pose");
@@ -727,9 +813,9 @@ int launch_pose(pf_tracker *tr, int *frame, const pf_tracker_outputs &out)
 // of a state dimension whose reduction fits its LDS).
 bool pose_adds_estimates(pf_tracker *tr) { return tr->D[0] == tr->D[1] && (tr->D[0] == 8 || tr->D[0] == 12); }
 
-int launch_pose_est(pf_tracker *tr, int *frame, const pf_tracker_outputs &out)
+int launch_pose_est(pf_tracker *tr)
 {
-    const PoseArgs pa = pose_args(tr, frame, out);
+    const PoseArgs pa = pose_args(tr, tr->fctr, nullptr);
     const EstFinalArgs e0 = eng::estimate_final_args(tr->arm[0]), e1 = eng::estimate_final_args(tr->arm[1]);
     if (tr->D[0] == 8)
         hipLaunchKernelGGL((k_pose_est<8>), dim3(1), dim3(512), 0, tr->s[0], pa, e0, e1);
@@ -738,19 +824,17 @@ int launch_pose_est(pf_tracker *tr, int *frame, const pf_tracker_outputs &out)
     return launch_check("k_pose_est");
 }
 
-// One frame of the pipeline; `parity` alternates from frame to frame (it
-// selects the handles' frame counter and maximum slot).
-int enqueue_frame(pf_tracker *tr, int parity, int T, const uint8_t *lik, const int *roi, const pf_tracker_outputs &out)
+// One frame of the run, whose image is blurred already; `parity` alternates
+// from frame to frame (it selects the handles' frame counter and maximum slot).
+int enqueue_frame(pf_tracker *tr, int parity)
 {
-    int st = launch_blur(tr, lik, tr->fctr, tr->blur);
-    if (st) return st;
-    const PropParams p = prop_params(tr, roi, tr->fctr);
+    const PropParams p = prop_params(tr);
     const ArmDev a0 = arm_dev(tr, 0), a1 = arm_dev(tr, 1);
     const int pairs = tr->n_c / 2;
     const int pblocks = std::min((pairs + kProposeBlock - 1) / kProposeBlock, tr->prop_blocks);
     hipLaunchKernelGGL(k_propose, dim3(pblocks, 2), dim3(kProposeBlock), 0,
                        tr->s[0], p, a0, a1, (const uint8_t *)tr->blur, tr->rec);
-    st = launch_check("k_propose");
+    int st = launch_check("k_propose");
     if (st) return st;
     SelectArgs sa[2];
     for (int a = 0; a < 2; ++a) {
@@ -760,8 +844,8 @@ int enqueue_frame(pf_tracker *tr, int parity, int T, const uint8_t *lik, const i
         sa[a].Z = tr->Z[a];
     }
     const size_t sel_lds = 8 * (size_t)resolve_lds_words(sa[0].pend.nb);
-    const uint32_t *u_arm[2] = {tr->uni, tr->uni + 2 * (size_t)tr->uni_cap};
-    double *lml[2] = {out.lml, out.lml ? out.lml + T : nullptr};
+    const uint32_t *u_arm[2] = {tr->uni, tr->uni + 2 * (size_t)tr->run_cap};
+    double *lml[2] = {tr->lml, tr->lml + tr->run_cap};
     if (eng::pair_compatible(tr->arm[0], tr->arm[1])) {
         // both arms advance together on stream 0, one launch per stage
         hipLaunchKernelGGL(k_prop_select_pair, dim3((tr->N + 255) / 256, 2), dim3(256), sel_lds, tr->s[0], p, sa[0],
@@ -771,7 +855,7 @@ int enqueue_frame(pf_tracker *tr, int parity, int T, const uint8_t *lik, const i
         if (!st) st = eng::step_ref_pair(tr->arm[0], tr->arm[1], tr->Z[0], tr->Z[1], u_arm[0], u_arm[1], parity,
                                          lml[0], lml[1], !fold);
         if (st) return st;
-        return fold ? launch_pose_est(tr, tr->fctr, out) : launch_pose(tr, tr->fctr, out);
+        return fold ? launch_pose_est(tr) : launch_pose(tr, tr->fctr, nullptr);
     }
     // otherwise each arm on its own stream, forked here and joined before the pose
     TR_TRY(hipEventRecord(tr->ev_fork[parity], tr->s[0]));
@@ -787,35 +871,76 @@ int enqueue_frame(pf_tracker *tr, int parity, int T, const uint8_t *lik, const i
     }
     TR_TRY(hipEventRecord(tr->ev_join[parity], tr->s[1]));
     TR_TRY(hipStreamWaitEvent(tr->s[0], tr->ev_join[parity], 0));
-    return launch_pose(tr, tr->fctr, out);
+    return launch_pose(tr, tr->fctr, nullptr);
 }
 
-// Frame uniforms of global frames [g0, g0 + T) into the device table.
-int upload_uniforms(pf_tracker *tr, int T)
+// n frames of the run, the first of even index: their blurs, then the frames.
+int enqueue_group(pf_tracker *tr, int n)
 {
-    if (T > tr->uni_cap) {
-        (void)hipFree(tr->uni);
-        tr->uni = nullptr;
-        const int cap = std::max(T, 64);
-        TR_TRY(talloc(&tr->uni, (size_t)6 * cap));
-        tr->uni_cap = cap;
+    int st = launch_blur(tr, nullptr, tr->blur, n);
+    for (int f = 0; f < n && !st; ++f) st = enqueue_frame(tr, f & 1);
+    return st;
+}
+
+void drop_groups(pf_tracker *tr)
+{
+    for (auto &by_state : tr->groups)
+        for (hipGraphExec_t &g : by_state)
+            if (g) {
+                (void)hipStreamSynchronize(tr->s[0]);    // its last replay is done
+                (void)hipGraphExecDestroy(g);
+                g = nullptr;
+            }
+}
+
+// The buffers sized by a run's frames.
+int ensure_run(pf_tracker *tr, int T)
+{
+    if (T <= tr->run_cap) return PF_OK;
+    drop_groups(tr);
+    (void)hipFree(tr->uni);
+    (void)hipFree(tr->lml);
+    tr->uni = nullptr;
+    tr->lml = nullptr;
+    tr->run_cap = 0;
+    const int cap = std::max(T, 64);
+    TR_TRY(talloc(&tr->uni, (size_t)6 * cap));
+    TR_TRY(talloc(&tr->lml, (size_t)2 * cap));
+    tr->run_cap = cap;
+    return PF_OK;
+}
+
+// The captured group of 2^g frames for the arms' present state buffers
+// (captured on first use; capturing leaves the arms as they were).
+int frame_group(pf_tracker *tr, int g, hipGraphExec_t *out)
+{
+    for (int a = 0; a < 2; ++a)
+        if (tr->gen[a] != eng::generation(tr->arm[a])) {
+            drop_groups(tr);
+            tr->gen[0] = eng::generation(tr->arm[0]);
+            tr->gen[1] = eng::generation(tr->arm[1]);
+        }
+    hipGraphExec_t &ge = tr->groups[2 * eng::state_buffer(tr->arm[0]) + eng::state_buffer(tr->arm[1])][g];
+    if (!ge) {
+        hipGraph_t graph;
+        TR_TRY(hipStreamBeginCapture(tr->s[0], hipStreamCaptureModeThreadLocal));
+        const int sc = enqueue_group(tr, 1 << g);
+        const hipError_t ec = hipStreamEndCapture(tr->s[0], &graph);
+        if (g == 0)
+            for (pf_handle *arm : tr->arm) eng::swap_state_buffer(arm);
+        if (sc) {
+            if (ec == hipSuccess) (void)hipGraphDestroy(graph);
+            return sc;
+        }
+        if (ec != hipSuccess) return set_error(PF_ERR_HIP, "graph capture failed: %s", hipGetErrorString(ec));
+        const hipError_t ei = hipGraphInstantiate(&ge, graph, nullptr, nullptr, 0);
+        (void)hipGraphDestroy(graph);
+        if (ei != hipSuccess) {
+            ge = nullptr;
+            return set_error(PF_ERR_HIP, "graph instantiation failed: %s", hipGetErrorString(ei));
+        }
     }
-    const size_t cap = (size_t)tr->uni_cap;
-    tr->h_uni.assign(6 * cap, 0u);
-    std::vector<uint32_t> w(8 * (size_t)T);
-    philox_u32(tr->cfg.seed, kStreamFrame, 8 * (uint64_t)tr->frames_done, 8 * (int64_t)T, w.data());
-    for (int t = 0; t < T; ++t) {
-        const uint32_t *f = w.data() + 8 * (size_t)t;
-        tr->h_uni[2 * (size_t)t] = f[0];
-        tr->h_uni[2 * (size_t)t + 1] = f[1];
-        tr->h_uni[2 * cap + 2 * (size_t)t] = f[2];
-        tr->h_uni[2 * cap + 2 * (size_t)t + 1] = f[3];
-        tr->h_uni[4 * cap + 2 * (size_t)t] = f[4];
-        tr->h_uni[4 * cap + 2 * (size_t)t + 1] = f[5];
-    }
-    TR_TRY(hipMemcpyAsync(tr->uni, tr->h_uni.data(), sizeof(uint32_t) * tr->h_uni.size(), hipMemcpyHostToDevice,
-                          tr->s[0]));
-    TR_TRY(hipStreamSynchronize(tr->s[0]));
+    *out = ge;
     return PF_OK;
 }
 
@@ -886,6 +1011,7 @@ int pf_tracker_destroy(pf_tracker *tr)
 {
     if (!tr) return PF_OK;
     (void)hipSetDevice(tr->device);
+    drop_groups(tr);
     for (int a = 0; a < 2; ++a) {
         (void)hipFree(tr->hp[a]);
         (void)hipFree(tr->pm[a]);
@@ -903,6 +1029,8 @@ int pf_tracker_destroy(pf_tracker *tr)
     (void)hipFree(tr->fctr);
     (void)hipFree(tr->fctr_aux);
     (void)hipFree(tr->uni);
+    (void)hipFree(tr->lml);
+    (void)hipFree(tr->run);
     (void)hipFree(tr->stage_out.lml);
     (void)hipFree(tr->stage_out.pose);
     (void)hipFree(tr->stage_out.pos3d);
@@ -1024,7 +1152,8 @@ int pf_tracker_create(pf_tracker **out, const pf_tracker_config *cfg, pf_handle 
     st = hip_ok(talloc(&tr->taps, taps.size()), "hipMalloc");
     if (!st) st = hip_ok(hipMemcpy(tr->taps, taps.data(), sizeof(float) * taps.size(), hipMemcpyHostToDevice), "hipMemcpy");
     if (!st) st = hip_ok(talloc(&tr->img_stage, px), "hipMalloc");
-    if (!st) st = hip_ok(talloc(&tr->blur, px), "hipMalloc");
+    if (!st) st = hip_ok(talloc(&tr->blur, kBlurSlots * px), "hipMalloc");
+    if (!st) st = hip_ok(talloc(&tr->run, 1), "hipMalloc");
     if (!st) st = hip_ok(talloc(&tr->roi_stage, 4), "hipMalloc");
     if (!st) st = hip_ok(talloc(&tr->rec, 1), "hipMalloc");
     if (!st) st = hip_ok(hipMemset(tr->rec, 0, sizeof(FrameRec)), "hipMemset");
@@ -1076,40 +1205,54 @@ int pf_tracker_run_dev(pf_tracker *tr, int32_t T, const uint8_t *likelihood, con
         if (!in.tracks) return set_error(PF_ERR_STATE, "arm %d tracks not initialised", a + 1);
         if (in.N != tr->N) return set_error(PF_ERR_STATE, "arm %d particle count changed", a + 1);
     }
-    const bool graph = (flags & 1) != 0;
-    st = upload_uniforms(tr, T);
+    st = ensure_run(tr, T);
     if (st) return st;
     TR_TRY(hipEventRecord(tr->ev_t0, tr->s[0]));
-    hipLaunchKernelGGL(k_tr_set, dim3(1), dim3(64), 0, tr->s[0], tr->fctr, 0);
-    st = launch_check("k_tr_set");
-    for (int a = 0; !st && a < 2; ++a) st = eng::set_frame(tr->arm[a], 0);
-    if (!st) st = prepare_estimates(tr);
+    st = prepare_estimates(tr);
     if (st) return st;
-    auto frame = [&](int f) { return enqueue_frame(tr, f & 1, T, likelihood, roi, out); };
-    st = frame(0);
+    BeginArgs ba{};
+    ba.v.lik = likelihood;
+    ba.v.roi = roi;
+    ba.v.lml = out.lml;
+    ba.v.pose = out.pose;
+    ba.v.pos3d = out.pos3d;
+    ba.v.tf = out.tf;
+    ba.v.pose2d = out.pose2d;
+    ba.v.g0 = tr->frames_done;
+    ba.v.uniform_frame = tr->uniform_frame;
+    ba.v.T = T;
+    ba.run = tr->run;
+    ba.fctr = tr->fctr;
+    for (int a = 0; a < 2; ++a) {
+        ba.arm_frame[a] = eng::frame_counters(tr->arm[a]);
+        ba.fs[a] = eng::scratch(tr->arm[a]);
+    }
+    for (int k = 0; k < 3; ++k) ba.uni[k] = tr->uni + (size_t)2 * k * tr->run_cap;
+    ba.seed = tr->cfg.seed;
+    hipLaunchKernelGGL(k_tr_begin, dim3((T + 63) / 64), dim3(64), 0, tr->s[0], ba);
+    st = launch_check("k_tr_begin");
     if (st) return st;
-    // kTrGraphFrames consecutive frames (an even count: frame f uses the
-    // buffers and counters of parity f & 1) captured once and replayed
-    const int reps = graph ? (T - 1) / kTrGraphFrames : 0;
-    if (reps > 0) {
-        hipGraph_t gr;
-        hipGraphExec_t ge;
-        TR_TRY(hipStreamBeginCapture(tr->s[0], hipStreamCaptureModeThreadLocal));
-        int sc = 0;
-        for (int f = 1; f <= kTrGraphFrames && !sc; ++f) sc = frame(f);
-        hipError_t ec = hipStreamEndCapture(tr->s[0], &gr);
-        if (sc) return sc;
-        if (ec != hipSuccess) return set_error(PF_ERR_HIP, "graph capture failed: %s", hipGetErrorString(ec));
-        TR_TRY(hipGraphInstantiate(&ge, gr, nullptr, nullptr, 0));
-        for (int q = 0; q < reps; ++q) TR_TRY(hipGraphLaunch(ge, tr->s[0]));
-        TR_TRY(hipStreamSynchronize(tr->s[0]));
-        (void)hipGraphExecDestroy(ge);
-        (void)hipGraphDestroy(gr);
+    for (int f = 0; f < T;) {
+        int g = kTrGroups - 1;
+        while ((1 << g) > T - f) --g;
+        if (flags & 1) {
+            hipGraphExec_t ge;
+            st = frame_group(tr, g, &ge);
+            if (st) return st;
+            TR_TRY(hipGraphLaunch(ge, tr->s[0]));
+            if (g == 0)
+                for (pf_handle *arm : tr->arm) eng::swap_state_buffer(arm);
+        } else {
+            st = enqueue_group(tr, 1 << g);
+            if (st) return st;
+        }
+        f += 1 << g;
     }
-    for (int f = 1 + reps * kTrGraphFrames; f < T; ++f) {
-        st = frame(f);
-        if (st) return st;
-    }
+    tr->last_slot = (T - 1) % kBlurSlots;
+    hipLaunchKernelGGL(k_tr_end, dim3((T + 255) / 256), dim3(256), 0, tr->s[0], (const TrackerRun *)tr->run,
+                       (const double *)tr->lml, (const double *)(tr->lml + tr->run_cap));
+    st = launch_check("k_tr_end");
+    if (st) return st;
     TR_TRY(hipEventRecord(tr->ev_t1, tr->s[0]));
     // arm 2's stream orders its later work after the run (the frames may
     // have advanced arm 2 on stream 0)
@@ -1158,7 +1301,7 @@ int pf_tracker_frame(pf_tracker *tr, const uint8_t *likelihood, const int32_t *r
     TR_TRY(hipMemcpyAsync(tr->img_stage, likelihood, px, hipMemcpyHostToDevice, tr->s[0]));
     TR_TRY(hipMemcpyAsync(tr->roi_stage, roi, sizeof(int32_t) * 4, hipMemcpyHostToDevice, tr->s[0]));
     TR_TRY(hipStreamSynchronize(tr->s[0]));
-    st = pf_tracker_run_dev(tr, 1, tr->img_stage, tr->roi_stage, &tr->stage_out, 0);
+    st = pf_tracker_run_dev(tr, 1, tr->img_stage, tr->roi_stage, &tr->stage_out, 1);
     if (st) return st;
     st = copy_stage_out(tr, o);
     if (st) return st;
@@ -1173,11 +1316,12 @@ int pf_tracker_get_last(pf_tracker *tr, uint8_t *blurred, double *proposals, dou
     if (!tr->ran) return set_error(PF_ERR_STATE, "no frame yet");
     hipStream_t s = tr->s[0];
     const size_t px = (size_t)tr->cfg.rows * tr->cfg.cols;
-    if (blurred) TR_TRY(hipMemcpyAsync(blurred, tr->blur, px, hipMemcpyDeviceToHost, s));
+    if (blurred)
+        TR_TRY(hipMemcpyAsync(blurred, tr->blur + tr->last_slot * px, px, hipMemcpyDeviceToHost, s));
     if (proposals) {
         double *d = nullptr;
         TR_TRY(talloc(&d, (size_t)4 * tr->n_c));
-        PropParams p = prop_params(tr, nullptr, nullptr);
+        PropParams p = prop_params(tr);
         hipLaunchKernelGGL(k_dump_proposals, dim3((tr->n_c + 255) / 256, 2), dim3(256), 0, s, p,
                            (const FrameRec *)tr->rec, d);
         st = launch_check("k_dump_proposals");
@@ -1216,7 +1360,7 @@ int pf_tracker_pose(pf_tracker *tr, const pf_tracker_outputs *out)
     if (st) return st;
     hipLaunchKernelGGL(k_tr_set, dim3(1), dim3(64), 0, tr->s[0], tr->fctr_aux, 0);
     st = launch_check("k_tr_set");
-    if (!st) st = launch_pose(tr, tr->fctr_aux, tr->stage_out);
+    if (!st) st = launch_pose(tr, tr->fctr_aux, &tr->stage_out);
     if (st) return st;
     pf_tracker_outputs o{};
     if (out) o = *out;
@@ -1234,7 +1378,7 @@ int pf_tracker_blur(pf_tracker *tr, const uint8_t *src, uint8_t *dst)
     TR_TRY(talloc(&d, px));
     hipError_t e = hipMemcpyAsync(tr->img_stage, src, px, hipMemcpyHostToDevice, tr->s[0]);
     if (e == hipSuccess) {
-        st = launch_blur(tr, tr->img_stage, nullptr, d);
+        st = launch_blur(tr, tr->img_stage, d, 1);
         if (!st) e = hipMemcpyAsync(dst, d, px, hipMemcpyDeviceToHost, tr->s[0]);
         if (!st && e == hipSuccess) e = hipStreamSynchronize(tr->s[0]);
     }
