@@ -732,13 +732,15 @@ int pf_batch_destroy(pf_batch *b)
     (void)hipSetDevice(b->device);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     void *ptrs[] = {b->bx[0], b->bx[1], b->bP[0], b->bP[1], b->lw, b->tables, b->mus, b->sigs, b->Tis, b->Ts,
-                    b->bexp, b->bpow, b->partial, b->est, b->gbuf, b->anc, b->frame, b->maxkey, b->cloc, b->bsum,
+                    b->bexp, b->bpow, b->partial, b->gbuf, b->anc, b->frame, b->maxkey, b->cloc, b->bsum,
                     b->cloc1, b->bsum1, b->bexp1, b->bpow1, b->status, b->seqs, b->tile_seq, b->tile_j0, b->n_tiles, b->wb_seq, b->wb_b,
                     b->n_wblocks, b->fs, b->rec_comp, b->rec_anc, b->rec_bins, b->ck_x, b->ck_P, b->seg_x[0],
                     b->seg_x[1], b->seg_P[0], b->seg_P[1], b->adj_x[0], b->adj_x[1], b->adj_P[0], b->adj_P[1], b->first, b->tacc, b->gsum,
                     b->t256_seq, b->t256_j0, b->t256_first};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    (void)hipHostFree(b->est);
+    (void)hipHostFree(b->h_bins);
     if (b->stream) (void)hipStreamDestroy(b->stream);
     if (b->stream2) {
         (void)hipStreamSynchronize(b->stream2);
@@ -816,7 +818,8 @@ int pf_batch_create(pf_batch **out, int32_t S, const int32_t *n_particles, const
     e = e ? e : dallocb(&b->frame, 2);
     e = e ? e : dallocb(&b->rec_bins, (size_t)b->ld);
     e = e ? e : dallocb(&b->partial, (size_t)kMaxScanBlocks * 64);
-    e = e ? e : dallocb(&b->est, 64);
+    e = e ? e : hipHostMalloc((void **)&b->est, 64 * sizeof(double), hipHostMallocDefault);
+    e = e ? e : hipHostMalloc((void **)&b->h_bins, std::min(sizeof(int) * (size_t)b->ld, kMailMax), hipHostMallocDefault);
     e = e ? e : dallocb(&b->fs, 1);
     if (e == hipSuccess) e = hipMemset(b->maxkey, 0, sizeof(unsigned long long) * 2 * S);
     if (e == hipSuccess) e = hipMemset(b->status, 0, sizeof(unsigned) * S);
@@ -900,7 +903,14 @@ int pf_batch_reset(pf_batch *b, int32_t s, const int32_t *bins)
     const SeqDesc &sd = b->h_seqs[i];
     for (int j = 0; j < sd.N; ++j)
         if (bins[j] < 0 || bins[j] >= b->K) return set_error(PF_ERR_ARG, "bins[%d] out of range", j);
-    HIP_TRYB(hipMemcpyAsync(b->rec_bins + sd.pofs, bins, sizeof(int) * sd.N, hipMemcpyHostToDevice, b->stream));
+    if (sizeof(int) * (size_t)sd.N <= kMailMax) {
+        std::memcpy(b->h_bins, bins, sizeof(int) * (size_t)sd.N);
+        hipLaunchKernelGGL(k_copy_words, dim3((sd.N + 255) / 256), dim3(256), 0, b->stream,
+                           reinterpret_cast<const uint32_t *>(b->h_bins),
+                           reinterpret_cast<uint32_t *>(b->rec_bins + sd.pofs), sd.N);
+    } else {
+        HIP_TRYB(hipMemcpyAsync(b->rec_bins + sd.pofs, bins, sizeof(int) * sd.N, hipMemcpyHostToDevice, b->stream));
+    }
     auto reset = b->D == 24 ? launch_reset<24> : launch_reset<kBD>;
     reset(b->stream, b->rec_bins + sd.pofs, b->mus + (size_t)i * b->K * b->D,
           b->sigs + (size_t)i * b->K * npacked(b->D), b->bx[0] + sd.pofs, b->bP[0] + sd.pofs, b->anc + sd.pofs, sd.N,
@@ -1058,8 +1068,8 @@ int pf_batch_estimate(pf_batch *b, int32_t s, double *xbar)
         launch_estimate<kBD>(b->stream, b->bx[buf] + sd.pofs, b->anc + sd.pofs, sd.N, Lay{b->ld, 1}, b->partial,
                              b->Tis + (size_t)i * b->D * b->D, b->est);
     HIP_TRYB(hipGetLastError());
-    HIP_TRYB(hipMemcpyAsync(xbar, b->est, sizeof(double) * b->D, hipMemcpyDeviceToHost, b->stream));
     HIP_TRYB(hipStreamSynchronize(b->stream));
+    std::memcpy(xbar, b->est, sizeof(double) * b->D);
     return PF_OK;
 }
 

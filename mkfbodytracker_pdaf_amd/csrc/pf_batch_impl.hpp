@@ -160,7 +160,9 @@ struct pf_batch {
     hipStream_t stream = nullptr;
     float *bx[2] = {nullptr, nullptr}, *bP[2] = {nullptr, nullptr};
     float *lw = nullptr, *tables = nullptr, *mus = nullptr, *sigs = nullptr;
-    double *Tis = nullptr, *Ts = nullptr, *bexp = nullptr, *bexp1 = nullptr, *partial = nullptr, *est = nullptr;
+    double *Tis = nullptr, *Ts = nullptr, *bexp = nullptr, *bexp1 = nullptr, *partial = nullptr;
+    double *est = nullptr;         // pinned host memory, as the next
+    int *h_bins = nullptr;         // a sequence's bins on their way to rec_bins
     double *gbuf = nullptr;
     int *bpow = nullptr, *bpow1 = nullptr;
     size_t gbuf_bytes = 0;

@@ -97,9 +97,12 @@ struct pf_handle {
     unsigned long long *cloc1 = nullptr, *bsum1 = nullptr;
     double *bexp1 = nullptr;
     int *bpow1 = nullptr;
-    // staging for host-driven calls
+    // pinned host buffer of the host-driven calls: the estimate (64 doubles),
+    // then a frame's or a reset's data
+    unsigned char *mail = nullptr;
+    size_t mail_bytes = 0;
+    // device inputs of host-driven calls
     float *zbuf = nullptr;
-    int *cntbuf = nullptr;
     float *candbuf = nullptr;
     double *est_partial = nullptr, *est_out = nullptr;
     double *gbuf = nullptr;
@@ -208,6 +211,21 @@ int ensure_ibuf(pf_handle *h, size_t bytes)
     return PF_OK;
 }
 
+constexpr size_t kMailHead = 64 * sizeof(double);   // the estimate's place
+
+// At least `bytes` of the pinned buffer after its head (the stream is idle:
+// every call that uses the buffer waits before it returns).
+int ensure_mail(pf_handle *h, size_t bytes)
+{
+    if (kMailHead + bytes <= h->mail_bytes) return PF_OK;
+    (void)hipHostFree(h->mail);
+    h->mail = nullptr;
+    h->mail_bytes = 0;
+    HIP_TRY(hipHostMalloc((void **)&h->mail, kMailHead + bytes, hipHostMallocDefault));
+    h->mail_bytes = kMailHead + bytes;
+    return PF_OK;
+}
+
 int check_launch(const char *what)
 {
     hipError_t e = hipGetLastError();
@@ -277,7 +295,8 @@ template <int D>
 struct EstimateL {
     static void run(pf_handle *h)
     {
-        launch_estimate<D>(h->stream, h->xA, h->anc, h->N, h->lay, h->est_partial, h->Tinv, h->est_out);
+        launch_estimate<D>(h->stream, h->xA, h->anc, h->N, h->lay, h->est_partial, h->Tinv, h->est_out,
+                           (double *)h->mail);
     }
 };
 
@@ -545,7 +564,7 @@ struct AncEstimateL {
         hipLaunchKernelGGL((k_ancestors_estimate<D>), dim3(anc_blocks(h->N)), dim3(256), lds, h->stream, an, (const float *)h->xB,
                            h->lay, h->est_partial);
         hipLaunchKernelGGL((k_estimate_final<D>), dim3(1), dim3(256), 0, h->stream, (const double *)h->est_partial, nb,
-                           h->N, (const double *)h->Tinv, h->est_out);
+                           h->N, (const double *)h->Tinv, h->est_out, (double *)nullptr);
     }
 };
 
@@ -764,10 +783,11 @@ int pf_destroy(pf_handle *h)
     drop_graphs(h);
     void *ptrs[] = {h->run_desc, h->run_ctr, h->rec[0], h->rec[1], h->anc, h->comp, h->bins, h->lw, h->table,
                     h->mu, h->sig, h->fs, h->frame, h->uni, h->lml1, h->cloc, h->bsum, h->bexp, h->bpow,
-                    h->gpre, h->gshf, h->cloc1, h->bsum1, h->bexp1, h->bpow1, h->zbuf, h->cntbuf, h->candbuf, h->est_partial, h->est_out, h->gbuf, h->ibuf,
+                    h->gpre, h->gshf, h->cloc1, h->bsum1, h->bexp1, h->bpow1, h->zbuf, h->candbuf, h->est_partial, h->est_out, h->gbuf, h->ibuf,
                     h->Tdev, h->Tinv};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
+    (void)hipHostFree(h->mail);
     for (hipEvent_t e : h->ev) (void)hipEventDestroy(e);
     if (h->stream) (void)hipStreamDestroy(h->stream);
     delete h;
@@ -793,8 +813,8 @@ int pf_load_model(pf_handle *h, int32_t K, int32_t d, int32_t npose, int32_t m, 
     (void)hipFree(h->rec[0]); (void)hipFree(h->rec[1]);
     h->rec[0] = h->rec[1] = nullptr;
     h->xA = h->PA = h->xB = h->PB = nullptr;
-    (void)hipFree(h->zbuf); (void)hipFree(h->cntbuf); (void)hipFree(h->candbuf);
-    h->zbuf = nullptr; h->cntbuf = nullptr; h->candbuf = nullptr;
+    (void)hipFree(h->zbuf); (void)hipFree(h->candbuf);
+    h->zbuf = nullptr; h->candbuf = nullptr;
     h->model = false;
     h->tracks = false;
     // room for either layout (a record is padded to 16 bytes)
@@ -835,7 +855,17 @@ int pf_reset(pf_handle *h, const int32_t *bins)
     if (!bins) return set_error(PF_ERR_ARG, "null bins");
     for (int j = 0; j < h->N; ++j)
         if (bins[j] < 0 || bins[j] >= h->K) return set_error(PF_ERR_ARG, "bins[%d]=%d out of range", j, bins[j]);
-    HIP_TRY(hipMemcpyAsync(h->bins, bins, sizeof(int) * h->N, hipMemcpyHostToDevice, h->stream));
+    const size_t bytes = sizeof(int) * (size_t)h->N;
+    if (bytes <= kMailMax) {
+        st = ensure_mail(h, bytes);
+        if (st) return st;
+        std::memcpy(h->mail + kMailHead, bins, bytes);
+        hipLaunchKernelGGL(k_copy_words, dim3((h->N + 255) / 256), dim3(256), 0, h->stream,
+                           reinterpret_cast<const uint32_t *>(h->mail + kMailHead),
+                           reinterpret_cast<uint32_t *>(h->bins), h->N);
+    } else {
+        HIP_TRY(hipMemcpyAsync(h->bins, bins, bytes, hipMemcpyHostToDevice, h->stream));
+    }
     st = dispatch_d<ResetL>(h->D, h);
     if (!st) st = check_launch("k_reset");
     if (st) return st;
@@ -881,22 +911,111 @@ int pf_get_tracks(pf_handle *h, double *x, double *P)
     return PF_OK;
 }
 
-static int finish_host_step(pf_handle *h, float *lw, int32_t *anc, int32_t *comp, double *lml)
+namespace {
+
+// Places of a host-driven frame in the pinned buffer: `words` input words,
+// then the outputs of N particles.
+struct MailLayout {
+    size_t lml, status, lw, anc, comp, total;
+    bool used;                    // else copies (kMailMax)
+    MailLayout(size_t words, size_t N)
+    {
+        lml = (4 * words + 15) & ~(size_t)15;
+        status = lml + 8;
+        lw = lml + 16;
+        anc = lw + 4 * N;
+        comp = anc + 4 * N;
+        total = comp + 4 * N;
+        used = total <= kMailMax;
+    }
+};
+
+// The frame's input words on their way to dst: in the pinned buffer, or in a
+// vector whose copy has to end before the vector does (host_step waits).
+struct MailWords {
+    std::vector<float> own;
+    float *p = nullptr;
+    int open(pf_handle *h, const MailLayout &L, size_t words)
+    {
+        if (!L.used) {
+            own.resize(words);
+            p = own.data();
+            return PF_OK;
+        }
+        int st = ensure_mail(h, L.total);
+        if (!st) p = reinterpret_cast<float *>(h->mail + kMailHead);
+        return st;
+    }
+};
+
+// Sends the frame's input words and its uniforms.
+int mail_in(pf_handle *h, const MailLayout &L, const MailWords &in, float *dst, size_t words, uint32_t u_comp,
+            uint32_t u_res)
 {
-    int st = launch_weights(h, h->uni, 0);
-    if (st) return st;
-    st = launch_ancestors(h, h->N, h->N, h->anc, 0, 0, h->lml1);
+    if (!L.used) {
+        HIP_TRY(hipMemcpyAsync(dst, in.p, 4 * words, hipMemcpyHostToDevice, h->stream));
+        words = 0;
+    }
+    MailIn m{};
+    m.src = reinterpret_cast<const uint32_t *>(in.p);
+    m.dst = reinterpret_cast<uint32_t *>(dst);
+    m.words = (int)words;
+    m.u0 = u_comp;
+    m.u1 = u_res;
+    m.uni = h->uni;
+    m.frame = h->frame;
+    m.fs = h->fs;
+    hipLaunchKernelGGL(k_mail_in, dim3((unsigned)((words / 4 + 256) / 256)), dim3(256), 0, h->stream, m);
+    return check_launch("k_mail_in");
+}
+
+// The step of a host-driven frame, its resampling and its outputs.
+int host_step(pf_handle *h, StepArgs &a, int mode, const MailLayout &L, float *lw, int32_t *anc, int32_t *comp,
+              double *lml)
+{
+    const int block = h->cfg.block_size > 0 ? h->cfg.block_size : 256;
+    const bool fused = block == kWeightsBlock;     // the step writes the frame's weights itself
+    if (fused) write_weights(h, a, 0);
+    int st = launch_step(h, a, mode);
+    if (!st && !fused) st = launch_weights(h, h->uni, 0);
+    if (!st) st = launch_ancestors(h, h->N, h->N, h->anc, 0, 0, h->lml1, nullptr, 0, fused ? h->frame : nullptr);
     if (st) return st;
     swap_state(h);
-    if (lw) HIP_TRY(hipMemcpyAsync(lw, h->lw, sizeof(float) * h->N, hipMemcpyDeviceToHost, h->stream));
-    if (anc) HIP_TRY(hipMemcpyAsync(anc, h->anc, sizeof(int) * h->N, hipMemcpyDeviceToHost, h->stream));
-    if (comp) HIP_TRY(hipMemcpyAsync(comp, h->comp, sizeof(int) * h->N, hipMemcpyDeviceToHost, h->stream));
-    if (lml) HIP_TRY(hipMemcpyAsync(lml, h->lml1, sizeof(double), hipMemcpyDeviceToHost, h->stream));
-    unsigned word = 0;
-    st = read_status(h, &word);
+    if (!L.used) {
+        if (lw) HIP_TRY(hipMemcpyAsync(lw, h->lw, sizeof(float) * h->N, hipMemcpyDeviceToHost, h->stream));
+        if (anc) HIP_TRY(hipMemcpyAsync(anc, h->anc, sizeof(int) * h->N, hipMemcpyDeviceToHost, h->stream));
+        if (comp) HIP_TRY(hipMemcpyAsync(comp, h->comp, sizeof(int) * h->N, hipMemcpyDeviceToHost, h->stream));
+        if (lml) HIP_TRY(hipMemcpyAsync(lml, h->lml1, sizeof(double), hipMemcpyDeviceToHost, h->stream));
+        unsigned word = 0;
+        st = read_status(h, &word);
+        return st ? st : status_code(word);
+    }
+    unsigned char *m = h->mail + kMailHead;
+    MailOut o{};
+    o.lw = h->lw;
+    o.anc = h->anc;
+    o.comp = h->comp;
+    o.h_lw = lw ? reinterpret_cast<float *>(m + L.lw) : nullptr;
+    o.h_anc = anc ? reinterpret_cast<int *>(m + L.anc) : nullptr;
+    o.h_comp = comp ? reinterpret_cast<int *>(m + L.comp) : nullptr;
+    o.lml = h->lml1;
+    o.h_lml = reinterpret_cast<double *>(m + L.lml);
+    o.fs = h->fs;
+    o.h_status = reinterpret_cast<unsigned *>(m + L.status);
+    o.N = h->N;
+    hipLaunchKernelGGL(k_mail_out, dim3((h->N + 255) / 256), dim3(256), 0, h->stream, o);
+    st = check_launch("k_mail_out");
     if (st) return st;
-    return status_code(word);
+    HIP_TRY(hipStreamSynchronize(h->stream));
+    const size_t bytes = sizeof(float) * (size_t)h->N;
+    if (lw) std::memcpy(lw, o.h_lw, bytes);
+    if (anc) std::memcpy(anc, o.h_anc, bytes);
+    if (comp) std::memcpy(comp, o.h_comp, bytes);
+    if (lml) *lml = *o.h_lml;
+    return status_code(*o.h_status);
 }
+
+}  // namespace
 
 int pf_step(pf_handle *h, const double *Z, uint32_t u_comp, uint32_t u_res, float *lw, int32_t *anc,
             int32_t *comp, double *lml)
@@ -906,18 +1025,18 @@ int pf_step(pf_handle *h, const double *Z, uint32_t u_comp, uint32_t u_res, floa
     if (!h->tracks) return set_error(PF_ERR_STATE, "tracks not initialised (pf_reset or pf_set_tracks)");
     if (!Z) return set_error(PF_ERR_ARG, "null measurement");
     const int m = h->m, N = h->N;
-    if (!h->zbuf) HIP_TRY(dalloc(&h->zbuf, (size_t)m * N));
-    std::vector<float> zf((size_t)m * N);
-    for (size_t i = 0; i < zf.size(); ++i) zf[i] = (float)Z[i];
-    const uint32_t u[2] = {u_comp, u_res};
-    HIP_TRY(hipMemcpyAsync(h->zbuf, zf.data(), sizeof(float) * zf.size(), hipMemcpyHostToDevice, h->stream));
-    HIP_TRY(hipMemcpyAsync(h->uni, u, sizeof(u), hipMemcpyHostToDevice, h->stream));
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, h->stream, h->frame, 0);
+    const size_t words = (size_t)m * N;
+    if (!h->zbuf) HIP_TRY(dalloc(&h->zbuf, words));
+    const MailLayout L(words, N);
+    MailWords in;
+    st = in.open(h, L, words);
+    if (st) return st;
+    for (size_t i = 0; i < words; ++i) in.p[i] = (float)Z[i];
+    st = mail_in(h, L, in, h->zbuf, words, u_comp, u_res);
+    if (st) return st;
     StepArgs a = step_args(h, kModeRef, h->uni, h->zbuf, 0, N, nullptr, nullptr, comp ? h->comp : nullptr, 0,
                            kAncArray, nullptr);
-    st = launch_step(h, a, kModeRef);
-    if (st) return st;
-    return finish_host_step(h, lw, anc, comp, lml);
+    return host_step(h, a, kModeRef, L, lw, anc, comp, lml);
 }
 
 int pf_step_candidates(pf_handle *h, const int32_t *count, const double *cand, uint32_t u_comp,
@@ -930,20 +1049,19 @@ int pf_step_candidates(pf_handle *h, const int32_t *count, const double *cand, u
     const int J = h->J, cap = h->cap;
     for (int b = 0; b < J; ++b)
         if (count[b] < 0 || count[b] > cap) return set_error(PF_ERR_ARG, "count[%d]=%d outside 0..%d", b, count[b], cap);
-    if (!h->cntbuf) HIP_TRY(dalloc(&h->cntbuf, (size_t)J));
-    if (!h->candbuf) HIP_TRY(dalloc(&h->candbuf, (size_t)J * cap * 2));
-    std::vector<float> cf((size_t)J * cap * 2);
-    for (size_t i = 0; i < cf.size(); ++i) cf[i] = (float)cand[i];
-    const uint32_t u[2] = {u_comp, u_res};
-    HIP_TRY(hipMemcpyAsync(h->cntbuf, count, sizeof(int) * J, hipMemcpyHostToDevice, h->stream));
-    HIP_TRY(hipMemcpyAsync(h->candbuf, cf.data(), sizeof(float) * cf.size(), hipMemcpyHostToDevice, h->stream));
-    HIP_TRY(hipMemcpyAsync(h->uni, u, sizeof(u), hipMemcpyHostToDevice, h->stream));
-    hipLaunchKernelGGL(k_set_int, dim3(1), dim3(64), 0, h->stream, h->frame, 0);
-    StepArgs a = step_args(h, kModeCand, h->uni, nullptr, 0, 0, h->cntbuf, h->candbuf, comp ? h->comp : nullptr, 0,
-                           kAncArray, nullptr);
-    st = launch_step(h, a, kModeCand);
+    const size_t nc = (size_t)J * cap * 2, words = nc + J;      // detections, then counts
+    if (!h->candbuf) HIP_TRY(dalloc(&h->candbuf, words));
+    const MailLayout L(words, h->N);
+    MailWords in;
+    st = in.open(h, L, words);
     if (st) return st;
-    return finish_host_step(h, lw, anc, comp, lml);
+    for (size_t i = 0; i < nc; ++i) in.p[i] = (float)cand[i];
+    std::memcpy(in.p + nc, count, sizeof(int) * J);
+    st = mail_in(h, L, in, h->candbuf, words, u_comp, u_res);
+    if (st) return st;
+    StepArgs a = step_args(h, kModeCand, h->uni, nullptr, 0, 0, reinterpret_cast<const int *>(h->candbuf + nc),
+                           h->candbuf, comp ? h->comp : nullptr, 0, kAncArray, nullptr);
+    return host_step(h, a, kModeCand, L, lw, anc, comp, lml);
 }
 
 int pf_estimate(pf_handle *h, double *xbar)
@@ -952,10 +1070,13 @@ int pf_estimate(pf_handle *h, double *xbar)
     if (st) return st;
     if (!h->tracks) return set_error(PF_ERR_STATE, "tracks not initialised");
     if (!xbar) return set_error(PF_ERR_ARG, "null output");
-    st = dispatch_d<EstimateL>(h->D, h);
+    st = ensure_mail(h, 0);
     if (st) return st;
-    HIP_TRY(hipMemcpyAsync(xbar, h->est_out, sizeof(double) * h->D, hipMemcpyDeviceToHost, h->stream));
+    st = dispatch_d<EstimateL>(h->D, h);
+    if (!st) st = check_launch("k_estimate");
+    if (st) return st;
     HIP_TRY(hipStreamSynchronize(h->stream));
+    std::memcpy(xbar, h->mail, sizeof(double) * h->D);
     return PF_OK;
 }
 

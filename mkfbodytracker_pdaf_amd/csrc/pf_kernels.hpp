@@ -1859,6 +1859,72 @@ __global__ void __launch_bounds__(256) k_blockmax64(const double *w, int L, Fram
     if ((threadIdx.x & 63) == 0 && isfinite(v)) atomicMax(&fs->maxkey[0], order_key(v));
 }
 
+// ------------------------------------------------- host-driven frames
+// A host-driven frame exchanges its inputs and outputs with the device
+// through one pinned host buffer, read by k_mail_in before the step and written
+// by k_mail_out after the resampling: one wait per call.  (Pageable copies,
+// each a copy kernel, most with a wait of its own: 153 us for a step at N = 500
+// with its outputs and the estimate, 57 through the buffer.)
+// Larger exchanges than this go by copies, from and to the caller's memory (a
+// pinned buffer of that size takes longer to allocate than it saves).
+constexpr size_t kMailMax = size_t(4) << 20;
+
+static __global__ void __launch_bounds__(256) k_copy_words(const uint32_t *src, uint32_t *dst, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+struct MailIn {
+    const uint32_t *src;      // words words from host memory ...
+    uint32_t *dst;            // ... to the frame's device inputs
+    int words;
+    uint32_t u0, u1;          // the frame's uniforms
+    uint32_t *uni;
+    int *frame;               // frame counter 0, set to 0
+    FrameScratch *fs;         // frame 0's exponent slot is cleared
+};
+
+static __global__ void __launch_bounds__(256) k_mail_in(MailIn a)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        a.uni[0] = a.u0;
+        a.uni[1] = a.u1;
+        *a.frame = 0;
+        a.fs->pow_max[0] = kPowEmpty;
+    }
+    const int n4 = a.words >> 2;
+    if (i < n4) reinterpret_cast<uint4 *>(a.dst)[i] = reinterpret_cast<const uint4 *>(a.src)[i];
+    if (i < (a.words & 3)) a.dst[4 * n4 + i] = a.src[4 * n4 + i];
+}
+
+struct MailOut {
+    const float *lw;          // N each; their host copies are nullable
+    const int *anc, *comp;
+    float *h_lw;
+    int *h_anc, *h_comp;
+    const double *lml;
+    double *h_lml;
+    FrameScratch *fs;         // its status word is read and cleared
+    unsigned int *h_status;
+    int N;
+};
+
+static __global__ void __launch_bounds__(256) k_mail_out(MailOut a)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i == 0) {
+        *a.h_lml = *a.lml;
+        *a.h_status = a.fs->status;
+        a.fs->status = 0u;
+    }
+    if (i >= a.N) return;
+    if (a.h_lw) a.h_lw[i] = a.lw[i];
+    if (a.h_anc) a.h_anc[i] = a.anc[i];
+    if (a.h_comp) a.h_comp[i] = a.comp[i];
+}
+
 // ---------------------------------------------------------------- helpers
 static __global__ void k_set_int(int *p, int v)
 {
@@ -2117,7 +2183,7 @@ __global__ void __launch_bounds__(256) k_estimate(const float *x, const int *anc
 // Sum of the nb block partials, / N, back to the model basis (xbar = Ti xbar').
 template <int D>
 __device__ __forceinline__ void estimate_final_body(const double *partial, int nb, int N, const double *Ti,
-                                                    double *out)
+                                                    double *out, double *out2 = nullptr)
 {
     __shared__ double s_v[D][16][17];
     __shared__ double s_run[D][16];
@@ -2134,14 +2200,16 @@ __device__ __forceinline__ void estimate_final_body(const double *partial, int n
         double r = 0.0;
         for (int k = 0; k < D; ++k) r = fma(Ti[threadIdx.x * D + k], s_sum[k] / (double)N, r);
         out[threadIdx.x] = r;
+        if (out2) out2[threadIdx.x] = r;
     }
 }
 
+// out2 (optional): a second copy, in pinned host memory for a caller that waits.
 template <int D>
 __global__ void __launch_bounds__(256) k_estimate_final(const double *partial, int nb, int N, const double *Ti,
-                                                        double *out)
+                                                        double *out, double *out2)
 {
-    estimate_final_body<D>(partial, nb, N, Ti, out);
+    estimate_final_body<D>(partial, nb, N, Ti, out, out2);
 }
 
 // The estimates of two filters (block b = filter b).
@@ -2208,11 +2276,12 @@ __host__ __device__ constexpr int anc_estimate_lds_bytes(int nb, int D)
 // Both estimate kernels on one stream.
 template <int D>
 inline void launch_estimate(hipStream_t st, const float *x, const int *anc, int N, Lay L, double *partial,
-                            const double *Ti, double *out)
+                            const double *Ti, double *out, double *out2 = nullptr)
 {
     const int nb = (N + 255) / 256;
     hipLaunchKernelGGL((k_estimate<D>), dim3(nb), dim3(256), 0, st, x, anc, N, L, partial);
-    hipLaunchKernelGGL((k_estimate_final<D>), dim3(1), dim3(256), 0, st, (const double *)partial, nb, N, Ti, out);
+    hipLaunchKernelGGL((k_estimate_final<D>), dim3(1), dim3(256), 0, st, (const double *)partial, nb, N, Ti, out,
+                       out2);
 }
 
 // getSamples (pf2DRao.cpp:85-103): out = y[0:2] + 0.8 scale n, y = Hp xbar + M.
