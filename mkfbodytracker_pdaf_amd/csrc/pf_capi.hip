@@ -551,6 +551,35 @@ int estimate(pf_handle *h)
     return check_launch("k_estimate");
 }
 
+template <int D>
+struct EstimatePairL {
+    static void run(hipStream_t s, EstPairArgs a)
+    {
+        const int n = std::max(a.N[0], a.N[1]);
+        hipLaunchKernelGGL((k_estimate_pair<D>), dim3((n + 255) / 256, 2), dim3(256), 0, s, a);
+        hipLaunchKernelGGL((k_estimate_final_pair<D>), dim3(2), dim3(256), 0, s, a);
+    }
+};
+
+int estimate_pair(pf_handle *h0, pf_handle *h1, hipStream_t s)
+{
+    if (h0->D != h1->D) return set_error(PF_ERR_ARG, "filters of different state dimensions");
+    EstPairArgs a{};
+    pf_handle *h[2] = {h0, h1};
+    for (int k = 0; k < 2; ++k) {
+        a.x[k] = h[k]->xA;
+        a.anc[k] = h[k]->anc;
+        a.N[k] = h[k]->N;
+        a.L[k] = h[k]->lay;
+        a.partial[k] = h[k]->est_partial;
+        a.Ti[k] = h[k]->Tinv;
+        a.out[k] = h[k]->est_out;
+    }
+    int st = dispatch_d<EstimatePairL>(h0->D, s, a);
+    if (st) return st;
+    return check_launch("k_estimate_pair");
+}
+
 Pending pending(pf_handle *h, int L) { return pending_of(h, L, false); }
 
 FrameScratch *scratch(pf_handle *h) { return h->fs; }
@@ -691,8 +720,6 @@ int step_ref_pair(pf_handle *h0, pf_handle *h1, const float *Z0, const float *Z1
     swap_state(h1);
     return PF_OK;
 }
-
-int take_status(pf_handle *h, unsigned *word) { return read_status(h, word); }
 
 }  // namespace eng
 }  // namespace mkfbt

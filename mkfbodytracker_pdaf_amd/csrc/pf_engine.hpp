@@ -38,6 +38,9 @@ int state_buffer(const pf_handle *h);
 void swap_state_buffer(pf_handle *h);
 // getEstimator (pf2DRao.cpp:23-31) of the current tracks into estimate_ptr().
 int estimate(pf_handle *h);
+
+// The same for two handles of one state dimension, in one launch pair on s.
+int estimate_pair(pf_handle *h0, pf_handle *h1, hipStream_t s);
 // ParticleFilter::update (pf2DRao.cpp:125-158) with one measurement column per
 // particle: Z (m x N floats, leading dimension N), uniforms uni[2t], uni[2t+1]
 // for t = the handle's frame counter `parity`; the frame's log mean weight goes
@@ -65,9 +68,6 @@ int step_ref_pair(pf_handle *h0, pf_handle *h1, const float *Z0, const float *Z1
                   const uint32_t *uni1, int parity, double *lml0, double *lml1, bool final_sums = true);
 // The block sums of the handle's last fused estimate and where it goes.
 EstFinalArgs estimate_final_args(pf_handle *h);
-// Reads and clears the handle's status word (kStatus* bits; synchronises
-// the handle's stream).
-int take_status(pf_handle *h, unsigned *word);
 
 }  // namespace eng
 }  // namespace mkfbt

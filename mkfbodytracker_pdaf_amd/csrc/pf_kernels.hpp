@@ -2273,6 +2273,43 @@ __host__ __device__ constexpr int anc_estimate_lds_bytes(int nb, int D)
                                                                         : 8 * (D * 16 * 17 + D * 16 + D);
 }
 
+// The same for two filters of one state dimension (blockIdx.y: which).
+struct EstPairArgs {
+    const float *x[2];
+    const int *anc[2];
+    int N[2];
+    Lay L[2];
+    double *partial[2];
+    const double *Ti[2];
+    double *out[2];
+};
+
+template <int D>
+__global__ void __launch_bounds__(256) k_estimate_pair(EstPairArgs a)
+{
+    __shared__ double s_v[D][16][17];
+    __shared__ double s_run[D][16];
+    __shared__ double s_sum[D];
+    const int k = blockIdx.y, N = k ? a.N[1] : a.N[0];
+    if ((int)blockIdx.x >= (N + 255) / 256) return;
+    const int *anc = k ? a.anc[1] : a.anc[0];
+    double *partial = k ? a.partial[1] : a.partial[0];
+    const int j = blockIdx.x * blockDim.x + threadIdx.x;
+    double v[D];
+    const int s = (j < N) ? (anc ? anc[j] : j) : 0;
+    load_x64<D>(k ? a.x[1] : a.x[0], k ? a.L[1] : a.L[0], s, j < N, v);
+    block_sum256<D>(v, s_v, s_run, s_sum);
+    if (threadIdx.x < D) partial[(size_t)blockIdx.x * D + threadIdx.x] = s_sum[threadIdx.x];
+}
+
+template <int D>
+__global__ void __launch_bounds__(256) k_estimate_final_pair(EstPairArgs a)
+{
+    const int k = blockIdx.x, N = k ? a.N[1] : a.N[0];
+    estimate_final_body<D>(k ? a.partial[1] : a.partial[0], (N + 255) / 256, N, k ? a.Ti[1] : a.Ti[0],
+                           k ? a.out[1] : a.out[0]);
+}
+
 // Both estimate kernels on one stream.
 template <int D>
 inline void launch_estimate(hipStream_t st, const float *x, const int *anc, int N, Lay L, double *partial,

@@ -662,6 +662,23 @@ __global__ void k_tr_end(const TrackerRun *run, const double *lml0, const double
     run->lml[T + t] = lml1[t];
 }
 
+// A host-driven frame: its image and face ROI from pinned host memory (n words
+// of 16 bytes), and after it the arms' status words, read and cleared.
+__global__ void __launch_bounds__(256) k_tr_stage(const uint4 *src, uint4 *dst, int n)
+{
+    const int i = blockIdx.x * blockDim.x + threadIdx.x;
+    if (i < n) dst[i] = src[i];
+}
+
+__global__ void k_tr_status(FrameScratch *fs0, FrameScratch *fs1, unsigned *out)
+{
+    if (threadIdx.x < 2) {
+        FrameScratch *fs = threadIdx.x ? fs1 : fs0;
+        out[threadIdx.x] = fs->status;
+        fs->status = 0u;
+    }
+}
+
 template <typename T>
 hipError_t talloc(T **p, size_t n)
 {
@@ -679,7 +696,6 @@ struct pf_tracker {
     double *hp[2] = {nullptr, nullptr}, *pm[2] = {nullptr, nullptr};
     float *taps = nullptr;
     uint8_t *img_stage = nullptr, *blur = nullptr;
-    int *roi_stage = nullptr;
     double *w[2] = {nullptr, nullptr};
     int *bins[2] = {nullptr, nullptr};
     float *Z[2] = {nullptr, nullptr};
@@ -695,7 +711,12 @@ struct pf_tracker {
     // allocated again (eng::generation)
     hipGraphExec_t groups[4][kTrGroups] = {};
     unsigned long long gen[2] = {0, 0};
-    pf_tracker_outputs stage_out{};     // device outputs of one host-driven frame
+    // pinned host memory: the outputs of one host-driven frame (kernels write
+    // them there) with the arms' status words, and its image and ROI
+    double *host_out = nullptr;
+    unsigned *host_status = nullptr;
+    uint8_t *host_img = nullptr;
+    pf_tracker_outputs stage_out{};     // the places in host_out
     hipEvent_t ev_fork[2] = {nullptr, nullptr}, ev_join[2] = {nullptr, nullptr}, ev_pre = nullptr;
     hipEvent_t ev_t0 = nullptr, ev_t1 = nullptr;
     long long frames_done = 0, uniform_frame = 0;
@@ -945,44 +966,35 @@ int frame_group(pf_tracker *tr, int g, hipGraphExec_t *out)
 }
 
 // Estimates of both arms' current tracks, stream 1 joined into stream 0.
+// (arms of one state dimension: on stream 0, after what stream 1 holds)
 int prepare_estimates(pf_tracker *tr)
 {
-    for (int a = 0; a < 2; ++a) {
-        int st = eng::estimate(tr->arm[a]);
-        if (st) return st;
-    }
+    const bool pair = tr->D[0] == tr->D[1];
+    int st = PF_OK;
+    for (int a = 0; a < 2 && !st && !pair; ++a) st = eng::estimate(tr->arm[a]);
+    if (st) return st;
     TR_TRY(hipEventRecord(tr->ev_pre, tr->s[1]));
     TR_TRY(hipStreamWaitEvent(tr->s[0], tr->ev_pre, 0));
-    return PF_OK;
+    return pair ? eng::estimate_pair(tr->arm[0], tr->arm[1], tr->s[0]) : PF_OK;
 }
 
-// Copies the staged device outputs of one frame to the host pointers of o
-// (each may be NULL) and waits for both streams.
+// Waits for both streams, then copies the outputs of one frame to the host
+// pointers of o (each may be NULL).
 int copy_stage_out(pf_tracker *tr, const pf_tracker_outputs &o)
 {
     const pf_tracker_outputs &d = tr->stage_out;
-    hipStream_t s = tr->s[0];
-    if (o.lml) TR_TRY(hipMemcpyAsync(o.lml, d.lml, sizeof(double) * 2, hipMemcpyDeviceToHost, s));
-    if (o.pose) TR_TRY(hipMemcpyAsync(o.pose, d.pose, sizeof(double) * 2 * tr->npose, hipMemcpyDeviceToHost, s));
-    if (o.pos3d) TR_TRY(hipMemcpyAsync(o.pos3d, d.pos3d, sizeof(double) * 30, hipMemcpyDeviceToHost, s));
-    if (o.tf) TR_TRY(hipMemcpyAsync(o.tf, d.tf, sizeof(double) * 24, hipMemcpyDeviceToHost, s));
-    if (o.pose2d) TR_TRY(hipMemcpyAsync(o.pose2d, d.pose2d, sizeof(double) * 16, hipMemcpyDeviceToHost, s));
     TR_TRY(hipStreamSynchronize(tr->s[0]));
     TR_TRY(hipStreamSynchronize(tr->s[1]));
+    if (o.lml) std::memcpy(o.lml, d.lml, sizeof(double) * 2);
+    if (o.pose) std::memcpy(o.pose, d.pose, sizeof(double) * 2 * tr->npose);
+    if (o.pos3d) std::memcpy(o.pos3d, d.pos3d, sizeof(double) * 30);
+    if (o.tf) std::memcpy(o.tf, d.tf, sizeof(double) * 24);
+    if (o.pose2d) std::memcpy(o.pose2d, d.pose2d, sizeof(double) * 16);
     return PF_OK;
 }
 
-int status_of_arms(pf_tracker *tr)
-{
-    unsigned word = 0;
-    for (int a = 0; a < 2; ++a) {
-        unsigned w = 0;
-        int st = eng::take_status(tr->arm[a], &w);
-        if (st) return st;
-        word |= w;
-    }
-    return status_code(word);
-}
+// Bytes of one image in a staging buffer, which the four ROI words follow.
+size_t stage_px(const pf_tracker *tr) { return ((size_t)tr->cfg.rows * tr->cfg.cols + 15) & ~(size_t)15; }
 
 }  // namespace
 
@@ -1024,18 +1036,14 @@ int pf_tracker_destroy(pf_tracker *tr)
     (void)hipFree(tr->taps);
     (void)hipFree(tr->img_stage);
     (void)hipFree(tr->blur);
-    (void)hipFree(tr->roi_stage);
     (void)hipFree(tr->rec);
     (void)hipFree(tr->fctr);
     (void)hipFree(tr->fctr_aux);
     (void)hipFree(tr->uni);
     (void)hipFree(tr->lml);
     (void)hipFree(tr->run);
-    (void)hipFree(tr->stage_out.lml);
-    (void)hipFree(tr->stage_out.pose);
-    (void)hipFree(tr->stage_out.pos3d);
-    (void)hipFree(tr->stage_out.tf);
-    (void)hipFree(tr->stage_out.pose2d);
+    (void)hipHostFree(tr->host_out);
+    (void)hipHostFree(tr->host_img);
     if (tr->ev_pre) (void)hipEventDestroy(tr->ev_pre);
     if (tr->ev_t0) (void)hipEventDestroy(tr->ev_t0);
     if (tr->ev_t1) (void)hipEventDestroy(tr->ev_t1);
@@ -1151,19 +1159,24 @@ int pf_tracker_create(pf_tracker **out, const pf_tracker_config *cfg, pf_handle 
     const size_t px = (size_t)c.rows * c.cols;
     st = hip_ok(talloc(&tr->taps, taps.size()), "hipMalloc");
     if (!st) st = hip_ok(hipMemcpy(tr->taps, taps.data(), sizeof(float) * taps.size(), hipMemcpyHostToDevice), "hipMemcpy");
-    if (!st) st = hip_ok(talloc(&tr->img_stage, px), "hipMalloc");
+    if (!st) st = hip_ok(talloc(&tr->img_stage, stage_px(tr) + 16), "hipMalloc");
     if (!st) st = hip_ok(talloc(&tr->blur, kBlurSlots * px), "hipMalloc");
     if (!st) st = hip_ok(talloc(&tr->run, 1), "hipMalloc");
-    if (!st) st = hip_ok(talloc(&tr->roi_stage, 4), "hipMalloc");
     if (!st) st = hip_ok(talloc(&tr->rec, 1), "hipMalloc");
     if (!st) st = hip_ok(hipMemset(tr->rec, 0, sizeof(FrameRec)), "hipMemset");
     if (!st) st = hip_ok(talloc(&tr->fctr, 1), "hipMalloc");
     if (!st) st = hip_ok(talloc(&tr->fctr_aux, 1), "hipMalloc");
-    if (!st) st = hip_ok(talloc(&tr->stage_out.lml, 2), "hipMalloc");
-    if (!st) st = hip_ok(talloc(&tr->stage_out.pose, (size_t)2 * npose), "hipMalloc");
-    if (!st) st = hip_ok(talloc(&tr->stage_out.pos3d, 30), "hipMalloc");
-    if (!st) st = hip_ok(talloc(&tr->stage_out.tf, 24), "hipMalloc");
-    if (!st) st = hip_ok(talloc(&tr->stage_out.pose2d, 16), "hipMalloc");
+    const size_t outs = 2 + 30 + 24 + 16 + (size_t)2 * npose + 1;
+    if (!st) st = hip_ok(hipHostMalloc((void **)&tr->host_out, sizeof(double) * outs, hipHostMallocDefault), "hipHostMalloc");
+    if (!st) {
+        std::memset(tr->host_out, 0, sizeof(double) * outs);
+        tr->stage_out.lml = tr->host_out;
+        tr->stage_out.pos3d = tr->stage_out.lml + 2;
+        tr->stage_out.tf = tr->stage_out.pos3d + 30;
+        tr->stage_out.pose2d = tr->stage_out.tf + 24;
+        tr->stage_out.pose = tr->stage_out.pose2d + 16;
+        tr->host_status = reinterpret_cast<unsigned *>(tr->stage_out.pose + (size_t)2 * npose);
+    }
     if (!st) st = hip_ok(hipEventCreateWithFlags(&tr->ev_pre, hipEventDisableTiming), "hipEventCreate");
     if (!st) st = hip_ok(hipEventCreate(&tr->ev_t0), "hipEventCreate");
     if (!st) st = hip_ok(hipEventCreate(&tr->ev_t1), "hipEventCreate");
@@ -1297,15 +1310,30 @@ int pf_tracker_frame(pf_tracker *tr, const uint8_t *likelihood, const int32_t *r
     }
     if (!likelihood) return set_error(PF_ERR_ARG, "null image");
     if (roi[2] <= 0 || roi[3] <= 0) return set_error(PF_ERR_ARG, "empty face ROI");
-    const size_t px = (size_t)tr->cfg.rows * tr->cfg.cols;
-    TR_TRY(hipMemcpyAsync(tr->img_stage, likelihood, px, hipMemcpyHostToDevice, tr->s[0]));
-    TR_TRY(hipMemcpyAsync(tr->roi_stage, roi, sizeof(int32_t) * 4, hipMemcpyHostToDevice, tr->s[0]));
-    TR_TRY(hipStreamSynchronize(tr->s[0]));
-    st = pf_tracker_run_dev(tr, 1, tr->img_stage, tr->roi_stage, &tr->stage_out, 1);
+    // Data in and out through pinned memory, one wait (a copy and a wait each
+    // for the image, the ROI, five outputs and the arms' statuses: 262 us a
+    // frame at N = 500 per arm, 134 so).
+    const size_t px = (size_t)tr->cfg.rows * tr->cfg.cols, rp = stage_px(tr);
+    if (!tr->host_img) TR_TRY(hipHostMalloc((void **)&tr->host_img, rp + 16, hipHostMallocDefault));
+    std::memcpy(tr->host_img, likelihood, px);
+    std::memcpy(tr->host_img + rp, roi, sizeof(int32_t) * 4);
+    const int n16 = (int)(rp / 16) + 1;
+    hipLaunchKernelGGL(k_tr_stage, dim3((n16 + 255) / 256), dim3(256), 0, tr->s[0],
+                       reinterpret_cast<const uint4 *>(tr->host_img), reinterpret_cast<uint4 *>(tr->img_stage), n16);
+    st = launch_check("k_tr_stage");
+    if (!st)
+        st = pf_tracker_run_dev(tr, 1, tr->img_stage, reinterpret_cast<const int32_t *>(tr->img_stage + rp),
+                                &tr->stage_out, 1);
+    if (st) {
+        (void)hipStreamSynchronize(tr->s[0]);
+        return st;
+    }
+    hipLaunchKernelGGL(k_tr_status, dim3(1), dim3(64), 0, tr->s[0], eng::scratch(tr->arm[0]),
+                       eng::scratch(tr->arm[1]), tr->host_status);
+    st = launch_check("k_tr_status");
+    if (!st) st = copy_stage_out(tr, o);
     if (st) return st;
-    st = copy_stage_out(tr, o);
-    if (st) return st;
-    return status_of_arms(tr);
+    return status_code(tr->host_status[0] | tr->host_status[1]);
 }
 
 int pf_tracker_get_last(pf_tracker *tr, uint8_t *blurred, double *proposals, double *weights, int32_t *bins,
