@@ -471,6 +471,12 @@ int sync_tables(pf_batch *b)
     HIP_TRYB(hipMemcpy(b->Ts, b->h_T.data(), sizeof(double) * b->h_T.size(), hipMemcpyHostToDevice));
     HIP_TRYB(hipMemcpy(b->Tis, b->h_Ti.data(), sizeof(double) * b->h_Ti.size(), hipMemcpyHostToDevice));
     HIP_TRYB(hipMemcpy(b->seqs, b->h_seqs.data(), sizeof(SeqDesc) * b->S, hipMemcpyHostToDevice));
+    if (b->D == 24) {
+        if (!b->qrows) HIP_TRYB(dallocb(&b->qrows, (size_t)b->S * b->K * kQ24Row));
+        hipLaunchKernelGGL(k_q24_rows, dim3(b->S * b->K), dim3(128), 0, b->stream, (const float *)b->tables,
+                           (int)(b->h_tabs.size() / b->S), image_head_floats(b->K, b->m, 24, b->J), b->K, b->qrows);
+        HIP_TRYB(hipGetLastError());
+    }
     b->tables_stale = false;
     return PF_OK;
 }
@@ -517,6 +523,7 @@ BatchArgs batch_args(pf_batch *b, const int32_t *count, const float *cand, const
     a.J = b->J;
     a.cap = b->cap;
     a.table_floats = b->table_floats;
+    a.qrows = b->qrows;
     a.comp_head = b->comp_head;
     a.stage_floats = b->stage_floats();
     a.base = StepArgs{};
@@ -551,8 +558,9 @@ void launch_step_t(pf_batch *b, const BatchArgs &a, size_t lds)
     hipLaunchKernelGGL((k_batch_step<kBD, SELJ, PPL>), dim3(grid), dim3(b->sch.block), lds, b->stream, a);
 }
 
-int launch_batch_step(pf_batch *b, const BatchArgs &a)
+int launch_batch_step(pf_batch *b, const BatchArgs &args)
 {
+    const BatchArgs &a = args;
     const size_t lds = (size_t)step_lds_bytes(b->stage_floats(), b->nb_max);
     bool all_sel = true;
     for (int s = 0; s < b->S; ++s) all_sel = all_sel && b->sel_ok[s];
@@ -563,7 +571,14 @@ int launch_batch_step(pf_batch *b, const BatchArgs &a)
         // the vector ALU); one 256-particle tile per block
         if (b->sch.block != 256)
             return set_error(PF_ERR_UNSUPPORTED, "the four-lane d = 24 step runs 256-thread tiles");
-        const size_t qlds = lds + 256 * sizeof(int);
+        // LDS: the image without its component rows (the step reads its own
+        // copy, BatchArgs::qrows), detections, resolver workspace, ancestors
+        BatchArgs a = args;
+        a.table_floats = image_head_floats(b->K, b->m, 24, b->J);
+        a.stage_floats = a.table_floats + cand_lds_floats(b->J, b->cap);
+        a.base.table_floats = a.table_floats;      // where the detections are
+        a.base.stage_floats = a.stage_floats;
+        const size_t qlds = step_lds_bytes(a.stage_floats, b->nb_max) + 256 * sizeof(int);
         const int grid = b->all_tiles;
         const bool mf = b->variant == PF_BATCH_MFMA;
         if (selj == 3 && mf)
@@ -722,6 +737,29 @@ int batch_status(pf_batch *b)
     return status_code(word);
 }
 
+// A d = 24 sequence's state as rows: in place, or room for N particles of its
+// own that its records are copied from or to.
+struct SeqRows {
+    float *x = nullptr, *P = nullptr, *own = nullptr;
+    Lay lay{0, 0};
+    int open(pf_batch *b, const SeqDesc &sd, int buf)
+    {
+        if (b->D != 24) return PF_OK;
+        if (b->records()) {
+            HIP_TRYB(dallocb(&own, (size_t)(24 + npacked(24)) * sd.N));
+            x = own;
+            P = own + (size_t)24 * sd.N;
+            lay = Lay{sd.N, 1};
+        } else {
+            x = b->bx[buf] + sd.pofs;
+            P = b->bP[buf] + sd.pofs;
+            lay = Lay{b->ld, 1};
+        }
+        return PF_OK;
+    }
+    ~SeqRows() { (void)hipFree(own); }      // waits for the device
+};
+
 }  // namespace
 
 extern "C" {
@@ -731,8 +769,9 @@ int pf_batch_destroy(pf_batch *b)
     if (!b) return PF_OK;
     (void)hipSetDevice(b->device);
     if (b->stream) (void)hipStreamSynchronize(b->stream);
+    if (b->D == 24) b->bP[0] = b->bP[1] = nullptr;       // parts of bx
     void *ptrs[] = {b->bx[0], b->bx[1], b->bP[0], b->bP[1], b->lw, b->tables, b->mus, b->sigs, b->Tis, b->Ts,
-                    b->bexp, b->bpow, b->partial, b->gbuf, b->anc, b->frame, b->maxkey, b->cloc, b->bsum,
+                    b->bexp, b->bpow, b->partial, b->gbuf, b->qrows, b->anc, b->frame, b->maxkey, b->cloc, b->bsum,
                     b->cloc1, b->bsum1, b->bexp1, b->bpow1, b->status, b->seqs, b->tile_seq, b->tile_j0, b->n_tiles, b->wb_seq, b->wb_b,
                     b->n_wblocks, b->fs, b->rec_comp, b->rec_anc, b->rec_bins, b->ck_x, b->ck_P, b->seg_x[0],
                     b->seg_x[1], b->seg_P[0], b->seg_P[1], b->adj_x[0], b->adj_x[1], b->adj_P[0], b->adj_P[1], b->first, b->tacc, b->gsum,
@@ -799,8 +838,12 @@ int pf_batch_create(pf_batch **out, int32_t S, const int32_t *n_particles, const
     const size_t NP = npacked(d);
     hipError_t e = hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking);
     for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-        e = dallocb(&b->bx[k], (size_t)d * b->ld);
-        if (e == hipSuccess) e = dallocb(&b->bP[k], NP * b->ld);
+        // d = 24: one buffer, for records or for rows (P's after x's)
+        e = dallocb(&b->bx[k], (size_t)(d == 24 ? kQ24Rec : d) * b->ld);
+        if (d == 24)
+            b->bP[k] = b->bx[k] ? b->bx[k] + (size_t)d * b->ld : nullptr;
+        else if (e == hipSuccess)
+            e = dallocb(&b->bP[k], NP * b->ld);
     }
     e = e ? e : dallocb(&b->lw, (size_t)b->ld);
     e = e ? e : dallocb(&b->anc, (size_t)b->ld);
@@ -911,8 +954,13 @@ int pf_batch_reset(pf_batch *b, int32_t s, const int32_t *bins)
     } else {
         HIP_TRYB(hipMemcpyAsync(b->rec_bins + sd.pofs, bins, sizeof(int) * sd.N, hipMemcpyHostToDevice, b->stream));
     }
-    auto reset = b->D == 24 ? launch_reset<24> : launch_reset<kBD>;
-    reset(b->stream, b->rec_bins + sd.pofs, b->mus + (size_t)i * b->K * b->D,
+    if (b->records())
+        hipLaunchKernelGGL(k_q24_reset, q24_words_grid(sd.N), dim3(256), 0, b->stream,
+                           (const int *)(b->rec_bins + sd.pofs), (const float *)(b->mus + (size_t)i * b->K * b->D),
+                           (const float *)(b->sigs + (size_t)i * b->K * npacked(b->D)),
+                           b->bx[0] + (size_t)sd.pofs * kQ24Rec, b->anc + sd.pofs, sd.N);
+    else (b->D == 24 ? launch_reset<24> : launch_reset<kBD>)(
+          b->stream, b->rec_bins + sd.pofs, b->mus + (size_t)i * b->K * b->D,
           b->sigs + (size_t)i * b->K * npacked(b->D), b->bx[0] + sd.pofs, b->bP[0] + sd.pofs, b->anc + sd.pofs, sd.N,
           Lay{b->ld, 1});
     HIP_TRYB(hipGetLastError());
@@ -985,10 +1033,15 @@ int pf_batch_get_tracks(pf_batch *b, int32_t s, double *x, double *P)
         b->gbuf_bytes = sizeof(double) * (nx + np);
     }
     const int buf = sd.T & 1;   // frame f writes buffer (f + 1) & 1; the last frame is T - 1
+    SeqRows rows;
+    if ((st = rows.open(b, sd, buf))) return st;
+    if (b->records())
+        hipLaunchKernelGGL(k_q24_to_rows, q24_words_grid(sd.N), dim3(256), 0, b->stream,
+                           (const float *)(b->bx[buf] + (size_t)sd.pofs * kQ24Rec), rows.x, (size_t)sd.N, sd.N);
     if (d == 24)
         hipLaunchKernelGGL((k_export_rows<24>), dim3((unsigned)(((long long)sd.N * 24 + 255) / 256)), dim3(256), 0,
-                           b->stream, b->bx[buf] + sd.pofs, b->bP[buf] + sd.pofs, b->anc + sd.pofs,
-                           b->Tis + (size_t)i * d * d, b->gbuf, b->gbuf + nx, sd.N, Lay{b->ld, 1});
+                           b->stream, rows.x, rows.P, b->anc + sd.pofs, b->Tis + (size_t)i * d * d, b->gbuf,
+                           b->gbuf + nx, sd.N, rows.lay);
     else
         hipLaunchKernelGGL((k_export<kBD>), dim3((sd.N + 255) / 256), dim3(256), 0, b->stream, b->bx[buf] + sd.pofs,
                            b->bP[buf] + sd.pofs, b->anc + sd.pofs, b->Tis + (size_t)i * d * d, b->gbuf,
@@ -1021,12 +1074,16 @@ int pf_batch_set_tracks(pf_batch *b, int32_t s, const double *x, const double *P
     HIP_TRYB(hipMemcpyAsync(b->gbuf, x, sizeof(double) * nx, hipMemcpyHostToDevice, b->stream));
     HIP_TRYB(hipMemcpyAsync(b->gbuf + nx, P, sizeof(double) * np, hipMemcpyHostToDevice, b->stream));
     // x' = T x, P' = T P T^T into buffer 0 (frame 0 reads it), ancestors = identity
+    SeqRows rows;
+    if ((st = rows.open(b, sd, 0))) return st;
     if (d == 24)
         hipLaunchKernelGGL((k_import_rows<24>), dim3((unsigned)(((long long)sd.N * 24 + 255) / 256)), dim3(256), 0,
                            b->stream, (const double *)b->gbuf, (const double *)(b->gbuf + nx),
-                           (const double *)(b->Ts + (size_t)i * d * d), b->bx[0] + sd.pofs, b->bP[0] + sd.pofs, sd.N,
-                           Lay{b->ld, 1});
-    else
+                           (const double *)(b->Ts + (size_t)i * d * d), rows.x, rows.P, sd.N, rows.lay);
+    if (b->records())
+        hipLaunchKernelGGL(k_q24_from_rows, q24_words_grid(sd.N), dim3(256), 0, b->stream, (const float *)rows.x,
+                           (size_t)sd.N, b->bx[0] + (size_t)sd.pofs * kQ24Rec, sd.N);
+    if (d != 24)
         hipLaunchKernelGGL((k_import<kBD>), dim3((sd.N + 255) / 256), dim3(256), 0, b->stream,
                            (const double *)b->gbuf, (const double *)(b->gbuf + nx),
                            (const double *)(b->Ts + (size_t)i * d * d), b->bx[0] + sd.pofs, b->bP[0] + sd.pofs, sd.N,
@@ -1062,7 +1119,8 @@ int pf_batch_estimate(pf_batch *b, int32_t s, double *xbar)
     const SeqDesc &sd = b->h_seqs[i];
     const int buf = sd.T & 1;
     if (b->D == 24)
-        launch_estimate<24>(b->stream, b->bx[buf] + sd.pofs, b->anc + sd.pofs, sd.N, Lay{b->ld, 1}, b->partial,
+        launch_estimate<24>(b->stream, b->bx[buf] + (size_t)sd.pofs * (b->records() ? kQ24Rec : 1),
+                            b->anc + sd.pofs, sd.N, b->records() ? Lay{1, kQ24Rec} : Lay{b->ld, 1}, b->partial,
                             b->Tis + (size_t)i * b->D * b->D, b->est);
     else
         launch_estimate<kBD>(b->stream, b->bx[buf] + sd.pofs, b->anc + sd.pofs, sd.N, Lay{b->ld, 1}, b->partial,
@@ -1106,6 +1164,27 @@ int pf_batch_set_variant(pf_batch *b, int32_t variant)
         const pf_batch_schedule s256{256, 1, b->sch.blocks_per_cu};
         st = pf_batch_set_schedule(b, &s256);
         if (st) return st;
+    }
+    const bool had = b->records();
+    if (b->D == 24 && had != (variant != PF_BATCH_VALU)) {
+        // the state in the other kernel's layout
+        float *tmp = nullptr;
+        const size_t n = (size_t)kQ24Rec * b->ld;
+        HIP_TRYB(dallocb(&tmp, n));
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < 2 && e == hipSuccess; ++k) {
+            e = hipMemcpyAsync(tmp, b->bx[k], sizeof(float) * n, hipMemcpyDeviceToDevice, b->stream);
+            if (had)
+                hipLaunchKernelGGL(k_q24_to_rows, q24_words_grid(b->ld), dim3(256), 0, b->stream, (const float *)tmp,
+                                   b->bx[k], (size_t)b->ld, b->ld);
+            else
+                hipLaunchKernelGGL(k_q24_from_rows, q24_words_grid(b->ld), dim3(256), 0, b->stream,
+                                   (const float *)tmp, (size_t)b->ld, b->bx[k], b->ld);
+            e = e ? e : hipGetLastError();
+        }
+        e = e ? e : hipStreamSynchronize(b->stream);
+        (void)hipFree(tmp);
+        HIP_TRYB(e);
     }
     b->variant = variant;
     return PF_OK;

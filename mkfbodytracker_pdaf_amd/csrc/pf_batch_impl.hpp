@@ -22,6 +22,8 @@ namespace mkfbt {
 namespace batch {
 
 constexpr int kBD = 12;           // state dimension of the batched engine
+constexpr int kQ24Row = 4 + 32 + 21 * 16;   // floats of a component row of the four-lane step
+constexpr int kQ24Rec = 32 + 21 * 16;       // floats of a particle's state record there
 constexpr int kSeqAlign = 512;    // particle offset alignment (largest tile)
 
 struct SeqDesc {
@@ -51,6 +53,7 @@ struct BatchArgs {
     const int *count;
     const float *cand;
     double *lml;
+    const float *qrows;           // component rows in the four-lane d = 24 step's order (kQ24Row floats each)
     int comp_head;                // >= 0: component rows read from global memory at tables + table_ofs + comp_head
     int *rec_comp;                // optional record: components of frame t at rec_comp[t * ld + column]
     int *rec_anc;                 // optional record: ancestors of frame t's resampling, same layout
@@ -157,10 +160,13 @@ struct pf_batch {
     bool tracks = false;
     pf_batch_schedule sch{256, 1, 2};
     int variant = PF_BATCH_MFMA;   // kernel of the 24-dimensional state
+    // the four-lane kernels' state: a record per particle (bx[k]: kQ24Rec * ld floats)
+    bool records() const { return D == 24 && variant != PF_BATCH_VALU; }
     hipStream_t stream = nullptr;
     float *bx[2] = {nullptr, nullptr}, *bP[2] = {nullptr, nullptr};
     float *lw = nullptr, *tables = nullptr, *mus = nullptr, *sigs = nullptr;
     double *Tis = nullptr, *Ts = nullptr, *bexp = nullptr, *bexp1 = nullptr, *partial = nullptr;
+    float *qrows = nullptr;        // BatchArgs::qrows (d = 24)
     double *est = nullptr;         // pinned host memory, as the next
     int *h_bins = nullptr;         // a sequence's bins on their way to rec_bins
     double *gbuf = nullptr;

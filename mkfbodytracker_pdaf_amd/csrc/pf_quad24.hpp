@@ -59,11 +59,109 @@ __device__ __forceinline__ float qsel(int c, float v0, float v1, float v2, float
     return c == 0 ? v0 : (c == 1 ? v1 : (c == 2 ? v2 : v3));
 }
 
-// Packed row (pk(24, ., .)) of entry (4I + r, 4I + c) of diagonal tile I.
-__device__ __forceinline__ int qdiag_row(int I, int r, int c)
+// Register order of a state record (kQ24Rec floats, 23 runs of 64 bytes): x (24
+// floats, 8 unused), then per tile (I, K) and lane c the column P[4I + r][4K + c],
+// r = 0..3.  A wave's load of one tile touches 16 whole 64-byte runs of 16
+// contiguous records.  As rows over the particles (packed row p of all
+// particles contiguous) the same 1.3 KB were 324 runs of a few bytes in as many
+// pages: one frame of 32 x 31,250 particles took 1,045 us, 674 as records.
+__device__ __forceinline__ void q24_tile(int T, int &I, int &K)
 {
-    const int lo = r < c ? r : c, hi = r < c ? c : r;
-    return pk(24, 4 * I + lo, 4 * I + lo) + (hi - lo);
+    I = (T >= 6) + (T >= 11) + (T >= 15) + (T >= 18) + (T >= 20);
+    K = I + (T - qtile(I, I));
+}
+
+// 16-byte word e of a record (e < kQ24Rec / 4) from a state whose entry x[i] is
+// fx(i) and packed P[p] is fp(p).
+template <typename FX, typename FP>
+__device__ __forceinline__ q4f q24_word(int e, FX fx, FP fp)
+{
+    q4f v = {0.f, 0.f, 0.f, 0.f};
+    if (e < 6) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = fx(4 * e + r);
+    } else if (e >= 8) {
+        const int c = e & 3;
+        int I, K;
+        q24_tile((e - 8) >> 2, I, K);
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = fp(pk(24, 4 * I + r, 4 * K + c));
+    }
+    return v;
+}
+
+// Initial tracks: the record of the particle's component, ancestors = identity.
+__global__ void __launch_bounds__(256) k_q24_reset(const int *bins, const float *mu, const float *sig, float *rec,
+                                                   int *anc, int N)
+{
+    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = (int)(g / (kQ24Rec / 4)), e = (int)(g - (long long)j * (kQ24Rec / 4));
+    if (j >= N) return;
+    const float *m = mu + (size_t)bins[j] * 24, *s = sig + (size_t)bins[j] * npacked(24);
+    reinterpret_cast<q4f *>(rec)[g] = q24_word(e, [&](int i) { return m[i]; }, [&](int p) { return s[p]; });
+    if (e == 0) anc[j] = j;
+}
+
+// Records of N particles from or to rows: x[i] of particle j at rows[i * stride
+// + j], packed P[p] at rows[(24 + p) * stride + j].
+__global__ void __launch_bounds__(256) k_q24_from_rows(const float *rows, size_t stride, float *rec, int N)
+{
+    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = (int)(g / (kQ24Rec / 4)), e = (int)(g - (long long)j * (kQ24Rec / 4));
+    if (j >= N) return;
+    reinterpret_cast<q4f *>(rec)[g] = q24_word(e, [&](int i) { return rows[i * stride + j]; },
+                                               [&](int p) { return rows[(24 + p) * stride + j]; });
+}
+
+__global__ void __launch_bounds__(256) k_q24_to_rows(const float *rec, float *rows, size_t stride, int N)
+{
+    const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
+    const int j = (int)(g / (kQ24Rec / 4)), e = (int)(g - (long long)j * (kQ24Rec / 4));
+    if (j >= N) return;
+    const q4f v = reinterpret_cast<const q4f *>(rec)[g];
+    if (e < 6) {
+#pragma unroll
+        for (int r = 0; r < 4; ++r) rows[(4 * e + r) * stride + j] = v[r];
+    } else if (e >= 8) {
+        const int c = e & 3;
+        int I, K;
+        q24_tile((e - 8) >> 2, I, K);
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+            if (4 * I + r <= 4 * K + c) rows[(24 + pk(24, 4 * I + r, 4 * K + c)) * stride + j] = v[r];
+    }
+}
+
+inline dim3 q24_words_grid(int N) { return dim3((unsigned)(((long long)N * (kQ24Rec / 4) + 255) / 256)); }
+
+// Component row k of a sequence in the step's register order, so that a lane
+// reads it in 24 loads of up to 16 bytes:
+//   {g, g^2, 0, 0}, then per lane c the offsets of x[4K + c] (6 of 8 floats),
+//   then per tile (I, K) and lane c the noise of P[4I + r][4K + c], r = 0..3.
+// src: the packed row {g, g^2, x offsets, packed noise} (2 + 24 + 300 floats).
+// As 92 loads of single floats the 16 rows of a wave cost 1,472 cache accesses a
+// round, here 384.
+__global__ void __launch_bounds__(128) k_q24_rows(const float *tables, int table_stride, int comp, int K, float *qrows)
+{
+    constexpr int CS = 2 + 24 + npacked(24);
+    const int s = blockIdx.x / K, k = blockIdx.x - s * K;
+    const float *src = tables + (size_t)s * table_stride + comp + k * CS;
+    float *dst = qrows + (size_t)blockIdx.x * kQ24Row;
+    for (int e = threadIdx.x; e < kQ24Row; e += blockDim.x) {
+        float v = 0.f;
+        if (e < 2) {
+            v = src[e];
+        } else if (e >= 4 && e < 36) {
+            const int c = (e - 4) >> 3, Kt = (e - 4) & 7;
+            if (Kt < 6) v = src[2 + 4 * Kt + c];
+        } else if (e >= 36) {
+            const int q = (e - 36) >> 4, c = ((e - 36) >> 2) & 3, r = (e - 36) & 3;
+            int I, Kt;
+            q24_tile(q, I, Kt);
+            v = src[2 + 24 + pk(24, 4 * I + r, 4 * Kt + c)];
+        }
+        dst[e] = v;
+    }
 }
 
 // Tile (I, K) += a b^T for every particle of the wave (a, b: the lanes'
@@ -83,20 +181,24 @@ __device__ __forceinline__ q4f qrank1(float a, float b, q4f acc)
 }
 
 // One 256-particle tile per block; each wave takes four rounds of 16
-// particles (round r, wave w: tile particles 64 r + 16 w + q).
+// particles (round r, wave w: tile particles 64 r + 16 w + q).  Bound by memory:
+// 2.9 KB of records a particle and frame, 674 us for 10^6 particles (4.3 TB/s
+// counted without the ancestors that are read once for several children).
+// Before, with the state as rows: 1,045 us in place at two waves per SIMD, 975
+// with the component rows in register order at three, 915 with the lanes
+// permuted so that 16 of them read one row.
 template <int SELJ, bool MFMA>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))) k_batch_step_q24(BatchArgs a)
 {
-    constexpr int D = 24, NP = npacked(24), CS = 2 + D + NP;
+    constexpr int D = 24;
     extern __shared__ float4 sm4[];
     const int t = *a.frame;
     const int ntiles = a.n_tiles[t];
     if ((int)blockIdx.x >= ntiles) return;              // block-uniform: inactive sequences' tiles
     const int tile = xcd_tile(ntiles);
     const bool odd = (t & 1) != 0;
-    const float *xin = odd ? a.buf_x[1] : a.buf_x[0], *Pin = odd ? a.buf_P[1] : a.buf_P[0];
-    float *xout = odd ? a.buf_x[0] : a.buf_x[1], *Pout = odd ? a.buf_P[0] : a.buf_P[1];
-    const unsigned rowb = (unsigned)a.ld * 4u;
+    const float *recin = odd ? a.buf_x[1] : a.buf_x[0];
+    float *recout = odd ? a.buf_x[0] : a.buf_x[1];
     unsigned long long *wsp = reinterpret_cast<unsigned long long *>(reinterpret_cast<float *>(sm4) + a.stage_floats);
     int *s_src = reinterpret_cast<int *>(wsp + resolve_lds_words(a.nb_max));
     const int s = uni_int(a.tile_seq[tile]);
@@ -123,56 +225,37 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
     const float *BHs = sm + 2 * a.K + a.m * D;
     const float *Rs = BHs + a.m;
     const double *J64 = reinterpret_cast<const double *>(sm + image_j64_floats(a.K, a.m, D, a.J));
-    const float *comp_global = seq_comp_global(a, sd);
-    const float *stab = comp_global ? comp_global : sm + image_head_floats(a.K, a.m, D, a.J);
+    const float *qrows = a.qrows + (size_t)s * a.K * kQ24Row;
     const uint32_t U1 = a.uni[(size_t)(sd.tofs + t) * 2];
     int *comp_out = a.rec_comp ? a.rec_comp + (size_t)t * a.ld + sd.pofs : nullptr;
     const int lane = (int)threadIdx.x & 63, w = (int)threadIdx.x >> 6, q = lane >> 2, c = lane & 3;
-    const __amdgpu_buffer_rsrc_t rx = soa_rsrc(xin, rowb * D), rP = soa_rsrc(Pin, rowb * NP);
-    const __amdgpu_buffer_rsrc_t wx = soa_rsrc(xout, rowb * D), wP = soa_rsrc(Pout, rowb * NP);
-    const unsigned crow = (unsigned)c * rowb;
-    // packed rows of the diagonal tiles' entries held by this lane
-    int drow[6][4];
-#pragma unroll
-    for (int I = 0; I < 6; ++I)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) drow[I][r] = qdiag_row(I, r, c);
-
 #pragma unroll 1
     for (int round = 0; round < 4; ++round) {
         const int jl = 64 * round + 16 * w + q;
         const int j = jt0 + jl;
         const bool live = j < sd.N;                        // quad-uniform; dead particles read ancestor 0
-        const unsigned vb = (unsigned)(sd.pofs + s_src[jl]) * 4u;
+        const float *rin = recin + (size_t)(sd.pofs + s_src[jl]) * kQ24Rec;
+        const q4f *tin = reinterpret_cast<const q4f *>(rin + 32) + c;
         float x[6];
         q4f Pt[kQ24Tiles];
 #pragma unroll
-        for (int K = 0; K < 6; ++K) x[K] = soa_ld(rx, vb + crow, rowb * (unsigned)(4 * K));
+        for (int K = 0; K < 6; ++K) x[K] = rin[4 * K + c];
 #pragma unroll
-        for (int I = 0; I < 6; ++I)
-#pragma unroll
-            for (int K = I; K < 6; ++K)
-#pragma unroll
-                for (int r = 0; r < 4; ++r)
-                    Pt[qtile(I, K)][r] = (K > I) ? soa_ld(rP, vb + crow, rowb * (unsigned)pk(24, 4 * I + r, 4 * K))
-                                                 : soa_ld(rP, vb + (unsigned)drow[I][r] * rowb, 0);
+        for (int T = 0; T < kQ24Tiles; ++T) Pt[T] = tin[4 * T];
 
         // component draw (pf2DRao.cpp:128) and predict (KF_model.cpp:11-15)
         const int k = draw_component(keys, a.K, (uint32_t)j, U1);
-        const float *ck = stab + k * CS;
-        const float g = ck[0], g2 = ck[1];
+        const q4f *ck = reinterpret_cast<const q4f *>(qrows + (size_t)k * kQ24Row);
+        const float g = ck[0][0], g2 = ck[0][1];
+        const q4f xo = ck[1 + 2 * c], xo2 = ck[2 + 2 * c];
 #pragma unroll
-        for (int K = 0; K < 6; ++K) x[K] = fmaf(g, x[K], ck[2 + 4 * K + c]);
-        const float *cq = ck + 2 + D;
+        for (int K = 0; K < 6; ++K) x[K] = fmaf(g, x[K], K < 4 ? xo[K & 3] : xo2[K & 3]);
 #pragma unroll
-        for (int I = 0; I < 6; ++I)
+        for (int T = 0; T < kQ24Tiles; ++T) {
+            const q4f qv = ck[9 + 4 * T + c];
 #pragma unroll
-            for (int K = I; K < 6; ++K)
-#pragma unroll
-                for (int r = 0; r < 4; ++r) {
-                    const float qv = (K > I) ? cq[pk(24, 4 * I + r, 4 * K) + c] : cq[drow[I][r]];
-                    Pt[qtile(I, K)][r] = fmaf(g2, Pt[qtile(I, K)][r], qv);
-                }
+            for (int r = 0; r < 4; ++r) Pt[T][r] = fmaf(g2, Pt[T][r], qv[r]);
+        }
 
         float acc = 0.f;
         unsigned pflags = 0;
@@ -344,24 +427,16 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 8))
         }
 
         if (live) {
-            const unsigned vo = (unsigned)(sd.pofs + j) * 4u;
+            float *rout = recout + (size_t)(sd.pofs + j) * kQ24Rec;
+            q4f *tout = reinterpret_cast<q4f *>(rout + 32) + c;
 #pragma unroll
-            for (int K = 0; K < 6; ++K) soa_st_partial(wx, vo + crow, rowb * (unsigned)(4 * K), x[K]);
+            for (int K = 0; K < 6; ++K) rout[4 * K + c] = x[K];
 #pragma unroll
-            for (int I = 0; I < 6; ++I)
-#pragma unroll
-                for (int K = I; K < 6; ++K)
-#pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        if (K > I)
-                            soa_st_partial(wP, vo + crow, rowb * (unsigned)pk(24, 4 * I + r, 4 * K), Pt[qtile(I, K)][r]);
-                        else if (r <= c)
-                            soa_st_partial(wP, vo + (unsigned)drow[I][r] * rowb, 0, Pt[qtile(I, K)][r]);
-                    }
-            if (c == 0) {
-                a.lw[sd.pofs + j] = acc;
-                if (comp_out) comp_out[j] = k;
-            }
+            for (int T = 0; T < kQ24Tiles; ++T) tout[4 * T] = Pt[T];
+        }
+        if (live && c == 0) {
+            a.lw[sd.pofs + j] = acc;
+            if (comp_out) comp_out[j] = k;
         }
         report_flags(live ? pflags : 0u, &a.status[s]);
     }
