@@ -2,10 +2,11 @@
 // gfx950 GPU (C ABI in include/pf_batch.h).
 //
 // Layout: all sequences share one structure-of-arrays state (x[D][ld],
-// P[D(D+1)/2][ld], double buffered), sequence s owning particles
+// P[D(D+1)/2][ld], double buffered; records for the four-lane d = 24 kernels,
+// pf_quad24.hpp), sequence s owning particles
 // [pofs_s, pofs_s + N_s) with pofs_s a multiple of 512.  Sequences are
 // ordered by length (longest first), so at frame t the active sequences are
-// a prefix and so are their tiles and resampler blocks; the persistent
+// a prefix and so are their tiles and resampler blocks; the
 // kernels read the active counts for frame t from device memory, which makes
 // one captured frame pair replayable for the whole run.
 //
@@ -473,6 +474,9 @@ int sync_tables(pf_batch *b)
     HIP_TRYB(hipMemcpy(b->seqs, b->h_seqs.data(), sizeof(SeqDesc) * b->S, hipMemcpyHostToDevice));
     if (b->D == 24) {
         if (!b->qrows) HIP_TRYB(dallocb(&b->qrows, (size_t)b->S * b->K * kQ24Row));
+        if (!b->qcomps) HIP_TRYB(dallocb(&b->qcomps, (size_t)b->S * b->K * kQ24Rec));
+        hipLaunchKernelGGL(k_q24_comps, dim3(b->S * b->K), dim3(128), 0, b->stream, (const float *)b->mus,
+                           (const float *)b->sigs, b->qcomps);
         hipLaunchKernelGGL(k_q24_rows, dim3(b->S * b->K), dim3(128), 0, b->stream, (const float *)b->tables,
                            (int)(b->h_tabs.size() / b->S), image_head_floats(b->K, b->m, 24, b->J), b->K, b->qrows);
         HIP_TRYB(hipGetLastError());
@@ -771,7 +775,7 @@ int pf_batch_destroy(pf_batch *b)
     if (b->stream) (void)hipStreamSynchronize(b->stream);
     if (b->D == 24) b->bP[0] = b->bP[1] = nullptr;       // parts of bx
     void *ptrs[] = {b->bx[0], b->bx[1], b->bP[0], b->bP[1], b->lw, b->tables, b->mus, b->sigs, b->Tis, b->Ts,
-                    b->bexp, b->bpow, b->partial, b->gbuf, b->qrows, b->anc, b->frame, b->maxkey, b->cloc, b->bsum,
+                    b->bexp, b->bpow, b->partial, b->gbuf, b->qrows, b->qcomps, b->anc, b->frame, b->maxkey, b->cloc, b->bsum,
                     b->cloc1, b->bsum1, b->bexp1, b->bpow1, b->status, b->seqs, b->tile_seq, b->tile_j0, b->n_tiles, b->wb_seq, b->wb_b,
                     b->n_wblocks, b->fs, b->rec_comp, b->rec_anc, b->rec_bins, b->ck_x, b->ck_P, b->seg_x[0],
                     b->seg_x[1], b->seg_P[0], b->seg_P[1], b->adj_x[0], b->adj_x[1], b->adj_P[0], b->adj_P[1], b->first, b->tacc, b->gsum,
@@ -956,8 +960,7 @@ int pf_batch_reset(pf_batch *b, int32_t s, const int32_t *bins)
     }
     if (b->records())
         hipLaunchKernelGGL(k_q24_reset, q24_words_grid(sd.N), dim3(256), 0, b->stream,
-                           (const int *)(b->rec_bins + sd.pofs), (const float *)(b->mus + (size_t)i * b->K * b->D),
-                           (const float *)(b->sigs + (size_t)i * b->K * npacked(b->D)),
+                           (const int *)(b->rec_bins + sd.pofs), (const float *)(b->qcomps + (size_t)i * b->K * kQ24Rec),
                            b->bx[0] + (size_t)sd.pofs * kQ24Rec, b->anc + sd.pofs, sd.N);
     else (b->D == 24 ? launch_reset<24> : launch_reset<kBD>)(
           b->stream, b->rec_bins + sd.pofs, b->mus + (size_t)i * b->K * b->D,

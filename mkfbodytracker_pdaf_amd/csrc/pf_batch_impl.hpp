@@ -167,6 +167,7 @@ struct pf_batch {
     float *lw = nullptr, *tables = nullptr, *mus = nullptr, *sigs = nullptr;
     double *Tis = nullptr, *Ts = nullptr, *bexp = nullptr, *bexp1 = nullptr, *partial = nullptr;
     float *qrows = nullptr;        // BatchArgs::qrows (d = 24)
+    float *qcomps = nullptr;       // the components' initial tracks as records (d = 24)
     double *est = nullptr;         // pinned host memory, as the next
     int *h_bins = nullptr;         // a sequence's bins on their way to rec_bins
     double *gbuf = nullptr;

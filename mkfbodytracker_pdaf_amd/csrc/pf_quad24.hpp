@@ -90,15 +90,25 @@ __device__ __forceinline__ q4f q24_word(int e, FX fx, FP fp)
     return v;
 }
 
+// The record of each of n components' initial track (mu, packed sig).
+__global__ void __launch_bounds__(128) k_q24_comps(const float *mu, const float *sig, float *comps)
+{
+    const float *m = mu + (size_t)blockIdx.x * 24, *s = sig + (size_t)blockIdx.x * npacked(24);
+    const int e = threadIdx.x;
+    if (e < kQ24Rec / 4)
+        reinterpret_cast<q4f *>(comps)[(size_t)blockIdx.x * (kQ24Rec / 4) + e] =
+            q24_word(e, [&](int i) { return m[i]; }, [&](int p) { return s[p]; });
+}
+
 // Initial tracks: the record of the particle's component, ancestors = identity.
-__global__ void __launch_bounds__(256) k_q24_reset(const int *bins, const float *mu, const float *sig, float *rec,
-                                                   int *anc, int N)
+// Bound by the stores (46 MB for 31,250 particles): 14.1 us, 19.0 with every record put
+// together from the packed rows.
+__global__ void __launch_bounds__(256) k_q24_reset(const int *bins, const float *comps, float *rec, int *anc, int N)
 {
     const long long g = (long long)blockIdx.x * blockDim.x + threadIdx.x;
     const int j = (int)(g / (kQ24Rec / 4)), e = (int)(g - (long long)j * (kQ24Rec / 4));
     if (j >= N) return;
-    const float *m = mu + (size_t)bins[j] * 24, *s = sig + (size_t)bins[j] * npacked(24);
-    reinterpret_cast<q4f *>(rec)[g] = q24_word(e, [&](int i) { return m[i]; }, [&](int p) { return s[p]; });
+    reinterpret_cast<q4f *>(rec)[g] = reinterpret_cast<const q4f *>(comps)[(size_t)bins[j] * (kQ24Rec / 4) + e];
     if (e == 0) anc[j] = j;
 }
 
