@@ -74,7 +74,7 @@ def main():
                     help="also run a device-to-device copy of this size (PMC calibration)")
     ap.add_argument("--workload", choices=("single", "batched", "adjoint", "scaled", "tracker"), default="single",
                     help="single: one sequence of N particles (the headline line); batched: many ragged "
-                         "sequences in one persistent step per frame, tuned vs default schedule")
+                         "sequences in one step launch per frame, tuned vs default schedule")
     ap.add_argument("--sequences", type=int, default=256, help="batched: number of sequences")
     ap.add_argument("--tune-frames", type=int, default=32, help="batched: frames timed per candidate schedule")
     ap.add_argument("--scaled-variants", type=str, default="valu,quad_valu,mfma",
@@ -258,7 +258,7 @@ def measured_traffic(N, d, K):
 def run_batched(args):
     """Many independent sequences (lengths U{100..2000} frames, particle counts
     log-uniform in [1k, 64k], each with its own seeded GMM) advanced together,
-    one persistent step kernel and one weights kernel per frame, the frame
+    one step kernel per frame (and one weights kernel where the schedule needs it), the frame
     loop replayed from a hipGraph.  Times the whole run with the default
     schedule, autotunes, then times the whole run again with the tuned one."""
     from mkfbodytracker_pdaf_amd import synthetic
