@@ -293,10 +293,9 @@ struct ImportL {
 
 template <int D>
 struct EstimateL {
-    static void run(pf_handle *h)
+    static void run(pf_handle *h, double *host)
     {
-        launch_estimate<D>(h->stream, h->xA, h->anc, h->N, h->lay, h->est_partial, h->Tinv, h->est_out,
-                           (double *)h->mail);
+        launch_estimate<D>(h->stream, h->xA, h->anc, h->N, h->lay, h->est_partial, h->Tinv, h->est_out, host);
     }
 };
 
@@ -546,7 +545,7 @@ void swap_state_buffer(pf_handle *h) { swap_state(h); }
 
 int estimate(pf_handle *h)
 {
-    int st = dispatch_d<EstimateL>(h->D, h);
+    int st = dispatch_d<EstimateL>(h->D, h, (double *)nullptr);
     if (st) return st;
     return check_launch("k_estimate");
 }
@@ -1099,7 +1098,7 @@ int pf_estimate(pf_handle *h, double *xbar)
     if (!xbar) return set_error(PF_ERR_ARG, "null output");
     st = ensure_mail(h, 0);
     if (st) return st;
-    st = dispatch_d<EstimateL>(h->D, h);
+    st = dispatch_d<EstimateL>(h->D, h, reinterpret_cast<double *>(h->mail));
     if (!st) st = check_launch("k_estimate");
     if (st) return st;
     HIP_TRY(hipStreamSynchronize(h->stream));
@@ -1175,7 +1174,7 @@ static int samples_common(pf_handle *h, const double *Hp, const double *M, int n
     if (st) return st;
     if (!h->tracks) return set_error(PF_ERR_STATE, "tracks not initialised");
     if (!Hp || !M || npose < 2 || n <= 0) return set_error(PF_ERR_ARG, "bad sample arguments");
-    return dispatch_d<EstimateL>(h->D, h);
+    return dispatch_d<EstimateL>(h->D, h, (double *)nullptr);
 }
 
 int pf_get_samples(pf_handle *h, const double *Hp, const double *M, int32_t npose, int32_t n,
