@@ -881,18 +881,17 @@ int enqueue_frame(pf_tracker *tr, int parity)
     // otherwise each arm on its own stream, forked here and joined before the pose
     TR_TRY(hipEventRecord(tr->ev_fork[parity], tr->s[0]));
     TR_TRY(hipStreamWaitEvent(tr->s[1], tr->ev_fork[parity], 0));
-    for (int a = 0; a < 2; ++a) {
+    // (also after an error: a capture ends only with its streams joined)
+    for (int a = 0; a < 2 && !st; ++a) {
         pf_handle *h = tr->arm[a];
         hipLaunchKernelGGL(k_prop_select, dim3((tr->N + 255) / 256), dim3(256), sel_lds, tr->s[a], p, a, sa[a],
                            (const FrameRec *)tr->rec, tr->N);
         st = launch_check("k_prop_select");
-        if (st) return st;
-        st = eng::step_ref(h, tr->Z[a], u_arm[a], parity, lml[a], true);
-        if (st) return st;
+        if (!st) st = eng::step_ref(h, tr->Z[a], u_arm[a], parity, lml[a], true);
     }
     TR_TRY(hipEventRecord(tr->ev_join[parity], tr->s[1]));
     TR_TRY(hipStreamWaitEvent(tr->s[0], tr->ev_join[parity], 0));
-    return launch_pose(tr, tr->fctr, nullptr);
+    return st ? st : launch_pose(tr, tr->fctr, nullptr);
 }
 
 // n frames of the run, the first of even index: their blurs, then the frames.
@@ -944,11 +943,14 @@ int frame_group(pf_tracker *tr, int g, hipGraphExec_t *out)
     hipGraphExec_t &ge = tr->groups[2 * eng::state_buffer(tr->arm[0]) + eng::state_buffer(tr->arm[1])][g];
     if (!ge) {
         hipGraph_t graph;
+        const int before[2] = {eng::state_buffer(tr->arm[0]), eng::state_buffer(tr->arm[1])};
         TR_TRY(hipStreamBeginCapture(tr->s[0], hipStreamCaptureModeThreadLocal));
         const int sc = enqueue_group(tr, 1 << g);
         const hipError_t ec = hipStreamEndCapture(tr->s[0], &graph);
-        if (g == 0)
-            for (pf_handle *arm : tr->arm) eng::swap_state_buffer(arm);
+        // an arm swapped its buffers at each step that was enqueued (a group
+        // that fails may have stopped after one arm's)
+        for (int a = 0; a < 2; ++a)
+            if (eng::state_buffer(tr->arm[a]) != before[a]) eng::swap_state_buffer(tr->arm[a]);
         if (sc) {
             if (ec == hipSuccess) (void)hipGraphDestroy(graph);
             return sc;
