@@ -902,12 +902,16 @@ int enqueue_group(pf_tracker *tr, int n)
     return st;
 }
 
+// Waits for the last run's end (ev_t1; a run that fails has waited for its
+// replays itself) and not on the arms' stream: the arms may be gone already.
 void drop_groups(pf_tracker *tr)
 {
+    bool waited = false;
     for (auto &by_state : tr->groups)
         for (hipGraphExec_t &g : by_state)
             if (g) {
-                (void)hipStreamSynchronize(tr->s[0]);    // its last replay is done
+                if (!waited) (void)hipEventSynchronize(tr->ev_t1);
+                waited = true;
                 (void)hipGraphExecDestroy(g);
                 g = nullptr;
             }
@@ -1247,28 +1251,36 @@ int pf_tracker_run_dev(pf_tracker *tr, int32_t T, const uint8_t *likelihood, con
     hipLaunchKernelGGL(k_tr_begin, dim3((T + 63) / 64), dim3(64), 0, tr->s[0], ba);
     st = launch_check("k_tr_begin");
     if (st) return st;
-    for (int f = 0; f < T;) {
-        int g = kTrGroups - 1;
-        while ((1 << g) > T - f) --g;
-        if (flags & 1) {
-            hipGraphExec_t ge;
-            st = frame_group(tr, g, &ge);
-            if (st) return st;
-            TR_TRY(hipGraphLaunch(ge, tr->s[0]));
-            if (g == 0)
-                for (pf_handle *arm : tr->arm) eng::swap_state_buffer(arm);
-        } else {
-            st = enqueue_group(tr, 1 << g);
-            if (st) return st;
+    const auto frames = [&]() -> int {
+        for (int f = 0; f < T;) {
+            int g = kTrGroups - 1;
+            while ((1 << g) > T - f) --g;
+            if (flags & 1) {
+                hipGraphExec_t ge;
+                const int e = frame_group(tr, g, &ge);
+                if (e) return e;
+                TR_TRY(hipGraphLaunch(ge, tr->s[0]));
+                if (g == 0)
+                    for (pf_handle *arm : tr->arm) eng::swap_state_buffer(arm);
+            } else {
+                const int e = enqueue_group(tr, 1 << g);
+                if (e) return e;
+            }
+            f += 1 << g;
         }
-        f += 1 << g;
+        hipLaunchKernelGGL(k_tr_end, dim3((T + 255) / 256), dim3(256), 0, tr->s[0], (const TrackerRun *)tr->run,
+                           (const double *)tr->lml, (const double *)(tr->lml + tr->run_cap));
+        const int e = launch_check("k_tr_end");
+        if (e) return e;
+        TR_TRY(hipEventRecord(tr->ev_t1, tr->s[0]));
+        return PF_OK;
+    };
+    st = frames();
+    if (st) {
+        (void)hipStreamSynchronize(tr->s[0]);
+        return st;
     }
     tr->last_slot = (T - 1) % kBlurSlots;
-    hipLaunchKernelGGL(k_tr_end, dim3((T + 255) / 256), dim3(256), 0, tr->s[0], (const TrackerRun *)tr->run,
-                       (const double *)tr->lml, (const double *)(tr->lml + tr->run_cap));
-    st = launch_check("k_tr_end");
-    if (st) return st;
-    TR_TRY(hipEventRecord(tr->ev_t1, tr->s[0]));
     // arm 2's stream orders its later work after the run (the frames may
     // have advanced arm 2 on stream 0)
     TR_TRY(hipStreamWaitEvent(tr->s[1], tr->ev_t1, 0));

@@ -1,5 +1,6 @@
 """A tracker frame that an arm's kernels refuse: the call reports it and leaves
-both arms' tracks as they were, and the frame captured next runs."""
+both arms' tracks as they were, and the frame captured next runs.  A tracker
+destroyed after its arms."""
 import numpy as np
 import pytest
 
@@ -62,3 +63,17 @@ def test_refused_frame_leaves_tracks(refused):
     tr.close()
     for a in arms + [good]:
         a.close()
+
+
+@pytest.mark.parametrize("d2", [12, 16])     # the arms in paired launches, and on a stream each
+def test_tracker_destroyed_after_its_arms(d2):
+    parts = [_arm(3, 12), _arm(4, d2)]
+    arms = [p[0] for p in parts]
+    tr = PoseTracker(arms[0], arms[1], parts[0][1], parts[0][2], parts[1][1], parts[1][2], seed=2)
+    imgs, rois = synthetic.tracker_sequence(2, seed=8)
+    dev = DeviceArray(imgs), DeviceArray(rois)
+    tr.callback(imgs[0], rois[0])
+    tr.run_dev(2, dev[0].ptr, dev[1].ptr)    # captured frames of both kinds, the last run not waited for
+    for a in arms:
+        a.close()
+    tr.close()
