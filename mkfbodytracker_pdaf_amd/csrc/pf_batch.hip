@@ -565,7 +565,7 @@ void launch_step_t(pf_batch *b, const BatchArgs &a, size_t lds)
 int launch_batch_step(pf_batch *b, const BatchArgs &args)
 {
     const BatchArgs &a = args;
-    const size_t lds = (size_t)step_lds_bytes(b->stage_floats(), b->nb_max);
+    const size_t lds = (size_t)step_lds_bytes(b->step_stage_floats(), b->nb_max);
     bool all_sel = true;
     for (int s = 0; s < b->S; ++s) all_sel = all_sel && b->sel_ok[s];
     const int selj = all_sel ? b->J : 0;
@@ -575,14 +575,13 @@ int launch_batch_step(pf_batch *b, const BatchArgs &args)
         // the vector ALU); one 256-particle tile per block
         if (b->sch.block != 256)
             return set_error(PF_ERR_UNSUPPORTED, "the four-lane d = 24 step runs 256-thread tiles");
-        // LDS: the image without its component rows (the step reads its own
-        // copy, BatchArgs::qrows), detections, resolver workspace, ancestors
+        // LDS: the staged image and detections, resolver workspace, ancestors
         BatchArgs a = args;
-        a.table_floats = image_head_floats(b->K, b->m, 24, b->J);
-        a.stage_floats = a.table_floats + cand_lds_floats(b->J, b->cap);
+        a.table_floats = b->step_table_floats();
+        a.stage_floats = b->step_stage_floats();
         a.base.table_floats = a.table_floats;      // where the detections are
         a.base.stage_floats = a.stage_floats;
-        const size_t qlds = step_lds_bytes(a.stage_floats, b->nb_max) + 256 * sizeof(int);
+        const size_t qlds = lds + 256 * sizeof(int);
         const int grid = b->all_tiles;
         const bool mf = b->variant == PF_BATCH_MFMA;
         if (selj == 3 && mf)
@@ -982,7 +981,7 @@ int pf_batch_run_dev(pf_batch *b, const int32_t *count, const float *cand, const
     if (!count || !cand || !uniforms || !lml) return set_error(PF_ERR_ARG, "null run argument");
     b->tracks = false;                        // a run consumes the initial tracks
     std::fill(b->fresh.begin(), b->fresh.end(), 0);
-    if ((size_t)step_lds_bytes(b->stage_floats(), b->nb_max) > (size_t)kMaxLdsBytes)
+    if ((size_t)step_lds_bytes(b->step_stage_floats(), b->nb_max) > (size_t)kMaxLdsBytes)
         return set_error(PF_ERR_UNSUPPORTED, "model image and resampler workspace exceed the LDS budget");
     hipEvent_t e0, e1;
     HIP_TRYB(hipEventCreate(&e0));

@@ -162,6 +162,11 @@ struct pf_batch {
     int variant = PF_BATCH_MFMA;   // kernel of the 24-dimensional state
     // the four-lane kernels' state: a record per particle (bx[k]: kQ24Rec * ld floats)
     bool records() const { return D == 24 && variant != PF_BATCH_VALU; }
+    // What the current variant's step stages in LDS: the image (the four-lane
+    // kernels without its component rows, which they read in their own order,
+    // BatchArgs::qrows) and the detections.
+    int step_table_floats() const { return records() ? mkfbt::image_head_floats(K, m, 24, J) : table_floats; }
+    int step_stage_floats() const { return step_table_floats() + mkfbt::cand_lds_floats(J, cap); }
     hipStream_t stream = nullptr;
     float *bx[2] = {nullptr, nullptr}, *bP[2] = {nullptr, nullptr};
     float *lw = nullptr, *tables = nullptr, *mus = nullptr, *sigs = nullptr;
