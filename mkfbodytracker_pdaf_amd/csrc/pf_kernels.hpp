@@ -709,7 +709,9 @@ struct Joint {
         return !innovation_ill(s00, s01, s11);
     }
 
-    // x += W^T v ; P -= W^T M W with M = [[m00, m01], [m01, m11]].
+    // x += W^T v ; P -= W^T M W with M = [[m00, m01], [m01, m11]]; the entries'
+    // arithmetic is the same in either order.
+    template <bool ROWWISE = false>
     __device__ static __forceinline__ void apply(float (&x)[D], float (&P)[NP], float (&w0)[D], float (&w1)[D],
                                                  float v0, float v1, float m00, float m01, float m11)
     {
@@ -747,11 +749,34 @@ struct Joint {
             }
             return;
         }
+        if constexpr (ROWWISE) {
+            // M W first, then P by rows: the reference-mode records kernel
+            // without a selection basis (one wave per SIMD, 490 registers) has no
+            // scratch this way; by columns it spilled 41 registers, and N = 1000
+            // took 23.7 us per frame against 16.2, 100,000 50.7 against 35.9.
+            float u0[D], u1[D];
+#pragma unroll
+            for (int c = 0; c < D; ++c) {
+                x[c] = fmaf(w0[c], v0, fmaf(w1[c], v1, x[c]));
+                u0[c] = fmaf(m00, w0[c], m01 * w1[c]);
+                u1[c] = fmaf(m01, w0[c], m11 * w1[c]);
+            }
+#pragma unroll
+            for (int i = 0; i < D; ++i)
+#pragma unroll
+                for (int k = i; k < D; ++k) {
+                    const float p = fmaf(-w0[i], u0[k], P[pk(D, i, k)]);
+                    P[pk(D, i, k)] = fmaf(-w1[i], u1[k], p);
+                }
+            return;
+        }
         // column k of M W is formed when column k of P is updated: two live
         // temporaries instead of 2 D, which lets the row kernels fit three
         // waves per SIMD (165 registers instead of 190 to 230) with no spills.
         // These kernels are bound by memory latency: 150,000 particles 38.6 ->
-        // 32.9 us per frame, 262,144 52.1 -> 47.0, 10^6 200 -> 195.
+        // 32.9 us per frame, 262,144 52.1 -> 47.0, 10^6 200 -> 195.  Candidate
+        // mode without a selection basis gains too (records, N = 1000 47.4 -> 34.2,
+        // 100,000 108 -> 75).
 #pragma unroll
         for (int k = 0; k < D; ++k) {
             x[k] = fmaf(w0[k], v0, fmaf(w1[k], v1, x[k]));
@@ -1413,18 +1438,18 @@ __device__ __forceinline__ float particle_update(const StepArgs &a, int t, int j
             if (ok) {
                 acc += joint_measure<MODE>(a, t, j, b, clutter, cnt, cz, y0, y1, il00, l10, il11, logl, v0,
                                            v1, m00, m01, m11);
-                if constexpr (D <= 16) Joint<D>::apply(x, P, w0, w1, v0, v1, m00, m01, m11);
+                if constexpr (D <= 16) Joint<D>::template apply<MODE == kModeRef>(x, P, w0, w1, v0, v1, m00, m01, m11);
             } else {
                 Whiten64 wh;
                 if (joint_factor64<D, false>(x, P, 0, Hs + (2 * b) * D, Hs + (2 * b + 1) * D, J64 + 5 * b, wh, logl,
                                              w0, w1, flags)) {
                     acc += joint_measure<MODE>(a, t, j, b, clutter, cnt, cz, wh, logl, v0, v1, m00, m01, m11);
-                    if constexpr (D <= 16) Joint<D>::apply(x, P, w0, w1, v0, v1, m00, m01, m11);
+                    if constexpr (D <= 16) Joint<D>::template apply<MODE == kModeRef>(x, P, w0, w1, v0, v1, m00, m01, m11);
                 } else {
                     acc += joint_reject<D>(w0, w1, v0, v1, m00, m01, m11);   // zero weight, no update
                 }
             }
-            if constexpr (D > 16) Joint<D>::apply(x, P, w0, w1, v0, v1, m00, m01, m11);
+            if constexpr (D > 16) Joint<D>::template apply<MODE == kModeRef>(x, P, w0, w1, v0, v1, m00, m01, m11);
         }
     }
     return acc;
