@@ -1224,8 +1224,8 @@ int pf_batch_autotune(pf_batch *b, const int32_t *count, const float *cand, cons
     for (const auto &c : cands) {
         st = pf_batch_set_schedule(b, &c);
         if (st) return st;
-        // one untimed warm-up frame pair, then `frames` timed frames
-        st = run_all(b, count, cand, uniforms, lml, 3, false);
+        // up to three untimed frames, then `frames` timed ones
+        st = run_all(b, count, cand, uniforms, lml, std::min(3, b->Tmax), false);
         if (st) return st;
         HIP_TRYB(hipEventRecord(e0, b->stream));
         st = run_all(b, count, cand, uniforms, lml, frames, false);
