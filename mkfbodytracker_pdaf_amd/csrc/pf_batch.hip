@@ -1213,8 +1213,9 @@ int pf_batch_autotune(pf_batch *b, const int32_t *count, const float *cand, cons
     std::vector<pf_batch_schedule> cands;
     for (int blk : {64, 128, 256})
         for (int ppl : {1, 2})
-            for (int bpc : {1, 2, 3, 4})
-                if (b->D != 24 || (ppl == 1 && (b->variant == PF_BATCH_VALU || blk == 256)))
+            for (int bpc : {1, 2, 3, 4})      // (one particle per lane has a block per tile: timed once)
+                if ((ppl == 2 || bpc == def.blocks_per_cu) &&
+                    (b->D != 24 || (ppl == 1 && (b->variant == PF_BATCH_VALU || blk == 256))))
                     cands.push_back({blk, ppl, bpc});
     hipEvent_t e0, e1;
     HIP_TRYB(hipEventCreate(&e0));
