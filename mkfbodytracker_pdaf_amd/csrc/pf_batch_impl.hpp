@@ -222,7 +222,7 @@ int bcheck(pf_batch *b);
 int build_tiles(pf_batch *b);
 BatchArgs batch_args(pf_batch *b, const int32_t *count, const float *cand, const uint32_t *uni, double *lml,
                      int parity, int fused);
-int launch_batch_step(pf_batch *b, const BatchArgs &a);
+int launch_batch_step(pf_batch *b, const BatchArgs &a, int tiles);
 // Whether the d = 12 step writes its frame's resampler weights itself: its
 // tiles are resampler blocks (256 threads, one particle per lane); else
 // k_batch_weights runs after it.
