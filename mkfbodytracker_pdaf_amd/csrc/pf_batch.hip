@@ -1006,6 +1006,7 @@ int pf_batch_reset(pf_batch *b, int32_t s, const int32_t *bins)
     HIP_TRYB(hipGetLastError());
     HIP_TRYB(hipStreamSynchronize(b->stream));
     b->fresh[s] = 1;
+    b->state = true;
     b->tracks = std::all_of(b->fresh.begin(), b->fresh.end(), [](char c) { return c != 0; });
     return PF_OK;
 }
@@ -1132,6 +1133,7 @@ int pf_batch_set_tracks(pf_batch *b, int32_t s, const double *x, const double *P
     HIP_TRYB(hipGetLastError());
     HIP_TRYB(hipStreamSynchronize(b->stream));
     b->fresh[s] = 1;
+    b->state = true;
     b->tracks = std::all_of(b->fresh.begin(), b->fresh.end(), [](char c) { return c != 0; });
     return PF_OK;
 }
@@ -1200,30 +1202,34 @@ int pf_batch_set_variant(pf_batch *b, int32_t variant)
         return set_error(PF_ERR_ARG, "unknown variant %d", variant);
     if (variant != PF_BATCH_VALU && b->D != 24)
         return set_error(PF_ERR_UNSUPPORTED, "the four-lane variants are the d = 24 state's");
+    // The tracks, if any, in the other kernel's layout: each state buffer is
+    // converted into a free one, which takes its place.
+    const bool had = b->records(), convert = b->D == 24 && b->state && had != (variant != PF_BATCH_VALU);
+    float *room = nullptr;
+    if (convert) HIP_TRYB(dallocb(&room, (size_t)kQ24Rec * b->ld));
     if (variant != PF_BATCH_VALU && b->sch.block != 256) {
         const pf_batch_schedule s256{256, 1, b->sch.blocks_per_cu};
         st = pf_batch_set_schedule(b, &s256);
-        if (st) return st;
-    }
-    const bool had = b->records();
-    if (b->D == 24 && had != (variant != PF_BATCH_VALU)) {
-        // the state in the other kernel's layout
-        float *tmp = nullptr;
-        const size_t n = (size_t)kQ24Rec * b->ld;
-        HIP_TRYB(dallocb(&tmp, n));
-        hipError_t e = hipSuccess;
-        for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-            e = hipMemcpyAsync(tmp, b->bx[k], sizeof(float) * n, hipMemcpyDeviceToDevice, b->stream);
-            if (had)
-                hipLaunchKernelGGL(k_q24_to_rows, q24_words_grid(b->ld), dim3(256), 0, b->stream, (const float *)tmp,
-                                   b->bx[k], (size_t)b->ld, b->ld);
-            else
-                hipLaunchKernelGGL(k_q24_from_rows, q24_words_grid(b->ld), dim3(256), 0, b->stream,
-                                   (const float *)tmp, (size_t)b->ld, b->bx[k], b->ld);
-            e = e ? e : hipGetLastError();
+        if (st) {
+            (void)hipFree(room);
+            return st;
         }
-        e = e ? e : hipStreamSynchronize(b->stream);
-        (void)hipFree(tmp);
+    }
+    if (convert) {
+        float *free_buf = room;
+        hipError_t e = hipSuccess;
+        for (int k = 0; k < 2; ++k) {
+            e = q24_convert(b->bx[k], free_buf, b->ld, had, b->stream);
+            if (e != hipSuccess) break;
+            std::swap(b->bx[k], free_buf);
+        }
+        for (int k = 0; k < 2; ++k) b->bP[k] = b->bx[k] + (size_t)24 * b->ld;
+        if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
+        (void)hipFree(free_buf);
+        if (e != hipSuccess) {      // converted in part: the tracks are lost
+            b->state = b->tracks = false;
+            std::fill(b->fresh.begin(), b->fresh.end(), 0);
+        }
         HIP_TRYB(e);
     }
     b->variant = variant;

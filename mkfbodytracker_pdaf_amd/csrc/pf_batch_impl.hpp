@@ -158,6 +158,7 @@ struct pf_batch {
     int comp_head = -1;            // >= 0: component rows read from global memory (large images)
     int stage_floats() const { return table_floats + mkfbt::cand_lds_floats(J, cap); }
     bool tracks = false;
+    bool state = false;            // some sequence's tracks have been set
     pf_batch_schedule sch{256, 1, 2};
     int variant = PF_BATCH_MFMA;   // kernel of the 24-dimensional state
     // the four-lane kernels' state: a record per particle (bx[k]: kQ24Rec * ld floats)

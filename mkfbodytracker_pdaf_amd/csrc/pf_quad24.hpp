@@ -144,6 +144,25 @@ __global__ void __launch_bounds__(256) k_q24_to_rows(const float *rec, float *ro
 
 inline dim3 q24_words_grid(int N) { return dim3((unsigned)(((long long)N * (kQ24Rec / 4) + 255) / 256)); }
 
+// A state buffer of ld particles from records to rows of ld, or from rows to
+// records, in launches of at most 2^32 threads.
+inline hipError_t q24_convert(const float *src, float *dst, int ld, bool records, hipStream_t st)
+{
+    constexpr int kChunk = 1 << 24;
+    for (int j0 = 0; j0 < ld; j0 += kChunk) {
+        const int n = std::min(kChunk, ld - j0);
+        if (records)
+            hipLaunchKernelGGL(k_q24_to_rows, q24_words_grid(n), dim3(256), 0, st, src + (size_t)j0 * kQ24Rec,
+                               dst + j0, (size_t)ld, n);
+        else
+            hipLaunchKernelGGL(k_q24_from_rows, q24_words_grid(n), dim3(256), 0, st, src + j0, (size_t)ld,
+                               dst + (size_t)j0 * kQ24Rec, n);
+        const hipError_t e = hipGetLastError();
+        if (e != hipSuccess) return e;
+    }
+    return hipSuccess;
+}
+
 // Component row k of a sequence in the step's register order, so that a lane
 // reads it in 24 loads of up to 16 bytes:
 //   {g, g^2, 0, 0}, then per lane c the offsets of x[4K + c] (6 of 8 floats),
