@@ -778,28 +778,17 @@ int batch_status(pf_batch *b)
     return status_code(word);
 }
 
-// A d = 24 sequence's state as rows: in place, or room for N particles of its
-// own that its records are copied from or to.
-struct SeqRows {
-    float *x = nullptr, *P = nullptr, *own = nullptr;
-    Lay lay{0, 0};
-    int open(pf_batch *b, const SeqDesc &sd, int buf)
-    {
-        if (b->D != 24) return PF_OK;
-        if (b->records()) {
-            HIP_TRYB(dallocb(&own, (size_t)(24 + npacked(24)) * sd.N));
-            x = own;
-            P = own + (size_t)24 * sd.N;
-            lay = Lay{sd.N, 1};
-        } else {
-            x = b->bx[buf] + sd.pofs;
-            P = b->bP[buf] + sd.pofs;
-            lay = Lay{b->ld, 1};
-        }
-        return PF_OK;
-    }
-    ~SeqRows() { (void)hipFree(own); }      // waits for the device
-};
+// Room for a sequence's tracks on their way to or from the host.
+int ensure_gbuf(pf_batch *b, size_t bytes)
+{
+    if (bytes <= b->gbuf_bytes) return PF_OK;
+    (void)hipFree(b->gbuf);
+    b->gbuf = nullptr;
+    b->gbuf_bytes = 0;
+    HIP_TRYB(hipMalloc((void **)&b->gbuf, bytes));
+    b->gbuf_bytes = bytes;
+    return PF_OK;
+}
 
 }  // namespace
 
@@ -1067,22 +1056,17 @@ int pf_batch_get_tracks(pf_batch *b, int32_t s, double *x, double *P)
     const int i = b->rank[s], d = b->D;
     const SeqDesc &sd = b->h_seqs[i];
     const size_t nx = (size_t)sd.N * d, np = (size_t)sd.N * d * d;
-    if (b->gbuf_bytes < sizeof(double) * (nx + np)) {
-        (void)hipFree(b->gbuf);
-        b->gbuf = nullptr;
-        HIP_TRYB(hipMalloc((void **)&b->gbuf, sizeof(double) * (nx + np)));
-        b->gbuf_bytes = sizeof(double) * (nx + np);
-    }
+    if ((st = ensure_gbuf(b, sizeof(double) * (nx + np)))) return st;
     const int buf = sd.T & 1;   // frame f writes buffer (f + 1) & 1; the last frame is T - 1
-    SeqRows rows;
-    if ((st = rows.open(b, sd, buf))) return st;
-    if (b->records())
-        hipLaunchKernelGGL(k_q24_to_rows, q24_words_grid(sd.N), dim3(256), 0, b->stream,
-                           (const float *)(b->bx[buf] + (size_t)sd.pofs * kQ24Rec), rows.x, (size_t)sd.N, sd.N);
-    if (d == 24)
-        hipLaunchKernelGGL((k_export_rows<24>), dim3((unsigned)(((long long)sd.N * 24 + 255) / 256)), dim3(256), 0,
-                           b->stream, rows.x, rows.P, b->anc + sd.pofs, b->Tis + (size_t)i * d * d, b->gbuf,
-                           b->gbuf + nx, sd.N, rows.lay);
+    const dim3 by_row((unsigned)(((long long)sd.N * 24 + 255) / 256));      // d = 24
+    if (b->records()) {
+        const float *rec = b->bx[buf] + (size_t)sd.pofs * kQ24Rec;
+        hipLaunchKernelGGL((k_export_rows<24, Q24Entry>), by_row, dim3(256), 0, b->stream, rec, rec,
+                           b->anc + sd.pofs, b->Tis + (size_t)i * d * d, b->gbuf, b->gbuf + nx, sd.N, Lay{1, kQ24Rec});
+    } else if (d == 24)
+        hipLaunchKernelGGL((k_export_rows<24>), by_row, dim3(256), 0, b->stream, b->bx[buf] + sd.pofs,
+                           b->bP[buf] + sd.pofs, b->anc + sd.pofs, b->Tis + (size_t)i * d * d, b->gbuf, b->gbuf + nx,
+                           sd.N, Lay{b->ld, 1});
     else
         hipLaunchKernelGGL((k_export<kBD>), dim3((sd.N + 255) / 256), dim3(256), 0, b->stream, b->bx[buf] + sd.pofs,
                            b->bP[buf] + sd.pofs, b->anc + sd.pofs, b->Tis + (size_t)i * d * d, b->gbuf,
@@ -1105,24 +1089,21 @@ int pf_batch_set_tracks(pf_batch *b, int32_t s, const double *x, const double *P
     const int i = b->rank[s], d = b->D;
     const SeqDesc &sd = b->h_seqs[i];
     const size_t nx = (size_t)sd.N * d, np = (size_t)sd.N * d * d;
-    if (b->gbuf_bytes < sizeof(double) * (nx + np)) {
-        (void)hipFree(b->gbuf);
-        b->gbuf = nullptr;
-        b->gbuf_bytes = 0;
-        HIP_TRYB(hipMalloc((void **)&b->gbuf, sizeof(double) * (nx + np)));
-        b->gbuf_bytes = sizeof(double) * (nx + np);
-    }
+    // (a state in records comes by way of rows of its own, after the tracks)
+    const size_t nr = b->records() ? (size_t)(24 + npacked(24)) * sd.N : 0;
+    if ((st = ensure_gbuf(b, sizeof(double) * (nx + np) + sizeof(float) * nr))) return st;
     HIP_TRYB(hipMemcpyAsync(b->gbuf, x, sizeof(double) * nx, hipMemcpyHostToDevice, b->stream));
     HIP_TRYB(hipMemcpyAsync(b->gbuf + nx, P, sizeof(double) * np, hipMemcpyHostToDevice, b->stream));
     // x' = T x, P' = T P T^T into buffer 0 (frame 0 reads it), ancestors = identity
-    SeqRows rows;
-    if ((st = rows.open(b, sd, 0))) return st;
+    float *rows = b->records() ? reinterpret_cast<float *>(b->gbuf + nx + np) : b->bx[0] + sd.pofs;
+    float *rows_P = b->records() ? rows + (size_t)24 * sd.N : b->bP[0] + sd.pofs;
     if (d == 24)
         hipLaunchKernelGGL((k_import_rows<24>), dim3((unsigned)(((long long)sd.N * 24 + 255) / 256)), dim3(256), 0,
                            b->stream, (const double *)b->gbuf, (const double *)(b->gbuf + nx),
-                           (const double *)(b->Ts + (size_t)i * d * d), rows.x, rows.P, sd.N, rows.lay);
+                           (const double *)(b->Ts + (size_t)i * d * d), rows, rows_P, sd.N,
+                           Lay{b->records() ? sd.N : b->ld, 1});
     if (b->records())
-        hipLaunchKernelGGL(k_q24_from_rows, q24_words_grid(sd.N), dim3(256), 0, b->stream, (const float *)rows.x,
+        hipLaunchKernelGGL(k_q24_from_rows, q24_words_grid(sd.N), dim3(256), 0, b->stream, (const float *)rows,
                            (size_t)sd.N, b->bx[0] + (size_t)sd.pofs * kQ24Rec, sd.N);
     if (d != 24)
         hipLaunchKernelGGL((k_import<kBD>), dim3((sd.N + 255) / 256), dim3(256), 0, b->stream,

@@ -2109,7 +2109,13 @@ __global__ void __launch_bounds__(256) k_import_rows(const double *x, const doub
     }
 }
 
+// Where P[i][q] (i <= q) of particle s is.
 template <int D>
+struct PackedEntry {
+    static __device__ __forceinline__ size_t at(const Lay &L, int i, int q, int s) { return lidx(L, pk(D, i, q), s); }
+};
+
+template <int D, typename Entry = PackedEntry<D>>
 __global__ void __launch_bounds__(256) k_export_rows(const float *xs, const float *Ps, const int *anc,
                                                      const double *Ti, double *x, double *P, int N, Lay L)
 {
@@ -2124,7 +2130,7 @@ __global__ void __launch_bounds__(256) k_export_rows(const float *xs, const floa
     for (int k = 0; k < D; ++k) {
         double a = 0.0;
         for (int l = 0; l < D; ++l)
-            a = fma(Ti[i * D + l], (double)Ps[lidx(L, pk(D, l < k ? l : k, l < k ? k : l), s)], a);
+            a = fma(Ti[i * D + l], (double)Ps[Entry::at(L, l < k ? l : k, l < k ? k : l, s)], a);
         r[k] = a;
     }
     double *Po = P + (size_t)j * D * D;

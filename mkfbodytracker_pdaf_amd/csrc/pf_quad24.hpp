@@ -71,6 +71,15 @@ __device__ __forceinline__ void q24_tile(int T, int &I, int &K)
     K = I + (T - qtile(I, I));
 }
 
+// Where P[i][q] (i <= q) of record s is: exported tracks are read from the
+// records (by way of rows, with their own launch, 18 us more at N = 15: 139 us).
+struct Q24Entry {
+    static __device__ __forceinline__ size_t at(const Lay &, int i, int q, int s)
+    {
+        return (size_t)s * kQ24Rec + 32 + 16 * qtile(i >> 2, q >> 2) + 4 * (q & 3) + (i & 3);
+    }
+};
+
 // 16-byte word e of a record (e < kQ24Rec / 4) from a state whose entry x[i] is
 // fx(i) and packed P[p] is fp(p).
 template <typename FX, typename FP>

@@ -1,7 +1,8 @@
 """Changing the d = 24 batch's kernel: before any tracks it only selects the
 kernel (no conversion, the schedule's tile size included), afterwards the tracks
 move to the other layout bit for bit, from either state buffer (a recording of
-odd length ends in the second), and a change and back changes nothing."""
+odd length ends in the second), and a change and back changes nothing.  Imported
+tracks are the same bits in both layouts."""
 import numpy as np
 import pytest
 
@@ -62,4 +63,24 @@ def test_change_of_kernel(variant):
     b.run_dev(*(d.ptr for d in dev), lml.ptr)
     assert np.array_equal(lml.get(), want_lml)
     assert all(np.array_equal(p, q) for p, q in zip(_state(b), want))
+    b.close()
+
+
+@pytest.mark.parametrize("variant", [QUAD, MFMA])
+def test_imported_tracks(variant):
+    """The import's FP64 products and FP32 rounding do not depend on the
+    layout, nor does the export of what it stored (sequences of even length:
+    the initial tracks' buffer is the one read)."""
+    b, models, bins, _ = _batch()
+    _load(b, models)
+    even = [s for s in range(len(NS)) if TS[s] % 2 == 0]
+    got = []
+    for v in (ROWS, variant):
+        b.variant = v
+        for s in range(len(NS)):
+            a = np.random.default_rng(s).standard_normal((NS[s], 24, 24))
+            b.set_tracks(s, np.random.default_rng(9 + s).standard_normal((NS[s], 24)),
+                         a @ a.transpose(0, 2, 1) + np.eye(24))
+        got.append([q for s in even for q in b.get_tracks(s) + (b.estimate(s),)])
+    assert even and all(np.array_equal(p, q) for p, q in zip(*got))
     b.close()
