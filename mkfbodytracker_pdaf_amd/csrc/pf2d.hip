@@ -443,12 +443,9 @@ int pf2d_get_particles(pf2d_handle *h, double *particles, double *weights)
     return PF_OK;
 }
 
-int pf2d_update(pf2d_handle *h, const double *meas, uint32_t u, const double *normals, const double *reinit_unif,
-                float *lw, int32_t *anc)
+static int update_frame(pf2d_handle *h, const double *meas, uint32_t u, const double *normals,
+                        const double *reinit_unif, float *lw, int32_t *anc)
 {
-    if (!h || !meas || !normals || !reinit_unif) return set_error(PF_ERR_ARG, "null argument");
-    if (!h->gmm) return set_error(PF_ERR_STATE, "load the GMM first");
-    HIP_TRY2(hipSetDevice(h->device));
     const int N = h->N, nb = (N + kWeightsBlock - 1) / kWeightsBlock;
     const size_t steps = sizeof(float) * (size_t)N * kD;
     const bool mail = steps + 8 * (size_t)N <= kUpdateMail;
@@ -550,6 +547,18 @@ int pf2d_update(pf2d_handle *h, const double *meas, uint32_t u, const double *no
     if (!mail && anc) HIP_TRY2(hipMemcpyAsync(anc, h->anc, sizeof(int) * N, hipMemcpyDeviceToHost, h->stream));
     if (degenerate || !mail) HIP_TRY2(hipStreamSynchronize(h->stream));
     return degenerate ? PF_WARN_DEGENERATE : PF_OK;
+}
+
+int pf2d_update(pf2d_handle *h, const double *meas, uint32_t u, const double *normals, const double *reinit_unif,
+                float *lw, int32_t *anc)
+{
+    if (!h || !meas || !normals || !reinit_unif) return set_error(PF_ERR_ARG, "null argument");
+    if (!h->gmm) return set_error(PF_ERR_STATE, "load the GMM first");
+    HIP_TRY2(hipSetDevice(h->device));
+    const int st = update_frame(h, meas, u, normals, reinit_unif, lw, anc);
+    // nothing enqueued uses the pinned buffer or the caller's arrays after an error
+    if (st < 0) (void)hipStreamSynchronize(h->stream);
+    return st;
 }
 
 int pf2d_predict(pf2d_handle *h, const double *normals)

@@ -454,11 +454,12 @@ int build_batch_tables(pf_batch *b)
     return PF_OK;
 }
 
-// The device copies of the images brought up to date (the batch's stream is
-// idle: every call that enqueues on it waits for it).
+// The device copies of the images brought up to date (calls that enqueue on
+// the batch's stream wait for it, but not all do so with an error).
 int sync_tables(pf_batch *b)
 {
     if (!b->tables_stale) return PF_OK;
+    HIP_TRYB(hipStreamSynchronize(b->stream));
     if (!b->Tis) {
         HIP_TRYB(dallocb(&b->tables, b->h_tabs.size()));
         HIP_TRYB(dallocb(&b->mus, b->h_mus.size()));
@@ -992,8 +993,9 @@ int pf_batch_reset(pf_batch *b, int32_t s, const int32_t *bins)
           b->stream, b->rec_bins + sd.pofs, b->mus + (size_t)i * b->K * b->D,
           b->sigs + (size_t)i * b->K * npacked(b->D), b->bx[0] + sd.pofs, b->bP[0] + sd.pofs, b->anc + sd.pofs, sd.N,
           Lay{b->ld, 1});
-    HIP_TRYB(hipGetLastError());
-    HIP_TRYB(hipStreamSynchronize(b->stream));
+    const hipError_t e = hipGetLastError();
+    HIP_TRYB(hipStreamSynchronize(b->stream));      // (also after an error: h_bins is free)
+    HIP_TRYB(e);
     b->fresh[s] = 1;
     b->state = true;
     b->tracks = std::all_of(b->fresh.begin(), b->fresh.end(), [](char c) { return c != 0; });
@@ -1148,8 +1150,9 @@ int pf_batch_estimate(pf_batch *b, int32_t s, double *xbar)
     else
         launch_estimate<kBD>(b->stream, b->bx[buf] + sd.pofs, b->anc + sd.pofs, sd.N, Lay{b->ld, 1}, b->partial,
                              b->Tis + (size_t)i * b->D * b->D, b->est);
-    HIP_TRYB(hipGetLastError());
-    HIP_TRYB(hipStreamSynchronize(b->stream));
+    const hipError_t e = hipGetLastError();
+    HIP_TRYB(hipStreamSynchronize(b->stream));      // (also after an error: est is free)
+    HIP_TRYB(e);
     std::memcpy(xbar, b->est, sizeof(double) * b->D);
     return PF_OK;
 }

@@ -213,8 +213,16 @@ int ensure_ibuf(pf_handle *h, size_t bytes)
 
 constexpr size_t kMailHead = 64 * sizeof(double);   // the estimate's place
 
-// At least `bytes` of the pinned buffer after its head (the stream is idle:
-// every call that uses the buffer waits before it returns).
+// A call that uses the pinned buffer, or host memory of its own, waits before
+// it returns, also with an error (st < 0) after something was enqueued.
+int waited(pf_handle *h, int st)
+{
+    if (st < 0) (void)hipStreamSynchronize(h->stream);
+    return st;
+}
+
+// At least `bytes` of the pinned buffer after its head, which no kernel uses
+// (waited).
 int ensure_mail(pf_handle *h, size_t bytes)
 {
     if (kMailHead + bytes <= h->mail_bytes) return PF_OK;
@@ -894,7 +902,7 @@ int pf_reset(pf_handle *h, const int32_t *bins)
     }
     st = dispatch_d<ResetL>(h->D, h);
     if (!st) st = check_launch("k_reset");
-    if (st) return st;
+    if (st) return waited(h, st);
     HIP_TRY(hipStreamSynchronize(h->stream));
     h->tracks = true;
     return PF_OK;
@@ -1058,11 +1066,11 @@ int pf_step(pf_handle *h, const double *Z, uint32_t u_comp, uint32_t u_res, floa
     st = in.open(h, L, words);
     if (st) return st;
     for (size_t i = 0; i < words; ++i) in.p[i] = (float)Z[i];
-    st = mail_in(h, L, in, h->zbuf, words, u_comp, u_res);
-    if (st) return st;
     StepArgs a = step_args(h, kModeRef, h->uni, h->zbuf, 0, N, nullptr, nullptr, comp ? h->comp : nullptr, 0,
                            kAncArray, nullptr);
-    return host_step(h, a, kModeRef, L, lw, anc, comp, lml);
+    st = mail_in(h, L, in, h->zbuf, words, u_comp, u_res);
+    if (!st) st = host_step(h, a, kModeRef, L, lw, anc, comp, lml);
+    return waited(h, st);
 }
 
 int pf_step_candidates(pf_handle *h, const int32_t *count, const double *cand, uint32_t u_comp,
@@ -1083,11 +1091,11 @@ int pf_step_candidates(pf_handle *h, const int32_t *count, const double *cand, u
     if (st) return st;
     for (size_t i = 0; i < nc; ++i) in.p[i] = (float)cand[i];
     std::memcpy(in.p + nc, count, sizeof(int) * J);
-    st = mail_in(h, L, in, h->candbuf, words, u_comp, u_res);
-    if (st) return st;
     StepArgs a = step_args(h, kModeCand, h->uni, nullptr, 0, 0, reinterpret_cast<const int *>(h->candbuf + nc),
                            h->candbuf, comp ? h->comp : nullptr, 0, kAncArray, nullptr);
-    return host_step(h, a, kModeCand, L, lw, anc, comp, lml);
+    st = mail_in(h, L, in, h->candbuf, words, u_comp, u_res);
+    if (!st) st = host_step(h, a, kModeCand, L, lw, anc, comp, lml);
+    return waited(h, st);
 }
 
 int pf_estimate(pf_handle *h, double *xbar)
@@ -1100,7 +1108,7 @@ int pf_estimate(pf_handle *h, double *xbar)
     if (st) return st;
     st = dispatch_d<EstimateL>(h->D, h, reinterpret_cast<double *>(h->mail));
     if (!st) st = check_launch("k_estimate");
-    if (st) return st;
+    if (st) return waited(h, st);
     HIP_TRY(hipStreamSynchronize(h->stream));
     std::memcpy(xbar, h->mail, sizeof(double) * h->D);
     return PF_OK;
