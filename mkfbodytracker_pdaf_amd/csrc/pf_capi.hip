@@ -351,10 +351,20 @@ int launch_weights(pf_handle *h, const uint32_t *uni, int parity)
     return check_launch("k_weights");
 }
 
-// Above this many input blocks (262,144 weights) the ancestors take their
-// prefix from k_prefix: two launches, against one whose every block repeats it
-// (14 us per call at 391 input blocks, where k_ancestors takes 7).
+// Above this many input blocks (262,144 weights) a frame's ancestors take their
+// prefix from k_prefix: two launches, against one whose every block repeats it.
+// Kernels, one launch / two with the gap between them: 391 blocks (100,000) 7 us /
+// 14, 1172 (300,000) 11.9 / 11, 1758 (450,000) 18.6 / 12.0, 3907 (10^6) 139 / 19.3.
+// A run's frames, one / two: 440,000 105.5 us / 99.8, 524,288 135 / 117, 700,000
+// 181 / 148.
 constexpr int kPrefixBlocks = 1024;
+// A resampling of the caller's weights (pf_resample*) stands alone: the second
+// launch costs it 20 us of wall time, which it repays where this many input
+// blocks, counted once per block of 256 outputs, are saved.  Whole calls, one
+// launch / two: 300,000 -> 1,000 151 us / 174, 450,000 -> 450,000 297 / 317,
+// 524,288 -> 524,288 (4.2e6) 353 / 357, 650,000 -> 650,000 (6.4e6) 410 / 409,
+// 800,000 -> 800,000 520 / 494, 10^6 -> 100,000 (1.5e6) 334 / 350.
+constexpr long long kPrefixPairs = 5LL << 20;
 
 // Materialise the pending resampling of L weights into N ancestors.  The log
 // mean weight goes to lml, or to lml[*lml_frame] when a frame counter is given.
@@ -371,7 +381,9 @@ int launch_ancestors(pf_handle *h, int L, int N, int *out, int parity, int kind_
     an.N = N;
     an.parity = parity;
     an.kind_linear = kind_linear;
-    if (an.pend.nb > kPrefixBlocks) {
+    const bool frame = lml != nullptr;
+    const long long pairs = (long long)an.pend.nb * ((N + 255) / 256);
+    if (an.pend.nb > kPrefixBlocks && (frame || pairs > kPrefixPairs)) {
         hipLaunchKernelGGL(k_prefix, dim3(1), dim3(kPrefixThreads), 0, h->stream, an, h->gpre, h->gshf);
         hipLaunchKernelGGL(k_ancestors_prefixed, dim3((N + 255) / 256), dim3(256), 0, h->stream, an,
                            (const unsigned long long *)h->gpre, (const int *)h->gshf);

@@ -1,5 +1,6 @@
 """Resampling with more than 1024 input blocks of 256 weights, where the
-prefix of the block sums is taken once in its own kernel, and, with more than
+prefix of the block sums is taken once in its own kernel (of the caller's weights,
+with 5 x 2^20 pairs of input and output blocks), and, with more than
 1700, the frames of a
 device-resident run are step, prefix and ancestor launches: indices bit-exact
 against the oracle, and a run equal to host-driven steps bit for bit, on both
@@ -41,6 +42,21 @@ def test_indices_bit_exact(L, kind):
         want, wst = oracle.resample_linear(w, N, u)
         assert st == wst
         assert np.array_equal(got, want)
+    rb.close()
+
+
+@pytest.mark.parametrize("L,blocks", [(1 << 20, 1280), (EDGE + 1, 5115), (600000, 2236)])
+def test_callers_weights_both_routes(L, blocks):
+    """On both sides of the product of input blocks and blocks of 256 outputs at
+    which the prefix gets its own kernel (EDGE + 1 weights are 1025 blocks)."""
+    nb = (L + 255) // 256
+    assert nb * blocks <= 5 << 20 < nb * (blocks + 1)
+    lw = np.random.default_rng(L).normal(0.0, 2.0, L)
+    rb = Rbpf(64)
+    for N in (256 * blocks, 256 * blocks + 1):
+        got, st = rb.resample(lw, N, 0x9E3779B9, log=True)
+        want, wst = oracle.resample_log(lw, N, 0x9E3779B9)
+        assert st == wst == 0 and np.array_equal(got, want)
     rb.close()
 
 
