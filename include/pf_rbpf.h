@@ -159,11 +159,10 @@ int pf_get_sample_prob(pf_handle *h, const double *Hp, const double *M, int32_t 
  * the handle's first such run (the frames read the run's pointers from
  * device memory, so the graphs serve every later run of any length; they
  * are captured again after pf_load_model or pf_set_joint_clutter; runs of
- * more than 435,200 particles, whose frames are three longer launches each, are
- * launched without graphs); bits 1
- * and 2 time the run (see
- * pf_last_run_kernel_time; bit 1 turns the graphs off).  Returns after
- * enqueueing; pf_synchronize waits. */
+ * more than 435,200 particles (465,920 at d = 16), whose frames are three
+ * longer launches each, are launched without graphs); bits 1 and 2 time the
+ * run (see pf_last_run_kernel_time; bit 1 turns the graphs off).  Returns
+ * after enqueueing; pf_synchronize waits. */
 int pf_run_ref_dev(pf_handle *h, int32_t T, const float *Z, const uint32_t *uniforms,
                    double *lml, int32_t use_graph);
 int pf_run_candidates_dev(pf_handle *h, int32_t T, const int32_t *count, const float *cand,

@@ -1314,12 +1314,17 @@ int ensure_events(pf_handle *h, size_t need)
 }
 
 // Up to this many input blocks a frame is one launch that resolves its own
-// ancestors; above, every block's prefix and the search's latency (and the
-// resolver's LDS, which leaves two blocks per CU) cost more than two more
-// launches.  Per frame (d = 12, 8 detections per hand), one launch against
-// step, k_prefix and k_ancestors_prefixed: N = 300k 52.4 / 58.1 us, 350k 62.2 /
-// 69.4, 400k 91.3 / 92.3, 450k 98.1 / 98.0, 524k 129 / 118, 650k 151 / 131.
-constexpr int kFusedBlocks = 1700;
+// ancestors; above, every block's prefix and the search's latency cost more than
+// two more launches, and from 1,850 blocks or so the resolver's LDS leaves two
+// blocks per CU instead of three.  d = 16 holds two by its registers, so its line
+// lies higher.  Per frame (8 detections per hand), one launch / step, k_prefix and
+// k_ancestors_prefixed:
+//   N =       400,000        440,000        450,000        465,000        480,000      524,288
+//   d = 8   52.5 / 52.4    55.8 / 55.6    56.8 / 55.5    62.1 / 56.5    63.7 / 57.5   69 / 62
+//   d = 12  92.8 / 92.2    98.9 / 100     104 / 105      118 / 114      123 / 110     136 / 120
+//   d = 16   153 / 153      162 / 167     166 / 170      176 / 176      175 / 174     189 / 184
+//   d = 24                                568 / 561                     597 / 583 (473,000)
+inline int fused_blocks(int D) { return D == 16 ? 1820 : 1700; }
 
 // Frames of many input blocks, or whose model image and resolver workspace do
 // not fit one workgroup's LDS: step and ancestor launches per frame, launched
@@ -1379,7 +1384,7 @@ static int run_frames(pf_handle *h, int T, int mode, const float *Z, const int *
     // (records: as much LDS as leaves the blocks that share a CU their place)
     const bool rec = h->lay.row == 1;
     const int lds_limit = !rec ? kMaxLdsBytes : (nbp <= h->cus ? kCuLdsBytes : kCuLdsBytes / 2);
-    const bool fused = nbp <= kFusedBlocks && step_lds_bytes_rec(rec, stage, nbp) <= lds_limit;
+    const bool fused = nbp <= fused_blocks(h->D) && step_lds_bytes_rec(rec, stage, nbp) <= lds_limit;
     if (!fused) {
         st = run_frames_split(h, T, mode, Z, count, cand, uniforms, lml, timing, run_timing);
     } else {

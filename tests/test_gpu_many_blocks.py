@@ -1,7 +1,7 @@
 """Resampling with more than 1024 input blocks of 256 weights, where the
 prefix of the block sums is taken once in its own kernel (of the caller's weights,
 with 5 x 2^20 pairs of input and output blocks), and, with more than
-1700, the frames of a
+1700 (1820 at d = 16), the frames of a
 device-resident run are step, prefix and ancestor launches: indices bit-exact
 against the oracle, and a run equal to host-driven steps bit for bit, on both
 sides of both boundaries and at the largest size."""
@@ -17,6 +17,7 @@ pytestmark = pytest.mark.gpu
 
 EDGE = 262144      # k_prefix above
 SPLIT = 435200     # separate launches above
+SPLIT16 = 465920   # the same at d = 16
 
 
 @pytest.mark.parametrize("L", [EDGE, EDGE + 1, 300007, 1 << 20])
@@ -60,10 +61,11 @@ def test_callers_weights_both_routes(L, blocks):
     rb.close()
 
 
-@pytest.mark.parametrize("N", [EDGE, EDGE + 1, SPLIT, SPLIT + 1])
-def test_run_equals_host_steps(N):
+@pytest.mark.parametrize("N,d", [(EDGE, 12), (EDGE + 1, 12), (SPLIT, 12), (SPLIT + 1, 12), (SPLIT + 1, 16),
+                                 (SPLIT16, 16), (SPLIT16 + 1, 16)])
+def test_run_equals_host_steps(N, d):
     T, cap = 3, 8
-    mdl = synthetic.make_model(seed=5)
+    mdl = synthetic.make_model(seed=5, d=d)
     seq = synthetic.simulate(mdl, T, seed=6, cand_per_joint=4, cap=cap)
     bins = oracle.resample_linear(mdl.weights, N, 7)[0]
     d_cnt, d_cand = DeviceArray(seq.count.astype(np.int32)), DeviceArray(seq.cand.astype(np.float32))
@@ -79,6 +81,7 @@ def test_run_equals_host_steps(N):
         rb.reset(bins)
         rb.run_candidates_dev(T, d_cnt.ptr, d_cand.ptr, d_uni.ptr, d_lml.ptr, flags)
         assert rb.synchronize() == 0
+        assert rb.last_graph_frames() == (T if flags and N <= (SPLIT16 if d == 16 else SPLIT) else 0)
         assert np.array_equal(d_lml.get(), np.array(want))
         assert np.array_equal(rb.estimate(), est)
     rb.close()
