@@ -895,6 +895,7 @@ int pf_batch_create(pf_batch **out, int32_t S, const int32_t *n_particles, const
     e = e ? e : hipHostMalloc((void **)&b->est, 64 * sizeof(double), hipHostMallocDefault);
     e = e ? e : hipHostMalloc((void **)&b->h_bins, std::min(sizeof(int) * (size_t)b->ld, kMailMax), hipHostMallocDefault);
     e = e ? e : dallocb(&b->fs, 1);
+    if (e == hipSuccess) e = hipMemset(b->anc, 0, sizeof(int) * (size_t)b->ld);   // valid before the first reset
     if (e == hipSuccess) e = hipMemset(b->maxkey, 0, sizeof(unsigned long long) * 2 * S);
     if (e == hipSuccess) e = hipMemset(b->status, 0, sizeof(unsigned) * S);
     if (e == hipSuccess) e = hipMemset(b->fs, 0, sizeof(FrameScratch));
