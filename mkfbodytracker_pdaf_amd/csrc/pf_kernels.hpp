@@ -148,7 +148,6 @@ struct Pending {
     const unsigned long long *__restrict__ bsum;
     const double *__restrict__ bexp;
     const int *__restrict__ bpow = nullptr;      // block exponents of block-scaled log-weights (null: none)
-    const int *pow_max = nullptr;                // their maximum, when its producer recorded it (else reduced)
     int L, nb;
     int bshift = 8;                              // log2 of the inputs per block (kWeightsBlock)
     int stage = kStageBlocks * kWeightsBlock;    // LDS elements of the staged search
@@ -439,15 +438,13 @@ __device__ __forceinline__ unsigned long long resolve_prefix_from(const Pending 
     return total;
 }
 
-template <typename Hook = NoHook>
 __device__ __forceinline__ unsigned long long resolve_prefix(const Pending &pd, unsigned long long *w, bool want_es,
-                                                             double &es_out, int &pow_out, Hook hook = Hook())
+                                                             double &es_out, int &pow_out)
 {
     const int per = prefix_per(pd);
     PrefixRegs r;
     prefix_load(pd, per, 0, r);
-    const bool have = pd.bpow && pd.pow_max;
-    return resolve_prefix_from(pd, w, per, r, have, have ? gload(pd.pow_max) : 0, want_es, es_out, pow_out, hook);
+    return resolve_prefix_from(pd, w, per, r, false, 0, want_es, es_out, pow_out);
 }
 
 // Phase 2: a_j for outputs j in [j0, j0 + blockDim) (j = j0 + threadIdx.x),
@@ -862,19 +859,11 @@ __device__ __forceinline__ float soa_ld(__amdgpu_buffer_rsrc_t r, unsigned voff,
 // on every XCD, and each store instruction writes whole 128-byte lines (64
 // consecutive particles of one row).  Measured at N = 100k, d = 12: 33.1 ->
 // 31.9 us per frame against default-scope stores, same results bit for bit.
-// Stores that write partial lines (the four-lane d = 24 kernels: 16
-// particles per instruction) keep the default policy (soa_st_partial): with
-// device scope they were 5% slower.
 constexpr int kStoreDeviceScope = 16;   // CPol::SC1
 
 __device__ __forceinline__ void soa_st(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, float v)
 {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, (int)voff, (int)soff, kStoreDeviceScope);
-}
-
-__device__ __forceinline__ void soa_st_partial(__amdgpu_buffer_rsrc_t r, unsigned voff, unsigned soff, float v)
-{
-    __builtin_amdgcn_raw_buffer_store_b32(__float_as_int(v), r, (int)voff, (int)soff, 0);
 }
 
 // Layout of a particle state buffer: element r of particle j of x (r < D)
@@ -885,7 +874,8 @@ __device__ __forceinline__ void soa_st_partial(__amdgpu_buffer_rsrc_t r, unsigne
 // particle's record is ~3 cache lines (d = 12) wherever its ancestor lies,
 // where rows cost one line per row for ancestors spread thinly; the record
 // gather and store go through LDS and hold more registers.  The batched
-// engine keeps rows; a single filter with d <= 12 may use records.
+// engine keeps rows (its four-lane d = 24 kernels have records of their own,
+// pf_quad24.hpp); a single filter with d <= 12 may use records.
 struct Lay {
     int row, part;
 };
@@ -1700,8 +1690,8 @@ __global__ void __launch_bounds__(kWeightsBlock) k_weights_pair(WeightArgs a0, W
     weights_body<KIND>(blockIdx.y ? a1 : a0);
 }
 
-// Materialises the pending resampling: anc[j] for every output j, and the
-// statistics of the resampled frame (block 0).
+// Materialises the pending resampling: anc[j] for every output j, and, in the
+// launch's last block, the statistics of the resampled frame.
 struct AncArgs {
     Pending pend;
     FrameScratch *fs;
@@ -1715,13 +1705,6 @@ struct AncArgs {
 
 // The pending resampling of a, with the recorded largest block exponent when
 // its producer wrote one.
-__device__ __forceinline__ Pending anc_pending(const AncArgs &a)
-{
-    Pending pd = a.pend;
-    if (a.pow_frame && pd.bpow) pd.pow_max = &a.fs->pow_max[*a.pow_frame % 3];
-    return pd;
-}
-
 // Both phases for one block of outputs of a (a_j is returned), or, in the
 // launch's last block, which has no outputs, the statistics of the resampled
 // frame (returns -1).  The block sums, the exponent maxima and the frame
@@ -1785,7 +1768,7 @@ static __global__ void __launch_bounds__(kPrefixThreads) k_prefix(AncArgs a, uns
     __shared__ double s_v[kMaxScanBlocks];
     __shared__ unsigned long long s_wave[kPrefixThreads / 64];
     __shared__ int s_max[kPrefixThreads / 64];
-    const Pending pd = anc_pending(a);
+    const Pending &pd = a.pend;
     const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, nb = pd.nb;
     const int c0 = tid * kPrefixPer;
     unsigned long long s[kPrefixPer];

@@ -1,6 +1,6 @@
 // pf_step.hpp -- launches of the single-filter step (k_step), one source per
-// state layout (pf_step_rec.hip, pf_step_rows.hip): the layouts' kernels are
-// compiled with the scheduling that suits each.
+// state layout (pf_step_rec.hip, pf_step_rows.hip), so that their many kernels
+// compile side by side.
 #pragma once
 
 #include "pf_kernels.hpp"
