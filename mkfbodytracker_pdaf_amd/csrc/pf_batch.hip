@@ -650,12 +650,13 @@ int launch_batch_finish(pf_batch *b, const BatchArgs &a)
 }
 
 // Blocks without a tile that the replays of a captured pair may still launch
-// before it is captured again.  One costs 0.07 ns of a frame (256 threads) to
-// 0.17 (64), a capture about 100 us.  One sequence of 1,000 particles and 1,500
-// frames beside 200 of 64,000 and 2, per frame with tiles of 64 / 128 / 256
-// particles: 24.6 / 23.7 / 23.2 us, with a block for every tile in all frames
-// 54.7 / 31.7 / 23.3 (30.8 / 27.5 / 25.4 with a persistent grid).
-constexpr long long kIdleBlocks = 4LL << 20;
+// before it is captured again: at 0.07 ns each (256 threads; 64: 0.17) 73 to 180
+// us, where a capture costs about 20 us more than launching its two frames.  One
+// sequence of 1,000 particles and 1,500 frames beside 200 of 64,000 and 2, per
+// frame with tiles of 64 / 128 / 256 particles: 24.6 / 23.8 / 23.2 us, with a
+// block for every tile in all frames 54.7 / 31.7 / 23.3 (30.8 / 27.5 / 25.4 with
+// a persistent grid).
+constexpr long long kIdleBlocks = 1LL << 20;
 
 int run_all(pf_batch *b, const int32_t *count, const float *cand, const uint32_t *uni, double *lml, int frames,
             bool graph, bool record)
