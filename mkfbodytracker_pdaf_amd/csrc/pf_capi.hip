@@ -76,6 +76,8 @@ struct pf_handle {
     float *table = nullptr;
     int table_floats = 0;          // floats of the image staged in LDS
     const float *comp_global = nullptr;   // component rows read from global memory (large images)
+    int image_floats = 0, head_floats = 0;   // the whole image's, and those before its component rows
+    bool image_in_lds = false;     // the image is within its LDS budget
     float *mu = nullptr, *sig = nullptr;
     HostModel hm;
     // state basis x' = T x (T = I when H has no usable row-selection basis)
@@ -501,6 +503,20 @@ int read_status(pf_handle *h, unsigned *word)
 }
 
 
+// What the steps stage of the model image: all of it, or, if it exceeds its
+// budget, or, with records, would leave one block per CU beside the record
+// rounds' LDS, the part before the component rows, which are then read from
+// global memory.  d = 12, K = 126 (46 KB): 1,000 particles 19.5 us per frame with
+// the rows in global memory, 19.7 staged; 100,000 26.1, 39.0 staged (92: 25.6, 38.0).
+void set_stage(pf_handle *h)
+{
+    const int cand = cand_lds_floats(h->J, h->cap);
+    const bool whole = h->image_in_lds && (h->lay.row != 1 ||
+                                           step_lds_bytes_rec(true, h->image_floats + cand, 0) <= kCuLdsBytes / 2);
+    h->table_floats = whole ? h->image_floats : h->head_floats;
+    h->comp_global = whole ? nullptr : h->table + h->head_floats;
+}
+
 // Builds the LDS model image, the reset table and the basis matrices of the
 // handle's model and uploads them.
 int build_tables(pf_handle *h)
@@ -524,8 +540,10 @@ int build_tables(pf_handle *h)
     HIP_TRY(hipMemcpyAsync(h->Tdev, img.T.data(), sizeof(double) * img.T.size(), hipMemcpyHostToDevice, h->stream));
     HIP_TRY(hipMemcpyAsync(h->Tinv, img.Ti.data(), sizeof(double) * img.Ti.size(), hipMemcpyHostToDevice, h->stream));
     HIP_TRY(hipStreamSynchronize(h->stream));
-    h->table_floats = img.comp_in_lds ? (int)img.blob.size() : img.head_floats;
-    h->comp_global = img.comp_in_lds ? nullptr : h->table + img.head_floats;
+    h->image_floats = (int)img.blob.size();
+    h->head_floats = img.head_floats;
+    h->image_in_lds = img.comp_in_lds;
+    set_stage(h);
     return PF_OK;
 }
 }  // namespace
@@ -1524,6 +1542,7 @@ int pf_set_state_layout(pf_handle *h, int32_t layout)
     const int a = h->xA == h->xbuf[1] ? 1 : 0;
     if (!h->tracks) {
         set_views(h, rec, a);
+        set_stage(h);
         return PF_OK;
     }
     // the current state copied into the other buffer in the new layout, which
@@ -1531,6 +1550,7 @@ int pf_set_state_layout(pf_handle *h, int32_t layout)
     const float *xs = h->xA, *Ps = h->PA;
     const Lay Ls = h->lay;
     set_views(h, rec, 1 - a);
+    set_stage(h);
     st = dispatch_d<RelayoutL>(h->D, h, xs, Ps, Ls);
     if (st) return st;
     st = check_launch("k_relayout");
