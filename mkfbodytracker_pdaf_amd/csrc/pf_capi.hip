@@ -158,25 +158,42 @@ void drop_graphs(pf_handle *h)
                 }
 }
 
+// The resampler scratch of L weights.  A set is replaced only by a whole one:
+// steps use it without asking again.
+struct ResampleScratch {
+    unsigned long long *cloc = nullptr, *bsum = nullptr, *gpre = nullptr;
+    double *bexp = nullptr;
+    int *bpow = nullptr, *gshf = nullptr;
+    hipError_t open(int L, bool prefix)
+    {
+        const size_t nb = ((size_t)L + kWeightsBlock - 1) / kWeightsBlock;
+        hipError_t e = dalloc(&cloc, (size_t)L);
+        if (e == hipSuccess) e = dalloc(&bsum, nb);
+        if (e == hipSuccess) e = dalloc(&bexp, nb);
+        if (e == hipSuccess) e = dalloc(&bpow, nb);
+        if (e == hipSuccess && prefix) e = dalloc(&gpre, nb + 1);
+        if (e == hipSuccess && prefix) e = dalloc(&gshf, nb);
+        return e;
+    }
+    ~ResampleScratch()
+    {
+        for (void *p : {(void *)cloc, (void *)bsum, (void *)bexp, (void *)bpow, (void *)gpre, (void *)gshf})
+            if (p) (void)hipFree(p);
+    }
+};
+
 int ensure_resample_scratch(pf_handle *h, int L)
 {
     if (L <= h->Lcap) return PF_OK;
+    ResampleScratch s;
+    HIP_TRY(s.open(L, true));
     drop_graphs(h);
-    (void)hipFree(h->cloc);
-    (void)hipFree(h->bsum);
-    (void)hipFree(h->bexp);
-    (void)hipFree(h->bpow);
-    (void)hipFree(h->gpre);
-    (void)hipFree(h->gshf);
-    h->cloc = nullptr; h->bsum = nullptr; h->bexp = nullptr; h->bpow = nullptr; h->gpre = nullptr; h->gshf = nullptr;
-    h->Lcap = 0;
-    const int nb = (L + kWeightsBlock - 1) / kWeightsBlock;
-    HIP_TRY(dalloc(&h->cloc, (size_t)L));
-    HIP_TRY(dalloc(&h->bsum, (size_t)nb));
-    HIP_TRY(dalloc(&h->bexp, (size_t)nb));
-    HIP_TRY(dalloc(&h->bpow, (size_t)nb));
-    HIP_TRY(dalloc(&h->gpre, (size_t)nb + 1));
-    HIP_TRY(dalloc(&h->gshf, (size_t)nb));
+    std::swap(h->cloc, s.cloc);
+    std::swap(h->bsum, s.bsum);
+    std::swap(h->bexp, s.bexp);
+    std::swap(h->bpow, s.bpow);
+    std::swap(h->gpre, s.gpre);
+    std::swap(h->gshf, s.gshf);
     h->Lcap = L;
     return PF_OK;
 }
@@ -185,11 +202,12 @@ int ensure_resample_scratch(pf_handle *h, int L)
 int ensure_run_scratch(pf_handle *h)
 {
     if (h->cloc1) return PF_OK;
-    const int nb = (h->N + kWeightsBlock - 1) / kWeightsBlock;
-    HIP_TRY(dalloc(&h->cloc1, (size_t)h->N));
-    HIP_TRY(dalloc(&h->bsum1, (size_t)nb));
-    HIP_TRY(dalloc(&h->bexp1, (size_t)nb));
-    HIP_TRY(dalloc(&h->bpow1, (size_t)nb));
+    ResampleScratch s;
+    HIP_TRY(s.open(h->N, false));
+    std::swap(h->cloc1, s.cloc);
+    std::swap(h->bsum1, s.bsum);
+    std::swap(h->bexp1, s.bexp);
+    std::swap(h->bpow1, s.bpow);
     return PF_OK;
 }
 
