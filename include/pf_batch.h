@@ -106,7 +106,9 @@ int pf_batch_autotune(pf_batch *b, const int32_t *count, const float *cand, cons
  *   PF_BATCH_QUAD_VALU  the MFMA variant's layout with the tile updates on
  *                       the vector ALU (for comparison).
  * All three run the algorithm of pf_step_candidates(); results agree to FP32
- * rounding (the order of the sums differs). */
+ * rounding (the order of the sums differs).  Tracks that have been set move to
+ * the other kernel's layout, bit for bit, by way of memory for one more state
+ * buffer (PF_ERR_HIP, and nothing changed, if there is none). */
 #define PF_BATCH_VALU 0
 #define PF_BATCH_MFMA 1
 #define PF_BATCH_QUAD_VALU 2

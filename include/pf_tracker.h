@@ -79,6 +79,7 @@ void pf_tracker_config_default(pf_tracker_config *cfg);
 int pf_tracker_create(pf_tracker **out, const pf_tracker_config *cfg, pf_handle *arm1, pf_handle *arm2,
                       int32_t npose, const double *pca_proj1, const double *pca_mean1,
                       const double *pca_proj2, const double *pca_mean2);
+/* Before or after its arms. */
 int pf_tracker_destroy(pf_tracker *tr);
 /* Back to frame 0: the next frame uses the uniform proposals (the arms'
  * tracks are the caller's, e.g. pf_reset). */
